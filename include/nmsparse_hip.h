@@ -415,6 +415,29 @@ int nm_gemv_plan(int h, int w, int nnz, int m, int config_id, int splits,
                  int* out_config_id, int* out_splits, int* out_blocks,
                  int* out_rows_per_block);
 
+/*
+ * The attention of one decode token over the transposed static caches:
+ * out[h, :] = softmax over positions p <= *pos of q[h, :] . K[h / g, :, p] /
+ * sqrt(head_dim), times V[h / g, :, p], with g = n_heads / kv_heads query heads
+ * per key/value head (g <= 16). q rows q_row_stride elements apart;
+ * k_cache_t [kv_heads, >= head_dim, cache_len] and v_cache_t [kv_heads,
+ * head_dim, cache_len] with heads k_head_stride / v_head_stride elements
+ * apart (the layouts the q/k/v launch writes); out [n_heads, head_dim]
+ * contiguous. fp16 and bf16; head_dim 64 or 128; cache_len a multiple of 8;
+ * strides multiples of 8 elements, pointers 16-byte aligned, the workspace
+ * as nm_gemv_launch's. *pos is read on the device; past the cache it stands
+ * for every position, below zero for none (the outputs are then NaN). `span`:
+ * positions per workgroup (64, 128, 256), 0 = the library's choice. Scores,
+ * softmax and sums in fp32, probabilities and outputs rounded to the element
+ * type; splits merge in a fixed order. No reference counterpart (the
+ * reference's attention is PyTorch's, model.py:219-246).
+ */
+size_t nm_attention_decode_workspace_bytes(int n_heads, int kv_heads, int head_dim, int cache_len, int span);
+int nm_attention_decode(int dtype, const void* q, long long q_row_stride, const void* k_cache_t,
+                        long long k_head_stride, const void* v_cache_t, long long v_head_stride, void* out,
+                        const long long* pos, void* workspace, size_t workspace_bytes, int n_heads, int kv_heads,
+                        int head_dim, int cache_len, int span, void* stream);
+
 /* Human-readable text for a status code returned above. */
 const char* nm_strerror(int code);
 

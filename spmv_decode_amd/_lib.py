@@ -92,13 +92,15 @@ ABI = {
                               ctypes.POINTER(_ll), _ip, _vp, _sz, _i, _i, _i, _i, _i, _vp]),
     "nm_spmm_mc_group_plan": (_i, [_i, _i, _ip, _i, _i, _i, _i, _i, _ip, _ip, _ip, _ip]),
     "nm_gather_columns": (_i, [_i, _vp, _ll, _i, _vp, _i, _i, _i, _vp, _ll, _vp]),
+    "nm_attention_decode_workspace_bytes": (_sz, [_i, _i, _i, _i, _i]),
+    "nm_attention_decode": (_i, [_i, _vp, _ll, _vp, _ll, _vp, _ll, _vp, _vp, _vp, _sz, _i, _i, _i, _i, _i, _vp]),
     "nm_config_describe": (_i, [_i, ctypes.c_char_p, _i]),
     "nm_gemv_plan": (_i, [_i, _i, _i, _i, _i, _i, _ip, _ip, _ip, _ip]),
     "nm_strerror": (ctypes.c_char_p, [_i]),
     "nm_abi_version": (_i, []),
     "nm_stream_capture_id": (_i, [_vp, ctypes.POINTER(ctypes.c_ulonglong)]),
 }
-ABI_VERSION = 12
+ABI_VERSION = 13
 
 _lib = None
 _lock = threading.Lock()

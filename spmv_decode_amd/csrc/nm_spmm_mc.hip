@@ -37,7 +37,7 @@
 //    the last arrival sums the partials in split order and rounds to T.
 //    Deterministic for a given plan; not bit-identical to the GEMV (the
 //    matrix core's dot products have their own order).
-#include "nm_gemv_kernel.h"
+#include "nm_mfma.h"
 
 namespace nm_hip {
 namespace {
@@ -46,28 +46,6 @@ constexpr int kMcCK = 64;         // compressed columns per chunk: two MFMA K st
 constexpr int kMcNumConfigs = 6;  // output tile HT = 64, 128, 256; register-staged (0-2) or DMA (3-5) weights
 static_assert(NM_MC_MAX_BATCH == 128, "batch tiles of 16, 32, 64 and 128 rows");
 
-typedef short s4 __attribute__((ext_vector_type(4)));
-typedef short s8 __attribute__((ext_vector_type(8)));
-typedef float f4 __attribute__((ext_vector_type(4)));
-typedef _Float16 h8 __attribute__((ext_vector_type(8)));
-typedef __bf16 b8 __attribute__((ext_vector_type(8)));
-typedef __attribute__((address_space(3))) s4 lds_s4;
-
-template <int DT>
-__device__ inline f4 mfma16x16x32(s8 a, s8 b, f4 c);
-template <>
-__device__ inline f4 mfma16x16x32<NM_DTYPE_F16>(s8 a, s8 b, f4 c) {
-  return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, a), __builtin_bit_cast(h8, b), c, 0, 0, 0);
-}
-template <>
-__device__ inline f4 mfma16x16x32<NM_DTYPE_BF16>(s8 a, s8 b, f4 c) {
-  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(b8, a), __builtin_bit_cast(b8, b), c, 0, 0, 0);
-}
-
-// MFMA 16x16x32 register layout (gfx950; checked on the GPU): A[16 x 32]:
-// lane l holds row l % 16, K elements 8*(l/16) .. +7; B[32 x 16]: column
-// l % 16, K elements 8*(l/16) .. +7; D[16 x 16]: column l % 16, rows
-// 4*(l/16) .. +3.
 // LDS stages of the DMA variant per tile width (S - 1 chunks of 64 x HT
 // weights and their activation fragments in flight): 4 / 3 / 3 for 64- /
 // 128- / 256-column tiles, fitted to graph-replay sweeps of 2-8 stages at

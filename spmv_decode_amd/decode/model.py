@@ -18,7 +18,10 @@ mask lives in the key cache: each head has KEY_PAD extra rows, the first of
 them holding the additive mask (0 at positions <= pos, -inf after), and the
 query buffer holds a 1 in that column, so one plain batched product yields the
 masked scores (an additive mask operand makes PyTorch copy it into the output
-before the product: one more kernel per layer and a slower GEMM).
+before the product: one more kernel per layer and a slower GEMM). On the GPU
+in fp16 / bf16 the three kernels of that form (product, softmax, product) give
+way to one, which reads the position itself and only the cached positions up
+to it (attend_at).
 
 Numerics follow the published architectures: RMSNorm in fp32 (one fused
 `F.rms_norm` kernel), rotary embeddings on interleaved (even, odd) pairs as a
@@ -44,7 +47,7 @@ When every projection of every layer is an `NmSparseLinear` (after
 rotary embedding and the KV-cache write happen inside the grouped q/k/v
 launch, the residual adds inside the o and down launches (in place on the
 residual stream), and the post-attention RMSNorm inside the gate/up launch.
-A layer is then 7 kernels: q/k/v, three attention kernels, o, gate/up, down.
+A layer is then 5 kernels: q/k/v, attention, o, gate/up, down.
 The per-Linear path above stays for dense models and for comparison.
 """
 from __future__ import annotations
@@ -160,6 +163,21 @@ def attend(q_pad: torch.Tensor, k_cache_t: torch.Tensor, v_cache_t: torch.Tensor
     scores = torch.baddbmm(zero, q3, k_cache_t, beta=0.0, alpha=1.0 / math.sqrt(cfg.head_dim))
     probs = torch.softmax(scores, dim=-1)  # fp16 in/out, fp32 inside
     return torch.bmm(probs, v_cache_t.transpose(1, 2))
+
+
+def attend_at(at, q: torch.Tensor, k_cache_t: torch.Tensor, v_cache_t: torch.Tensor, zero: torch.Tensor,
+              pos: torch.Tensor) -> torch.Tensor:
+    """attend over the positions <= pos (at: the attention module). Where
+    Decoder.setup_cache found the caches within the library's attention kernel
+    (at.decode_kernel) one launch reads the position on the device and the
+    cached positions up to it; the mask row and q's columns past head_dim are
+    not read then. Otherwise attend (q the padded query buffer, the mask row
+    written for pos)."""
+    c = at.cfg
+    if at.decode_kernel:
+        y = torch.ops.nmsparse.attention_decode(q, k_cache_t, v_cache_t, pos, c.head_dim)
+        return y.view(c.n_kv_heads, c.n_heads // c.n_kv_heads, c.head_dim)
+    return attend(q, k_cache_t, v_cache_t, c, zero)
 
 
 def linear_into(lin: nn.Module, x2d: torch.Tensor, out: torch.Tensor) -> torch.Tensor:
@@ -292,6 +310,7 @@ def grouped_sparse(mods) -> bool:
 class Attention(nn.Module):
     group_launches = True  # one q/k/v launch when all three are sparse (Decoder.set_launch_mode)
     call_modules = False   # every projection through its module's forward (Decoder.set_launch_mode)
+    decode_kernel = False  # attention in the library's one launch (Decoder.setup_cache)
 
     def __init__(self, cfg: DecoderConfig):
         super().__init__()
@@ -355,7 +374,7 @@ def _(cache, pos, values):
 def attention_core(at, qkv, freqs, k_cache_t, v_cache_t, pos, q_pad, zero):
     """The attention of one decode token from its projections qkv [1, q + k + v]
     (at: the attention module, for its config and Qwen3's q/k norms): head
-    norms, rotary embedding, the cache write at `pos`, attend. Returns
+    norms, rotary embedding, the cache write at `pos`, attend_at. Returns
     [kv_heads, g, head_dim]."""
     c = at.cfg
     qd, kvd = c.n_heads * c.head_dim, c.n_kv_heads * c.head_dim
@@ -365,13 +384,15 @@ def attention_core(at, qkv, freqs, k_cache_t, v_cache_t, pos, q_pad, zero):
     qk = rotate(qk, freqs)
     q, k = qk[:c.n_heads], qk[c.n_heads:]
     v = qkv[0, qd + kvd:].view(c.n_kv_heads, c.head_dim, 1)
-    q_pad[:, :c.head_dim].copy_(q)
+    if not at.decode_kernel:
+        q_pad[:, :c.head_dim].copy_(q)
+        q = q_pad
     if torch.compiler.is_compiling():
         cache_write(k_cache_t, pos, k)
     else:
         k_cache_t[:, :c.head_dim].index_copy_(2, pos, k.unsqueeze(-1))
     v_cache_t.index_copy_(2, pos, v)
-    return attend(q_pad, k_cache_t, v_cache_t, c, zero)
+    return attend_at(at, q, k_cache_t, v_cache_t, zero, pos)
 
 
 class MLP(nn.Module):
@@ -421,6 +442,8 @@ class GptFastAttention(nn.Module):
     fused `wqkv` Linear [q + k + v rows] and `wo`; Qwen3's q/k norms when the
     config has them. Same math as Attention; every projection is a module call,
     as unmodified gpt-fast code makes it."""
+
+    decode_kernel = False  # attention in the library's one launch (Decoder.setup_cache)
 
     def __init__(self, cfg: DecoderConfig):
         super().__init__()
@@ -501,7 +524,7 @@ def fused_block_step(blk: Block, x2d, k_cache_t, v_cache_t, pos, q_pad, zero, ro
                    qp.block_width, qp.vec_width, q_pad, k_cache_t, v_cache_t, pos, rope, c.head_dim, ln1.weight,
                    ln1.eps, at.q_norm.weight if c.qk_norm else None, at.k_norm.weight if c.qk_norm else None,
                    c.norm_eps, None)
-    y = attend(q_pad, k_cache_t, v_cache_t, c, zero).view(1, qd)
+    y = attend_at(at, q_pad, k_cache_t, v_cache_t, zero, pos).view(1, qd)
     o = at.o_proj
     ops.gemv_add_(y, o.mat_data, o.mat_index, o.block_width, o.vec_width, x2d)
     gp, up = mlp.gate_proj, mlp.up_proj
@@ -574,7 +597,7 @@ def fused_layers_carried(layers, x2d, h2d, carry_o, carry_d, k_caches, v_caches,
             ops.qkv_decode(x2d, *qkv, None)
         else:
             ops.qkv_decode_carried(h2d, carry_d, x2d, *qkv, None)
-        y = attend(q_pad, k_caches[i], v_caches[i], c, zero).view(1, c.n_heads * c.head_dim)
+        y = attend_at(at, q_pad, k_caches[i], v_caches[i], zero, pos).view(1, c.n_heads * c.head_dim)
         o = at.o_proj
         ops.gemv_partials_(y, o.mat_data, o.mat_index, o.block_width, o.vec_width, carry_o)
         gp, up = mlp.gate_proj, mlp.up_proj
@@ -623,7 +646,7 @@ def fused_layers_accumulated(layers, x2d, h2d, acc_op, acc_d, ssq_n, k_caches, v
             ops.qkv_decode(x2d, *qkv, acc_op)
         else:
             ops.qkv_decode_carried(h2d, acc_d, x2d, *qkv, acc_op)
-        y = attend(q_pad, k_caches[i], v_caches[i], c, zero).view(1, c.n_heads * c.head_dim)
+        y = attend_at(at, q_pad, k_caches[i], v_caches[i], zero, pos).view(1, c.n_heads * c.head_dim)
         o = at.o_proj
         ops.gemv_accumulate_(y, o.mat_data, o.mat_index, o.block_width, o.vec_width, acc_o, None)
         gp, up = mlp.gate_proj, mlp.up_proj
@@ -686,6 +709,7 @@ class Decoder(nn.Module):
         self.norm = RMSNorm(cfg.dim, cfg.norm_eps)
         self.lm_head = nn.Linear(cfg.dim, cfg.vocab, bias=False)
         self.max_seq = 0
+        self.attention_kernel = False  # setup_cache: the layers' decode_kernel
         self.gemv_forms = {}  # (n_out, n_in) -> dense_gemv form, filled by tune_dense_gemv
         self.dense_fusion = "none"  # set_dense_fusion's mode
 
@@ -792,7 +816,7 @@ class Decoder(nn.Module):
     def setup_cache(self, max_seq: int, device, dtype=torch.float16):
         """Static caches for max_seq positions (see attend for the layouts); the
         key caches of all layers are views of one tensor so that one kernel per
-        step rewrites every layer's mask row."""
+        step rewrites every layer's mask row (where attend needs it: attend_at)."""
         c = self.cfg
         self.max_seq = max_seq
         hd, D = c.head_dim, c.head_dim + KEY_PAD
@@ -810,6 +834,14 @@ class Decoder(nn.Module):
         self.rope = torch.polar(torch.ones_like(ang), ang).to(torch.complex64).to(device)
         self.rope_real = torch.view_as_real(self.rope)  # the same table as fp32 (cos, sin) pairs
         self.positions = torch.arange(max_seq, device=device)
+        kernel = False
+        if self.q_pad.is_cuda:
+            from ..hip_spmv import attention_supported
+
+            kernel = attention_supported(self.q_pad, self.k_cache_t[0], self.v_cache_t[0], hd)
+        self.attention_kernel = kernel
+        for blk in self.layers:
+            (blk.self_attn if isinstance(blk, Block) else blk.attention).decode_kernel = kernel
         self._carry = None
         self.prepare_decode()
 
@@ -923,12 +955,13 @@ class Decoder(nn.Module):
         """One decode step: token [1, 1] int64 and pos [1] int64 on the device
         -> logits [1, vocab]. No host synchronisation."""
         x = self.embed_tokens(token)  # [1, 1, dim]
-        # causal mask of this step in every layer's key cache: 0 up to pos, -inf after
-        keep = (self.positions <= pos).expand_as(self.k_mask)
-        if torch.compiler.is_compiling():  # the tracer takes no strided out=; the compiler fuses the copy
-            self.k_mask.copy_(torch.where(keep, self.zero, self.neg_inf))
-        else:
-            torch.where(keep, self.zero, self.neg_inf, out=self.k_mask)
+        if not self.attention_kernel:
+            # causal mask of this step in every layer's key cache: 0 up to pos, -inf after
+            keep = (self.positions <= pos).expand_as(self.k_mask)
+            if torch.compiler.is_compiling():  # the tracer takes no strided out=; the compiler fuses the copy
+                self.k_mask.copy_(torch.where(keep, self.zero, self.neg_inf))
+            else:
+                torch.where(keep, self.zero, self.neg_inf, out=self.k_mask)
         if self.fuse_epilogues and all(fusable(b, x.dtype) and b.self_attn.group_launches for b in self.layers):
             x2d = x.view(1, -1)
             if not torch.compiler.is_compiling():

@@ -864,8 +864,62 @@ def nmsparse_qkv_decode(vec, q, k, v, BLOCK_WIDTH, VEC_WIDTH, *, q_out, k_cache_
                                 splits=splits, carry_in=carry_in, vec_out=vec_out, zero=zero)
 
 
+def attention_supported(q: torch.Tensor, k_cache_t: torch.Tensor, v_cache_t: torch.Tensor, head_dim: int) -> bool:
+    """Whether nmsparse_attention_decode takes these tensors: fp16 / bf16 on
+    the GPU, q [n_heads, >= head_dim] and caches [kv_heads, >= head_dim, S] /
+    [kv_heads, head_dim, S] with unit last strides and whole 16-byte rows
+    (S a multiple of 8), head_dim 64 or 128, at most 16 query heads per
+    key/value head, S within the library's merge limit. No GPU work."""
+    if not (q.is_cuda and k_cache_t.is_cuda and v_cache_t.is_cuda and q.dtype in (torch.float16, torch.bfloat16)
+            and q.dtype == k_cache_t.dtype == v_cache_t.dtype and q.device == k_cache_t.device == v_cache_t.device):
+        return False
+    if q.dim() != 2 or k_cache_t.dim() != 3 or v_cache_t.dim() != 3 or q.shape[1] < head_dim:
+        return False
+    kvh, kd, S = k_cache_t.shape
+    if kd < head_dim or tuple(v_cache_t.shape) != (kvh, head_dim, S) or kvh == 0 or q.shape[0] % kvh:
+        return False
+    if (q.stride(1) != 1 or k_cache_t.stride(2) != 1 or k_cache_t.stride(1) != S or v_cache_t.stride(2) != 1
+            or v_cache_t.stride(1) != S or q.stride(0) % 8 or k_cache_t.stride(0) % 8 or v_cache_t.stride(0) % 8
+            or q.stride(0) < head_dim or k_cache_t.stride(0) < head_dim * S or v_cache_t.stride(0) < head_dim * S):
+        return False
+    return _lib.load().nm_attention_decode_workspace_bytes(q.shape[0], kvh, int(head_dim), S, 0) > 0
+
+
+def nmsparse_attention_decode(q, k_cache_t, v_cache_t, pos, head_dim, *, out=None, span=0):
+    """The attention of one decode token, one launch: softmax over positions
+    p <= pos of q[h, :head_dim] . k_cache_t[h // g, :head_dim, p] /
+    sqrt(head_dim), times v_cache_t[h // g, :, p]. q [n_heads, >= head_dim],
+    caches as nmsparse_qkv_decode writes them (attention_supported says which
+    are taken), pos a device int64 tensor of one element. Returns [1, n_heads *
+    head_dim] (or writes `out`); fp32 scores and sums. `span`: positions per
+    workgroup (64, 128, 256; 0 = the library's choice)."""
+    if not attention_supported(q, k_cache_t, v_cache_t, head_dim):
+        raise ValueError(f"attention over q {tuple(q.shape)} {q.dtype}, k {tuple(k_cache_t.shape)}, "
+                         f"v {tuple(v_cache_t.shape)} with head_dim {head_dim} is not supported")
+    if pos.dtype != torch.int64 or pos.numel() != 1 or pos.device != q.device:
+        raise ValueError("pos must be a device int64 tensor of one element")
+    nh = q.shape[0]
+    kvh, _, S = k_cache_t.shape
+    out = _prepare_out(out, nh * head_dim, q)
+    if any(t.data_ptr() % 16 for t in (q, k_cache_t, v_cache_t)):
+        raise ValueError("q and the caches must be 16-byte aligned")
+    lib = _lib.load()
+    need = lib.nm_attention_decode_workspace_bytes(nh, kvh, int(head_dim), S, int(span))
+    if need == 0:
+        raise ValueError(f"span {span} is outside what libnmsparse_hip supports for {S} positions")
+    with torch.cuda.device(q.device):
+        stream = torch.cuda.current_stream(q.device).cuda_stream
+        ws = workspace_for(q.device, need, stream)
+        rc = lib.nm_attention_decode(_DTYPE_CODE[q.dtype], q.data_ptr(), q.stride(0), k_cache_t.data_ptr(),
+                                     k_cache_t.stride(0), v_cache_t.data_ptr(), v_cache_t.stride(0), out.data_ptr(),
+                                     pos.data_ptr(), ws.data_ptr(), ws.numel(), nh, kvh, int(head_dim), S, int(span),
+                                     stream)
+    _lib.check(rc, "nm_attention_decode")
+    return out
+
+
 __all__ = ["nmsparse_spmv_forward_hip", "nmsparse_spmv_forward_triton_ptx", "nmsparse_gemv_grouped",
            "nmsparse_gate_up_silu", "nmsparse_gemv_launch", "nmsparse_qkv_decode", "nmsparse_spmm_forward_hip",
            "nmsparse_gemv_partials", "carry_splits", "GemvProblem", "launch_plan", "validate_args", "workspace_for",
            "nmsparse_gemv_accumulate", "nmsparse_gate_up_accumulate", "nmsparse_gemv_silu", "gate_up_ssq_slots",
-           "library_route"]
+           "library_route", "attention_supported", "nmsparse_attention_decode"]

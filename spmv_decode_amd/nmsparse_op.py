@@ -27,7 +27,8 @@ run to run) adds `nmsparse::gemv_accumulate_`, `nmsparse::gate_up_accumulate_`
 (the pair as a producer of raw sums), `nmsparse::gemv_silu_accumulate_` and
 `nmsparse::gemv_silu_add_` (down_proj taking the pair's SiLU product as it
 gathers its input), and the `zero` argument of the q/k/v ops (an accumulator
-cleared by the launch).
+cleared by the launch). `nmsparse::attention_decode` is the attention between
+the q/k/v launch and o_proj: one launch over the caches' positions up to pos.
 
 `nmsparse::gemv_grouped` (one launch for 1-4 gemv calls on the same input),
 `nmsparse::gemv_silu_mul` (silu(gemv gate) * gemv up in one launch), both
@@ -57,9 +58,9 @@ import torch
 
 from typing import Optional
 
-from .hip_spmv import (GemvProblem, nmsparse_gate_up_accumulate, nmsparse_gate_up_silu, nmsparse_gemv_accumulate,
-                       nmsparse_gemv_grouped, nmsparse_gemv_launch, nmsparse_gemv_partials, nmsparse_gemv_silu,
-                       nmsparse_qkv_decode, nmsparse_spmm_forward_hip, nmsparse_spmv_forward_hip)
+from .hip_spmv import (GemvProblem, nmsparse_attention_decode, nmsparse_gate_up_accumulate, nmsparse_gate_up_silu,
+                       nmsparse_gemv_accumulate, nmsparse_gemv_grouped, nmsparse_gemv_launch, nmsparse_gemv_partials,
+                       nmsparse_gemv_silu, nmsparse_qkv_decode, nmsparse_spmm_forward_hip, nmsparse_spmv_forward_hip)
 
 _kernel = os.environ.get("NM_KERNEL", "")
 if _kernel not in ("", "hip", "triton_ptx", "guarded", "fp16", "fp16_split"):
@@ -363,6 +364,20 @@ def _(silu_in, mat_data, mat_index, block_width, vec_width, ssq_n, silu_k, silu_
     return None
 
 
-__all__ = ["gemv", "spmm", "gemv_grouped", "gemv_silu_mul", "gemv_residual", "qkv_decode", "gemv_add_", "gate_up_silu", "gemv_partials_",
+@torch.library.custom_op("nmsparse::attention_decode", mutates_args=())
+def attention_decode(q: torch.Tensor, k_cache_t: torch.Tensor, v_cache_t: torch.Tensor, pos: torch.Tensor,
+                     head_dim: int) -> torch.Tensor:
+    """The attention of one decode token over positions <= pos of the
+    transposed caches, one launch -> [1, n_heads * head_dim]
+    (hip_spmv.nmsparse_attention_decode)."""
+    return nmsparse_attention_decode(q, k_cache_t, v_cache_t, pos, int(head_dim))
+
+
+@attention_decode.register_fake
+def _(q, k_cache_t, v_cache_t, pos, head_dim):
+    return q.new_empty((1, q.shape[0] * int(head_dim)))
+
+
+__all__ = ["attention_decode", "gemv", "spmm", "gemv_grouped", "gemv_silu_mul", "gemv_residual", "qkv_decode", "gemv_add_", "gate_up_silu", "gemv_partials_",
            "qkv_decode_carried", "gate_up_silu_carried", "gemv_accumulate_", "gate_up_accumulate_",
            "gemv_silu_accumulate_", "gemv_silu_add_"]

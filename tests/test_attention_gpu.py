@@ -1,0 +1,72 @@
+"""GPU parity of the one-launch decode attention (nm_attention_decode) against
+attention in 64 bits: both element types and head dimensions, 1 to 16 query
+heads per key/value head, positions at the edges of the splits (first, last
+of a split, first of the next, last of the cache), every span, padded key
+rows, and cached values past the position that are not finite."""
+import math
+
+import pytest
+import torch
+
+from spmv_decode_amd import hip_spmv
+
+pytestmark = pytest.mark.gpu
+
+
+def case(nh, kvh, hd, S, dtype, pad, seed):
+    gen = torch.Generator(device="cuda").manual_seed(seed)
+    q = torch.randn(nh, hd + pad, device="cuda", generator=gen).to(dtype)
+    k = torch.randn(kvh, hd + pad, S, device="cuda", generator=gen).to(dtype)
+    v = torch.randn(kvh, hd, S, device="cuda", generator=gen).to(dtype)
+    return q, k, v
+
+
+def exact(q, k, v, hd, n):
+    kvh = k.shape[0]
+    qd = q[:, :hd].double().view(kvh, -1, hd)
+    p = torch.softmax(torch.bmm(qd, k[:, :hd, :n].double().contiguous()) / math.sqrt(hd), dim=-1)
+    return torch.bmm(p, v[:, :, :n].double().transpose(1, 2).contiguous()).reshape(1, -1)
+
+
+# (query heads, key/value heads, head_dim, cache length, padding)
+SHAPES = [(32, 8, 128, 640, 32), (40, 8, 128, 4096, 32), (16, 8, 128, 128, 0), (64, 8, 128, 1032, 32),
+          (16, 1, 64, 264, 8), (4, 2, 64, 8, 32), (5, 5, 128, 9000, 0)]
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16], ids=str)
+@pytest.mark.parametrize("shape", SHAPES, ids=str)
+def test_attention_decode_matches_exact(gpu, shape, dtype):
+    nh, kvh, hd, S, pad = shape
+    q, k, v = case(nh, kvh, hd, S, dtype, pad, seed=S + nh)
+    # one rounding of each probability and of each output: two half-ulps, relative to the outputs' norm
+    bar = 2 * torch.finfo(dtype).eps
+    for pos in sorted({0, 1, 7, 63, 64, 127, 255, 256, S // 2, S - 2, S - 1, S + 5}):
+        if pos >= S and pos != S + 5:
+            continue
+        n = min(pos + 1, S)
+        ref = exact(q, k, v, hd, n)
+        kd, vd = k.clone(), v.clone()
+        vd[:, :, n:] = float("nan")  # stale cache contents must not reach the result
+        kd[:, :, n:] = float("nan")
+        at = torch.tensor([pos], device="cuda")
+        for span in (0, 64, 128, 256):
+            if span and 8 * -(-S // span) * (nh // kvh) + 4112 > 2 * hd * span:
+                continue
+            y = hip_spmv.nmsparse_attention_decode(q, kd, vd, at, hd, span=span)
+            again = hip_spmv.nmsparse_attention_decode(q, kd, vd, at, hd, span=span)
+            assert torch.equal(y, again), (shape, pos, span)
+            rel = float((y.double() - ref).norm() / ref.norm())
+            assert rel <= bar, (shape, dtype, pos, span, rel)
+
+
+def test_attention_decode_edges(gpu):
+    q, k, v = case(8, 2, 128, 64, torch.float16, 0, seed=3)
+    none = hip_spmv.nmsparse_attention_decode(q, k, v, torch.tensor([-1], device="cuda"), 128)
+    assert torch.isnan(none).all()
+    k[0, :, 5] = float("nan")  # a NaN score makes its heads' rows NaN, and no others
+    y = hip_spmv.nmsparse_attention_decode(q, k, v, torch.tensor([9], device="cuda"), 128).view(8, 128)
+    assert torch.isnan(y[:4]).all() and torch.isfinite(y[4:]).all()
+    for bad in ((q.float(), k.float(), v.float()), (q, k[:, :, :60], v[:, :, :60]), (q[:, :64], k, v), (q[:7], k, v)):
+        assert not hip_spmv.attention_supported(*bad, 128)
+        with pytest.raises(ValueError):
+            hip_spmv.nmsparse_attention_decode(*bad, torch.tensor([3], device="cuda"), 128)

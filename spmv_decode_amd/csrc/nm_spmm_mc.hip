@@ -16,10 +16,10 @@
 //  * A first kernel gathers the activations once per call, Xg[b, c] =
 //    x[b, (c/nnz)*m + mat_index[c]], into the workspace ([batch, wp], wp = w
 //    rounded up to whole 64-column chunks, zero past w).
-//  * The main kernel: a workgroup (256 lanes = 4 wave64) owns an output tile
-//    of HT columns r and all BT >= batch rows (16, 32, 64 or 128), over one
-//    split of the compressed columns c. The 4 waves split the tile into row
-//    ranges (one 16-row block each up to 32 rows, two / four blocks each at
+//  * The main kernel: a workgroup (4 wave64, 8 in the DMA variant) owns an
+//    output tile of HT columns r and all BT >= batch rows (16, 32, 64 or 128),
+//    over one split of the compressed columns c. The waves split the tile into
+//    row ranges (one 16-row block each up to 32 rows, two / four blocks each at
 //    64 / 128) x column ranges; a wave keeps its rows x columns as 16 x 16 fp32
 //    accumulator blocks in registers. Chunks of 64 compressed columns (two
 //    MFMA K steps): the weight rows [64 x HT] are staged through LDS. Up to
@@ -53,6 +53,14 @@ static_assert(NM_MC_MAX_BATCH == 128, "batch tiles of 16, 32, 64 and 128 rows");
 // up to 8% slower, two stages up to 30%). At most 65 KB of LDS per
 // workgroup.
 constexpr int mc_stages(int ht) { return ht == 64 ? 4 : 3; }
+// Lanes per workgroup: 4 wave64, 8 for the DMA tiles that give each a
+// 16-column block. The ring's reads and multiplies run back to back within a
+// wave (each read block ends with its wait), so with one wave per SIMD every
+// LDS round trip was exposed; a second wave multiplies meanwhile. Calls with
+// the gather, 4 -> 8 waves (graph replay): gate/up 4096 -> 2 x 14336 at 128 rows
+// 37.8 -> 35.0 us, 5120 -> 2 x 17408 at 33 / 128 rows 50.1 -> 45.9 / 79.1 -> 68.9,
+// down 17408 -> 5120 30.8 -> 28.5 at 33; up to 16 rows level (the weight stream).
+constexpr int mc_block(int bt, int ht, bool dma) { return dma && ht / (bt < 32 ? 8 : 4) >= 16 ? 512 : 256; }
 constexpr int kMcNtAux = 2;  // cache policy of the weight DMA: non-temporal
 
 // Inline asm with register constraints exists only in the device pass (the
@@ -116,12 +124,14 @@ __device__ __forceinline__ void mc_tile(const SpmmArgs& a, const int block) {
   // the whole weight tile from LDS four times over, and measured 2-9% slower
   // at 64 rows).
   constexpr int WM = RBT < 2 ? RBT : 2;
-  constexpr int WN = 4 / WM;                // waves along the output columns
+  constexpr int BLK = mc_block(BT, HT, DMA);
+  constexpr int NWV = BLK / 64;             // waves
+  constexpr int WN = NWV / WM;              // waves along the output columns
   constexpr int MB = RBT / WM;              // 16-row blocks per wave
   constexpr int NW = HT / WN;               // output columns per wave
   constexpr int NBK = NW / 16;              // 16-column blocks per wave
   constexpr int LPR = HT / 8;               // lanes per weight row (16 B each)
-  constexpr int RPI = kBlock / LPR;         // weight rows per load
+  constexpr int RPI = BLK / LPR;         // weight rows per load
   constexpr int NI = kMcCK / RPI;           // weight loads per lane per chunk
   constexpr int WSTR = HT + 16;             // LDS weight row stride (elements)
   constexpr int KS = kMcCK / 32;            // MFMA K steps per chunk
@@ -131,10 +141,10 @@ __device__ __forceinline__ void mc_tile(const SpmmArgs& a, const int block) {
   constexpr int RB = HT * 2;                 // DMA variant: bytes per LDS weight row (no padding)
   constexpr int SB = kMcCK * RB;             // DMA variant: weight bytes per stage
   constexpr int NFA = RBT * KS;              // DMA variant: activation fragments (1 KB) per chunk
-  constexpr int NA = (NFA + 3) / 4;          // DMA variant: activation fragments each wave loads per chunk
+  constexpr int NA = (NFA + NWV - 1) / NWV;  // DMA variant: activation fragments each wave loads per chunk
   constexpr int SA = NFA * 1024;             // DMA variant: activation bytes per stage
   // (waves without a fragment of their own load one into a spare 1 KB that is never read)
-  constexpr int kLdsBytes = DMA ? S * (SB + SA) + (4 * NA > NFA ? 1024 : 0) : 2 * kMcCK * WSTR * (int)sizeof(T);
+  constexpr int kLdsBytes = DMA ? S * (SB + SA) + (NWV * NA > NFA ? 1024 : 0) : 2 * kMcCK * WSTR * (int)sizeof(T);
   // The whole static LDS is the staging (the split-K tail reuses its first
   // word once every wave is past the main loop).
   __shared__ __attribute__((aligned(16))) char lds[kLdsBytes];
@@ -204,7 +214,7 @@ __device__ __forceinline__ void mc_tile(const SpmmArgs& a, const int block) {
     // one in-order vmcnt wait covers both and no load into registers is in
     // flight across the ring: the compiler's own wait for such a load, at
     // the ring's loop header, emptied the ring once every S chunks. Lane tid
-    // fills 16 B at byte i * kBlock * 16 + tid * 16 of a stage: row
+    // fills 16 B at byte i * BLK * 16 + tid * 16 of a stage: row
     // wrow + i * RPI, physical slot tid % LPR, which holds logical 16-B
     // column slot (tid % LPR) ^ sw(row), sw(row) = 2 * (row & 3); the four
     // rows one 16-lane transposed read addresses then fall in four distinct
@@ -227,12 +237,12 @@ __device__ __forceinline__ void mc_tile(const SpmmArgs& a, const int block) {
       for (int i = 0; i < NI; ++i) {
         const int r = live ? min(k * kMcCK + wrow + i * RPI, cw - 1) : cw - 1;
         __builtin_amdgcn_global_load_lds(md + (size_t)(c0 + r) * (size_t)h + gcol_d,
-                                         (lds_void*)(lds + s * SB + i * kBlock * 16 + wave * 1024), 16, 0, kMcNtAux);
+                                         (lds_void*)(lds + s * SB + i * BLK * 16 + wave * 1024), 16, 0, kMcNtAux);
       }
       const int q = c0 / kMcCK + min(k, nch - 1);
 #pragma unroll
       for (int i = 0; i < NA; ++i) {
-        const int f = wv + 4 * i;
+        const int f = wv + NWV * i;
         const bool own = f < NFA;
         const int ks = own ? f / RBT : 0, j = own ? f % RBT : 0;
         const size_t frag = ((size_t)q * KS + ks) * (size_t)rbk_n + (size_t)min(j, rbk_n - 1);
@@ -299,7 +309,7 @@ __device__ __forceinline__ void mc_tile(const SpmmArgs& a, const int block) {
 #pragma unroll
           for (int i = 0; i < NI; ++i)
             if (wrow + i * RPI >= z0)
-              *reinterpret_cast<u32x4*>(lds + s * SB + i * kBlock * 16 + tid * 16) = u32x4{0u, 0u, 0u, 0u};
+              *reinterpret_cast<u32x4*>(lds + s * SB + i * BLK * 16 + tid * 16) = u32x4{0u, 0u, 0u, 0u};
           mc_lds_wait();
           __builtin_amdgcn_s_barrier();
         }
@@ -479,7 +489,7 @@ __device__ __forceinline__ void mc_tile(const SpmmArgs& a, const int block) {
 }
 
 template <int DT, int BT, int HT, bool DMA>
-__global__ __launch_bounds__(kBlock) void nm_spmm_mc_kernel(SpmmArgs a) {
+__global__ __launch_bounds__(mc_block(BT, HT, DMA)) void nm_spmm_mc_kernel(SpmmArgs a) {
   mc_tile<DT, BT, HT, DMA>(a, (int)blockIdx.x);
 }
 
@@ -495,7 +505,7 @@ struct McGroupArgs {
 };
 
 template <int DT, int BT, int HT, bool DMA>
-__global__ __launch_bounds__(kBlock) void nm_spmm_mc_group_kernel(McGroupArgs g) {
+__global__ __launch_bounds__(mc_block(BT, HT, DMA)) void nm_spmm_mc_group_kernel(McGroupArgs g) {
   const int b = (int)blockIdx.x;
   int i = 0;
 #pragma unroll
@@ -812,7 +822,7 @@ int spmm_mc_run(int dtype, const void* x, const void* x2, long long x_row_stride
   a.rows_per_split = p.rows;
   const int bt = batch <= 16 ? 0 : (batch <= 32 ? 1 : (batch <= 64 ? 2 : 3));
   const McFn fn = (dtype == NM_DTYPE_F16 ? kMcKernelsF16 : kMcKernelsBF16)[p.cfg][bt];
-  hipLaunchKernelGGL(fn, dim3(p.blocks), dim3(kBlock), 0, st, a);
+  hipLaunchKernelGGL(fn, dim3(p.blocks), dim3(mc_block(16 << bt, kMcTileCols[p.cfg], p.cfg >= 3)), 0, st, a);
   e = hipGetLastError();
   return e == hipSuccess ? NM_OK : (int)e;
 }
@@ -959,7 +969,7 @@ int nm_spmm_mc_group(int dtype, const void* x, long long x_row_stride, int batch
   if (e != hipSuccess) return (int)e;
   const int bt = batch <= 16 ? 0 : (batch <= 32 ? 1 : (batch <= 64 ? 2 : 3));
   const McGroupFn fn = (dtype == NM_DTYPE_F16 ? kMcGroupKernelsF16 : kMcGroupKernelsBF16)[p.cfg][bt];
-  hipLaunchKernelGGL(fn, dim3(p.blocks), dim3(kBlock), 0, st, g);
+  hipLaunchKernelGGL(fn, dim3(p.blocks), dim3(mc_block(16 << bt, kMcTileCols[p.cfg], p.cfg >= 3)), 0, st, g);
   e = hipGetLastError();
   return e == hipSuccess ? NM_OK : (int)e;
 }

@@ -404,6 +404,35 @@ int nm_gather_columns(int dtype, const void* x, long long x_row_stride, int rows
                       int nnz, int m, void* out, long long out_row_stride, void* stream);
 
 /*
+ * nm_gather_columns of round(silu(gate) * up): the product formed in fp32 at
+ * the gathered positions with expf, a division and one rounding.
+ */
+int nm_gather_columns_silu_mul(int dtype, const void* gate, const void* up, long long x_row_stride, int rows,
+                               const uint8_t* mat_index, int w, int nnz, int m, void* out, long long out_row_stride,
+                               void* stream);
+
+/*
+ * The matrix-core product for 1 <= rows <= NM_ROWS_MAX rows (long prompts,
+ * large batches) of n <= NM_MC_MAX_GROUP products of the same activations
+ * (fp16 / bf16): one gather launch and one product launch over output tiles,
+ * row tiles and splits. With `up` (n = 1) the activations are round(silu(x) *
+ * up) as nm_gather_columns_silu_mul forms them. x (and up) rows x_row_stride
+ * >= K elements apart, out[i] rows out_row_stride[i] >= h[i] apart. `scratch`
+ * (nm_spmm_rows_scratch_bytes, any contents, 256-byte aligned) holds the
+ * gathered activations and the split partials; of `workspace` (256-byte
+ * aligned) only the zeroed arrival counters are used. splits 1 to 8, 0 = the
+ * library's choice. fp32 accumulation, one rounding; splits summed in order.
+ */
+#define NM_ROWS_MAX 65536
+size_t nm_spmm_rows_scratch_bytes(int rows, int n, const int* h, int w, int nnz, int m, int splits);
+int nm_spmm_rows_plan(int rows, int n, const int* h, int w, int nnz, int m, int splits, int* out_splits,
+                      int* out_blocks);
+int nm_spmm_rows(int dtype, const void* x, const void* up, long long x_row_stride, int rows, int n,
+                 const void* const* mat_data, const uint8_t* const* mat_index, void* const* out,
+                 const long long* out_row_stride, const int* h, void* scratch, size_t scratch_bytes, void* workspace,
+                 size_t workspace_bytes, int w, int nnz, int m, int splits, void* stream);
+
+/*
  * Configuration introspection. nm_config_describe writes a short text such as
  * "th32_u8" into buf (ids nm_num_configs() + j describe pair configuration j);
  * nm_gemv_plan reports the configuration and split count the library would

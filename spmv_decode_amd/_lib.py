@@ -30,6 +30,7 @@ NM_KIND_GROUPED, NM_KIND_GATE_UP = 0, 1
 NM_MAX_BATCH = 8
 NM_MC_MAX_BATCH = 128
 NM_MC_MAX_GROUP = 4
+NM_ROWS_MAX = 65536
 NM_STATIC_SCRATCH_BYTES = NM_TICKET_BYTES + (16 << 20)
 
 _vp = ctypes.c_void_p
@@ -92,6 +93,11 @@ ABI = {
                               ctypes.POINTER(_ll), _ip, _vp, _sz, _i, _i, _i, _i, _i, _vp]),
     "nm_spmm_mc_group_plan": (_i, [_i, _i, _ip, _i, _i, _i, _i, _i, _ip, _ip, _ip, _ip]),
     "nm_gather_columns": (_i, [_i, _vp, _ll, _i, _vp, _i, _i, _i, _vp, _ll, _vp]),
+    "nm_gather_columns_silu_mul": (_i, [_i, _vp, _vp, _ll, _i, _vp, _i, _i, _i, _vp, _ll, _vp]),
+    "nm_spmm_rows_scratch_bytes": (_sz, [_i, _i, _ip, _i, _i, _i, _i]),
+    "nm_spmm_rows_plan": (_i, [_i, _i, _ip, _i, _i, _i, _i, _ip, _ip]),
+    "nm_spmm_rows": (_i, [_i, _vp, _vp, _ll, _i, _i, ctypes.POINTER(_vp), ctypes.POINTER(_vp), ctypes.POINTER(_vp),
+                          ctypes.POINTER(_ll), _ip, _vp, _sz, _vp, _sz, _i, _i, _i, _i, _vp]),
     "nm_attention_decode_workspace_bytes": (_sz, [_i, _i, _i, _i, _i]),
     "nm_attention_decode": (_i, [_i, _vp, _ll, _vp, _ll, _vp, _ll, _vp, _vp, _vp, _sz, _i, _i, _i, _i, _i, _vp]),
     "nm_config_describe": (_i, [_i, ctypes.c_char_p, _i]),
@@ -192,6 +198,16 @@ def spmm_mc_group_plan(batch: int, hs, w: int, nnz: int, m: int, config_id: int 
     check(rc, "nm_spmm_mc_group_plan")
     return {"config_id": cfg.value, "splits": sp.value, "blocks": blocks.value, "rows_per_split": rows.value,
             "config": MC_CONFIGS[cfg.value]}
+
+
+def spmm_rows_plan(rows: int, hs, w: int, nnz: int, m: int, splits: int = 0) -> dict:
+    """Split count and grid size of an nm_spmm_rows launch."""
+    n = len(hs)
+    harr = (ctypes.c_int * max(n, 1))(*hs)
+    sp, blocks = ctypes.c_int(), ctypes.c_int()
+    rc = load().nm_spmm_rows_plan(rows, n, harr, w, nnz, m, splits, ctypes.byref(sp), ctypes.byref(blocks))
+    check(rc, "nm_spmm_rows_plan")
+    return {"splits": sp.value, "blocks": blocks.value}
 
 
 def describe(config_id: int) -> str:

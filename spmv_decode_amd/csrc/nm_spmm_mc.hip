@@ -38,6 +38,7 @@
 //    Deterministic for a given plan; not bit-identical to the GEMV (the
 //    matrix core's dot products have their own order).
 #include "nm_mfma.h"
+#include "nm_spmm_mc.h"
 
 namespace nm_hip {
 namespace {
@@ -61,6 +62,7 @@ constexpr int mc_stages(int ht) { return ht == 64 ? 4 : 3; }
 // 37.8 -> 35.0 us, 5120 -> 2 x 17408 at 33 / 128 rows 50.1 -> 45.9 / 79.1 -> 68.9,
 // down 17408 -> 5120 30.8 -> 28.5 at 33; up to 16 rows level (the weight stream).
 constexpr int mc_block(int bt, int ht, bool dma) { return dma && ht / (bt < 32 ? 8 : 4) >= 16 ? 512 : 256; }
+inline int ceil_div_mc(int a, int b) { return (a + b - 1) / b; }
 constexpr int kMcNtAux = 2;  // cache policy of the weight DMA: non-temporal
 
 // Inline asm with register constraints exists only in the device pass (the
@@ -493,17 +495,6 @@ __global__ __launch_bounds__(mc_block(BT, HT, DMA)) void nm_spmm_mc_kernel(SpmmA
   mc_tile<DT, BT, HT, DMA>(a, (int)blockIdx.x);
 }
 
-// Several products of the same activations in one grid (sibling Linears:
-// q/k/v, gate/up): product i owns workgroups first[i] .. first[i + 1] - 1,
-// with its own weights, gathered activations, outputs, partials and
-// arrival counters, the same tile width, batch and split count.
-constexpr int kMcMaxGroup = NM_MC_MAX_GROUP;
-struct McGroupArgs {
-  SpmmArgs p[kMcMaxGroup];
-  int first[kMcMaxGroup];
-  int n;
-};
-
 template <int DT, int BT, int HT, bool DMA>
 __global__ __launch_bounds__(mc_block(BT, HT, DMA)) void nm_spmm_mc_group_kernel(McGroupArgs g) {
   const int b = (int)blockIdx.x;
@@ -515,86 +506,216 @@ __global__ __launch_bounds__(mc_block(BT, HT, DMA)) void nm_spmm_mc_group_kernel
 
 // The gathered activations xg[b, c] = x[b, (c/nnz)*m + mat_index[c]] for
 // c < w, zero for positions outside x, for w <= c < wp and for rows past the
-// batch. Lane i writes 8 consecutive columns of one row as one 16-B store:
-// row-major (FRAG = false: rows wp apart, wp a multiple of 8; `batch` rows)
-// or in the matrix-core kernel's operand order (FRAG = true: lane i fills
-// 16-B slot i of the fragments described at nm_spmm_mc_kernel's load_a; wp
-// a multiple of 64; rbk row blocks of 16 rows).
+// batch; 8 consecutive columns of one row leave as one 16-B store: row-major
+// (FRAG = false: rows wp apart, wp a multiple of 8; `batch` rows) or in the
+// matrix-core kernels' operand order (FRAG = true: the fragments described at
+// mc_tile's load_a; wp a multiple of 64; rbk row blocks of 16 rows).
 // SDT >= 0 (an element type): the activations are round_SDT(silu(x) * x2)
 // of two inputs with the same row stride, computed in fp32 as the gate/up
-// pair's epilogue does, only at the gathered positions.
-template <bool FRAG, int SDT = -1>
-__device__ __forceinline__ void gather_slot(const uint16_t* __restrict__ x, long long x_row_stride, int batch,
-                                            const uint8_t* __restrict__ mat_index, int w, int wp, int nnz, int m,
-                                            int K, int rbk, uint16_t* __restrict__ xg,
-                                            const uint16_t* __restrict__ x2 = nullptr) {
-  const int per_row = wp / 8;  // rows * per_row < 2^31 (host)
+// pair's epilogue does, only at the gathered positions; IEEE: with expf and a
+// division in place of the hardware's exp2 and reciprocal, the arithmetic of
+// the SiLU product as PyTorch forms it in fp32.
+// Product blockIdx.z of a group (sibling Linears), its own masks and output.
+struct McGatherGroup {
+  const uint8_t* mat_index[kMcMaxGroup];
+  uint16_t* xg[kMcMaxGroup];
+};
+struct GatherArgs {
+  const uint16_t* x;
+  const uint16_t* x2;
+  long long x_row_stride;
+  int batch, w, wp, nnz, m, K, rbk;
+  McGatherGroup g;
+};
+
+template <int SDT, bool IEEE>
+__device__ inline uint16_t gathered(uint16_t t, uint16_t u) {
+  if constexpr (SDT >= 0) {
+    using E = Elem<SDT>;
+    if constexpr (IEEE) {
+      const float gf = E::to_f32(t);
+      float y = gf / (1.0f + expf(-gf)) * E::to_f32(u);
+#if defined(__HIP_DEVICE_COMPILE__)
+      asm volatile("" : "+v"(y));  // the fp32 product is rounded before the element type
+#endif
+      return E::from_f32(y);
+    } else {
+      return E::from_f32(silu(E::to_f32(t)) * E::to_f32(u));
+    }
+  } else {
+    return t;
+  }
+}
+
+__device__ inline u32x4 pack8(const uint16_t (&v)[8]) {
+  u32x4 word;
+  word.x = (uint32_t)v[0] | ((uint32_t)v[1] << 16);
+  word.y = (uint32_t)v[2] | ((uint32_t)v[3] << 16);
+  word.z = (uint32_t)v[4] | ((uint32_t)v[5] << 16);
+  word.w = (uint32_t)v[6] | ((uint32_t)v[7] << 16);
+  return word;
+}
+
+// Any layout: a lane gathers its 8 columns straight from memory.
+template <bool FRAG, int SDT, bool IEEE>
+__global__ __launch_bounds__(kBlock) void nm_gather_mc_kernel(GatherArgs a) {
+  const int per_row = a.wp / 8;  // rows * per_row < 2^31 (host)
   const int i = (int)blockIdx.x * kBlock + (int)threadIdx.x;
-  if (i >= (FRAG ? 16 * rbk : batch) * per_row) return;
+  if (i >= (FRAG ? 16 * a.rbk : a.batch) * per_row) return;
+  const uint8_t* __restrict__ mat_index = a.g.mat_index[blockIdx.z];
   int b, c0;
   if (FRAG) {  // slot i: fragment i / 64 = (chunk * 2 + ks) * rbk + j, lane l = i % 64
     const int f = i >> 6, l = i & 63;
-    const int j = f % rbk, qk = f / rbk;
+    const int j = f % a.rbk, qk = f / a.rbk;
     b = 16 * j + (l & 15);
     c0 = 32 * qk + 8 * (l >> 4);
   } else {
     b = i / per_row;
     c0 = (i - b * per_row) * 8;
   }
-  const bool row_ok = b < batch;
-  const uint16_t* __restrict__ xr = x + (long long)(row_ok ? b : 0) * x_row_stride;
+  const bool row_ok = b < a.batch;
+  const long long row = (long long)(row_ok ? b : 0) * a.x_row_stride;
   uint16_t v[8];
 #pragma unroll
   for (int e = 0; e < 8; ++e) {
     const int c = c0 + e;
-    const int cc = c < w ? c : w - 1;  // clamped: the load stays in range
-    const int p = (cc / nnz) * m + (int)mat_index[cc];
-    uint16_t t = xr[p < K ? p : 0];
-    if constexpr (SDT >= 0) {
-      using E = Elem<SDT>;
-      const uint16_t u = x2[(long long)(row_ok ? b : 0) * x_row_stride + (p < K ? p : 0)];
-      t = E::from_f32(silu(E::to_f32(t)) * E::to_f32(u));
-    }
-    v[e] = (row_ok && c < w && p < K) ? t : (uint16_t)0;
+    const int cc = c < a.w ? c : a.w - 1;  // clamped: the load stays in range
+    const int p = (cc / a.nnz) * a.m + (int)mat_index[cc];
+    const uint16_t t = a.x[row + (p < a.K ? p : 0)];
+    const uint16_t u = SDT >= 0 ? a.x2[row + (p < a.K ? p : 0)] : (uint16_t)0;
+    v[e] = (row_ok && c < a.w && p < a.K) ? gathered<SDT, IEEE>(t, u) : (uint16_t)0;
   }
-  u32x4 word;
-  word.x = (uint32_t)v[0] | ((uint32_t)v[1] << 16);
-  word.y = (uint32_t)v[2] | ((uint32_t)v[3] << 16);
-  word.z = (uint32_t)v[4] | ((uint32_t)v[5] << 16);
-  word.w = (uint32_t)v[6] | ((uint32_t)v[7] << 16);
-  *reinterpret_cast<u32x4*>(xg + (FRAG ? (long long)i * 8 : (long long)b * wp + c0)) = word;
+  *reinterpret_cast<u32x4*>(a.g.xg[blockIdx.z] + (FRAG ? (long long)i * 8 : (long long)b * a.wp + c0)) = pack8(v);
 }
 
-template <bool FRAG>
-__global__ __launch_bounds__(kBlock) void nm_gather_mc_kernel(const uint16_t* __restrict__ x, long long x_row_stride,
-                                                            int batch, const uint8_t* __restrict__ mat_index, int w,
-                                                            int wp, int nnz, int m, int K, int rbk,
-                                                            uint16_t* __restrict__ xg) {
-  gather_slot<FRAG>(x, x_row_stride, batch, mat_index, w, wp, nnz, m, K, rbk, xg);
+// Through LDS, for large gathers: a workgroup takes kGC compressed columns of
+// kGR rows. Their groups read one window of x (kGC m / nnz columns and up to a
+// group more), whose rows are loaded 16 B per lane; the 2-byte gathers then read
+// LDS, where the direct form's cost the vector memory path a cache line each.
+// Graph replay, fp16 at 32:64, direct / through LDS (us): 4096 columns of input,
+// 500 / 1024 / 2048 rows 4.1 / 5.0, 5.9 / 5.5, 9.5 / 6.9; 14336 columns, 200 / 500
+// / 2048 rows 4.9 / 5.3, 8.6 / 6.6, 28.3 / 22.3; small ones 2.7 / 3.8: so from
+// kGatherLds gathered elements on. Positions outside the window (a mask that
+// names another group) are loaded one by one.
+constexpr long long kGatherLds = 1 << 21;
+constexpr int kGC = 128, kGR = 32, kGWin = 512;
+template <bool FRAG, int SDT, bool IEEE>
+__global__ __launch_bounds__(kBlock) void nm_gather_mc_lds_kernel(GatherArgs a) {
+  constexpr int NIN = SDT >= 0 ? 2 : 1;
+  constexpr int STR = kGWin + 2;  // an odd number of words: the rows start in different banks
+  __shared__ __attribute__((aligned(16))) uint16_t xs[NIN][kGR * STR];
+  const uint8_t* __restrict__ mat_index = a.g.mat_index[blockIdx.z];
+  uint16_t* __restrict__ xg = a.g.xg[blockIdx.z];
+  const int tid = threadIdx.x;
+  const int cb = (int)blockIdx.x * kGC, rb = (int)blockIdx.y * kGR;
+  // the window: the groups of columns cb .. min(cb + kGC, w) - 1, from a multiple of 8
+  const int last = min(cb + kGC, a.w) - 1;
+  const int g0 = min(cb, last) / a.nnz;
+  const int win0 = (g0 * a.m) & ~7;
+  const int win = min((last / a.nnz + 1) * a.m, a.K) - win0;  // <= kGWin (host); K a multiple of 8
+  const int words = (win + 7) / 8;                            // 16-B words per row
+
+  // This lane's 8 columns (of two rows), their positions.
+  const int c = cb + (FRAG ? 32 * (tid >> 6) + 8 * ((tid & 63) >> 4) : 8 * (tid & 15));
+  const int r0 = FRAG ? (tid & 15) : (tid >> 4);
+  uint8_t idx[8];
+  if (c + 8 <= a.w && ((uintptr_t)mat_index & 7u) == 0) {
+    const unsigned long long q = *reinterpret_cast<const unsigned long long*>(mat_index + c);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) idx[e] = (uint8_t)(q >> (8 * e));
+  } else {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) idx[e] = mat_index[min(c + e, a.w - 1)];
+  }
+  for (int i = tid; i < kGR * words; i += kBlock) {
+    const int r = i / words, k = i - r * words;
+    const long long src = (long long)min(rb + r, a.batch - 1) * a.x_row_stride + win0 + 8 * k;
+#pragma unroll
+    for (int q = 0; q < NIN; ++q) {
+      const u32x4 v = *reinterpret_cast<const u32x4*>((q == 0 ? a.x : a.x2) + src);
+      uint32_t* dst = reinterpret_cast<uint32_t*>(&xs[q][r * STR + 8 * k]);
+      dst[0] = v.x, dst[1] = v.y, dst[2] = v.z, dst[3] = v.w;
+    }
+  }
+  __syncthreads();
+  if (c >= a.wp) return;
+  int pos[8];
+  int grp = min(c, a.w - 1) / a.nnz, in = min(c, a.w - 1) - grp * a.nnz;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    pos[e] = grp * a.m + (int)idx[e];
+    if (++in == a.nnz) in = 0, ++grp;
+  }
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const int r = r0 + 16 * h, b = rb + r;
+    if (b >= (FRAG ? 16 * a.rbk : a.batch)) break;
+    uint16_t v[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const int rel = pos[e] - win0;
+      const bool here = (unsigned)rel < (unsigned)win;
+      uint16_t t = xs[0][r * STR + (here ? rel : 0)], u = NIN > 1 ? xs[NIN - 1][r * STR + (here ? rel : 0)] : (uint16_t)0;
+      const bool ok = b < a.batch && c + e < a.w && pos[e] < a.K;
+      if (ok && !here) {
+        t = a.x[(long long)b * a.x_row_stride + pos[e]];
+        if (NIN > 1) u = a.x2[(long long)b * a.x_row_stride + pos[e]];
+      }
+      v[e] = ok ? gathered<SDT, IEEE>(t, u) : (uint16_t)0;
+    }
+    // FRAG: fragment (c / 32) * rbk + b / 16, lane tid % 64
+    const long long off = FRAG ? (((long long)(c >> 5) * a.rbk + (b >> 4)) * 64 + (tid & 63)) * 8
+                               : (long long)b * a.wp + c;
+    *reinterpret_cast<u32x4*>(xg + off) = pack8(v);
+  }
 }
 
-// The operand-order gather of round_SDT(silu(gate) * up).
-template <int SDT>
-__global__ __launch_bounds__(kBlock) void nm_gather_mc_silu_kernel(const uint16_t* __restrict__ gate,
-                                                                 const uint16_t* __restrict__ up,
-                                                                 long long x_row_stride, int batch,
-                                                                 const uint8_t* __restrict__ mat_index, int w,
-                                                                 int wp, int nnz, int m, int K, int rbk,
-                                                                 uint16_t* __restrict__ xg) {
-  gather_slot<true, SDT>(gate, x_row_stride, batch, mat_index, w, wp, nnz, m, K, rbk, xg, up);
+// One gather launch (n products). `rows` of the output: the batch, or whole
+// 16-row blocks in operand order.
+template <bool FRAG, int SDT, bool IEEE>
+void launch_gather(const GatherArgs& a, int n, hipStream_t st) {
+  const int rows = FRAG ? 16 * a.rbk : a.batch;
+  // the LDS form: aligned rows, and windows of at most kGWin columns (8 of them for win0's rounding)
+  const long long groups = kGC % a.nnz == 0 ? kGC / a.nnz : (a.nnz % kGC == 0 ? 1 : kGC / a.nnz + 2);
+  const bool lds = (long long)rows * a.wp >= kGatherLds && a.K % 8 == 0 && a.x_row_stride % 8 == 0 && ((uintptr_t)a.x & 15u) == 0 &&
+                   (SDT < 0 || ((uintptr_t)a.x2 & 15u) == 0) && groups * a.m + 8 <= kGWin &&
+                   rows <= kGR * 65535;  // grid y
+  if (lds)
+    hipLaunchKernelGGL((nm_gather_mc_lds_kernel<FRAG, SDT, IEEE>),
+                       dim3((unsigned)ceil_div_mc(a.wp, kGC), (unsigned)ceil_div_mc(rows, kGR), (unsigned)n),
+                       dim3(kBlock), 0, st, a);
+  else
+    hipLaunchKernelGGL((nm_gather_mc_kernel<FRAG, SDT, IEEE>),
+                       dim3((unsigned)(((long long)rows * (a.wp / 8) + kBlock - 1) / kBlock), 1, (unsigned)n),
+                       dim3(kBlock), 0, st, a);
 }
 
-// The operand-order gathers of a group's products, product blockIdx.y each.
-struct McGatherGroup {
-  const uint8_t* mat_index[kMcMaxGroup];
-  uint16_t* xg[kMcMaxGroup];
-};
+// Plain (x2 null) or of the SiLU product, for the element type.
+template <bool FRAG, bool IEEE>
+void launch_gather(int dtype, const GatherArgs& a, int n, hipStream_t st) {
+  if (!a.x2)
+    launch_gather<FRAG, -1, false>(a, n, st);  // fp16 and bf16 alike: a copy of 16-bit words
+  else if (dtype == NM_DTYPE_F16)
+    launch_gather<FRAG, NM_DTYPE_F16, IEEE>(a, n, st);
+  else
+    launch_gather<FRAG, NM_DTYPE_BF16, IEEE>(a, n, st);
+}
 
-__global__ __launch_bounds__(kBlock) void nm_gather_mc_group_kernel(const uint16_t* __restrict__ x,
-                                                                  long long x_row_stride, int batch, int w, int wp,
-                                                                  int nnz, int m, int K, int rbk, McGatherGroup gg) {
-  const int i = (int)blockIdx.y;
-  gather_slot<true>(x, x_row_stride, batch, gg.mat_index[i], w, wp, nnz, m, K, rbk, gg.xg[i]);
+GatherArgs gather_args(const void* x, const void* x2, long long x_row_stride, int batch, int w, int wp, int nnz, int m,
+                       long long K, int rbk) {
+  GatherArgs a;
+  memset(&a, 0, sizeof(a));
+  a.x = static_cast<const uint16_t*>(x);
+  a.x2 = static_cast<const uint16_t*>(x2);
+  a.x_row_stride = x_row_stride;
+  a.batch = batch;
+  a.w = w;
+  a.wp = wp;
+  a.nnz = nnz;
+  a.m = m;
+  a.K = (int)K;
+  a.rbk = rbk;
+  return a;
 }
 
 typedef void (*McFn)(SpmmArgs);
@@ -628,10 +749,10 @@ const McGroupFn kMcGroupKernelsBF16[kMcNumConfigs][4] = NM_MC_TABLE(NM_DTYPE_BF1
 #undef NM_MC_ROW
 #undef NM_MC_ROW3
 
+
 constexpr int kMcTileCols[kMcNumConfigs] = {64, 128, 256, 64, 128, 256};
 constexpr int kMcCUs = 256;  // MI355X compute units; split counts aim at about this many workgroups
 
-inline int ceil_div_mc(int a, int b) { return (a + b - 1) / b; }
 
 struct McPlan {
   int cfg, splits, rows, tiles, blocks, wp;
@@ -769,6 +890,60 @@ int make_mc_plan(int batch, int h, int w, int nnz, int m, int cfg, int splits, M
   return make_mc_plan(batch, 1, &h, w, nnz, m, cfg, splits, p);
 }
 
+// The plan of nm_spmm_rows: the split count whose rounds of workgroups (one per
+// CU) take the fewest chunk times, a split's handoff counted as 6 + 3 per split
+// (fitted to graph-replay sweeps of 1-6 splits at the Llama-3.1-8B and Qwen3
+// shapes, 129-2048 rows: a chunk takes about 0.5 us, 2 / 4 splits' handoffs 6 / 9). Scratch layout: the products' gathered
+// activations in operand order, then their partial tiles [splits, tiles] when
+// splits > 1.
+struct RowsPlan {
+  int mt, splits, rows_per_split, blocks, wp;
+  size_t xg_bytes, part_off, scratch;
+};
+
+int make_rows_plan(int rows, int n, const int* hs, int w, int nnz, int m, int splits, RowsPlan* p) {
+  if (rows < 1 || rows > NM_ROWS_MAX || n < 1 || n > kMcMaxGroup || !hs) return NM_ERR_BAD_SHAPE;
+  if (w <= 0 || nnz <= 0 || m <= 0 || m > 256 || nnz > m) return NM_ERR_BAD_SHAPE;
+  long long hsum = 0;
+  for (int i = 0; i < n; ++i) {
+    if (hs[i] <= 0) return NM_ERR_BAD_SHAPE;
+    if (hs[i] % kRowsTile != 0) return NM_ERR_H_NOT_MULTIPLE_128;
+    if ((long long)rows * (long long)hs[i] > 0x7fffffffLL) return NM_ERR_BAD_SHAPE;  // 32-bit output offsets
+    if (2LL * kMcCK * (long long)hs[i] > 0x7fffffffLL) return NM_ERR_BAD_SHAPE;      // 32-bit weight offsets
+    hsum += hs[i];
+  }
+  if (w % nnz != 0) return NM_ERR_W_NOT_MULTIPLE_NNZ;
+  if ((long long)(w / nnz) * (long long)m > 0x7fffffffLL || w > 0x7fffffff - kMcCK) return NM_ERR_BAD_SHAPE;
+  const int rbk = ceil_div_mc(rows, 16);
+  p->wp = ceil_div_mc(w, kMcCK) * kMcCK;
+  if (16LL * rbk * (p->wp / 8) > 0x7fffffffLL) return NM_ERR_BAD_SHAPE;
+  p->mt = ceil_div_mc(rows, kRowsTile);
+  const long long tiles = hsum / kRowsTile * p->mt;
+  if (tiles > kMaxTickets) return NM_ERR_BAD_SHAPE;
+  const int chunks = p->wp / kMcCK;
+  double best = 0.0;
+  p->splits = 0;
+  for (int s = 1; s <= 8; ++s) {
+    if (splits > 0 && s != splits) continue;
+    const int per = ceil_div_mc(chunks, s < chunks ? s : chunks);
+    const int eff = ceil_div_mc(chunks, per);
+    if (splits <= 0 && eff != s) continue;
+    const long long rounds = (tiles * eff + kMcCUs - 1) / kMcCUs;
+    const double cost = (double)rounds * per + (eff > 1 ? 6.0 + 3.0 * eff : 0.0);
+    if (p->splits == 0 || cost < best) {
+      best = cost;
+      p->splits = eff;
+      p->rows_per_split = per * kMcCK;
+    }
+  }
+  if (p->splits == 0) return NM_ERR_BAD_CONFIG;
+  p->blocks = (int)(tiles * p->splits);
+  p->xg_bytes = (size_t)rbk * 16 * (size_t)p->wp * 2;  // a multiple of 2 KB
+  p->part_off = (size_t)n * p->xg_bytes;
+  p->scratch = p->part_off + (p->splits > 1 ? (size_t)p->splits * (size_t)tiles * kRowsPartBytes : (size_t)0);
+  return NM_OK;
+}
+
 // nm_spmm_mc, and with x2 (the up projection's output, rows x_row_stride
 // apart like x) nm_spmm_mc_silu_mul: the gather then forms round_T(silu(x)
 // * x2) at the gathered positions.
@@ -787,18 +962,10 @@ int spmm_mc_run(int dtype, const void* x, const void* x2, long long x_row_stride
   hipStream_t st = static_cast<hipStream_t>(stream);
   void* xg = static_cast<char*>(workspace) + p.xg_off;
   const int rbk = ceil_div_mc(batch, 16);  // row blocks of 16 stored (operand order, zero rows past the batch)
-  const long long gathered = (long long)16 * rbk * (long long)(p.wp / 8);
-  const unsigned gblocks = (unsigned)((gathered + kBlock - 1) / kBlock);
-  if (!x2)
-    hipLaunchKernelGGL(nm_gather_mc_kernel<true>, dim3(gblocks), dim3(kBlock), 0, st,
-                       static_cast<const uint16_t*>(x), x_row_stride, batch, mat_index, w, p.wp, nnz, m, (int)K,
-                       rbk, static_cast<uint16_t*>(xg));  // fp16 and bf16 alike: a copy of 16-bit words
-  else
-    hipLaunchKernelGGL(dtype == NM_DTYPE_F16 ? nm_gather_mc_silu_kernel<NM_DTYPE_F16>
-                                             : nm_gather_mc_silu_kernel<NM_DTYPE_BF16>,
-                       dim3(gblocks), dim3(kBlock), 0, st, static_cast<const uint16_t*>(x),
-                       static_cast<const uint16_t*>(x2), x_row_stride, batch, mat_index, w, p.wp, nnz, m, (int)K,
-                       rbk, static_cast<uint16_t*>(xg));
+  GatherArgs ga = gather_args(x, x2, x_row_stride, batch, w, p.wp, nnz, m, K, rbk);
+  ga.g.mat_index[0] = mat_index;
+  ga.g.xg[0] = static_cast<uint16_t*>(xg);
+  launch_gather<true, false>(dtype, ga, 1, st);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return (int)e;
   SpmmArgs a;
@@ -824,6 +991,28 @@ int spmm_mc_run(int dtype, const void* x, const void* x2, long long x_row_stride
   const McFn fn = (dtype == NM_DTYPE_F16 ? kMcKernelsF16 : kMcKernelsBF16)[p.cfg][bt];
   hipLaunchKernelGGL(fn, dim3(p.blocks), dim3(mc_block(16 << bt, kMcTileCols[p.cfg], p.cfg >= 3)), 0, st, a);
   e = hipGetLastError();
+  return e == hipSuccess ? NM_OK : (int)e;
+}
+
+// nm_gather_columns, and with x2 nm_gather_columns_silu_mul.
+int gather_columns_run(int dtype, const void* x, const void* x2, long long x_row_stride, int rows,
+                       const uint8_t* mat_index, int w, int nnz, int m, void* out, long long out_row_stride,
+                       void* stream) {
+  if (dtype != NM_DTYPE_F16 && dtype != NM_DTYPE_BF16) return NM_ERR_BAD_CONFIG;
+  if (rows < 1 || w <= 0 || nnz <= 0 || m <= 0 || m > 256 || nnz > m || w % nnz != 0) return NM_ERR_BAD_SHAPE;
+  if (!x || !mat_index || !out) return NM_ERR_NULL_POINTER;
+  const long long K = (long long)(w / nnz) * (long long)m;
+  const long long wp = ((long long)w + 7) / 8 * 8;
+  if (K > 0x7fffffffLL || x_row_stride < K || out_row_stride < wp || out_row_stride % 8 != 0 ||
+      out_row_stride > 0x7fffffffLL || (long long)rows * (out_row_stride / 8) > 0x7fffffffLL)
+    return NM_ERR_BAD_SHAPE;
+  if (((uintptr_t)out & 15u) != 0) return NM_ERR_MISALIGNED;
+  // rows of out_row_stride elements: every column past w is written as zero
+  GatherArgs ga = gather_args(x, x2, x_row_stride, rows, w, (int)out_row_stride, nnz, m, K, 0);
+  ga.g.mat_index[0] = mat_index;
+  ga.g.xg[0] = static_cast<uint16_t*>(out);
+  launch_gather<false, true>(dtype, ga, 1, static_cast<hipStream_t>(stream));
+  const hipError_t e = hipGetLastError();
   return e == hipSuccess ? NM_OK : (int)e;
 }
 
@@ -853,22 +1042,7 @@ int nm_spmm_mc_plan(int batch, int h, int w, int nnz, int m, int config_id, int 
 
 int nm_gather_columns(int dtype, const void* x, long long x_row_stride, int rows, const uint8_t* mat_index, int w,
                       int nnz, int m, void* out, long long out_row_stride, void* stream) {
-  if (dtype != NM_DTYPE_F16 && dtype != NM_DTYPE_BF16) return NM_ERR_BAD_CONFIG;
-  if (rows < 1 || w <= 0 || nnz <= 0 || m <= 0 || m > 256 || nnz > m || w % nnz != 0) return NM_ERR_BAD_SHAPE;
-  if (!x || !mat_index || !out) return NM_ERR_NULL_POINTER;
-  const long long K = (long long)(w / nnz) * (long long)m;
-  const long long wp = ((long long)w + 7) / 8 * 8;
-  if (K > 0x7fffffffLL || x_row_stride < K || out_row_stride < wp || out_row_stride % 8 != 0 ||
-      out_row_stride > 0x7fffffffLL || (long long)rows * (out_row_stride / 8) > 0x7fffffffLL)
-    return NM_ERR_BAD_SHAPE;
-  if (((uintptr_t)out & 15u) != 0) return NM_ERR_MISALIGNED;
-  // rows of out_row_stride elements: every column past w is written as zero
-  const long long lanes = (long long)rows * (out_row_stride / 8);
-  hipLaunchKernelGGL(nm_gather_mc_kernel<false>, dim3((unsigned)((lanes + kBlock - 1) / kBlock)), dim3(kBlock), 0,
-                     static_cast<hipStream_t>(stream), static_cast<const uint16_t*>(x), x_row_stride, rows,
-                     mat_index, w, (int)out_row_stride, nnz, m, (int)K, 0, static_cast<uint16_t*>(out));
-  const hipError_t e = hipGetLastError();
-  return e == hipSuccess ? NM_OK : (int)e;
+  return gather_columns_run(dtype, x, nullptr, x_row_stride, rows, mat_index, w, nnz, m, out, out_row_stride, stream);
 }
 
 int nm_spmm_mc(int dtype, const void* x, long long x_row_stride, int batch, const void* mat_data,
@@ -961,10 +1135,9 @@ int nm_spmm_mc_group(int dtype, const void* x, long long x_row_stride, int batch
     block_off += tiles * p.splits;
     part_off += p.splits > 1 ? (size_t)p.splits * (size_t)batch * (size_t)h[i] : (size_t)0;
   }
-  const long long gathered = (long long)16 * rbk * (long long)(p.wp / 8);
-  const unsigned gblocks = (unsigned)((gathered + kBlock - 1) / kBlock);
-  hipLaunchKernelGGL(nm_gather_mc_group_kernel, dim3(gblocks, (unsigned)n), dim3(kBlock), 0, st,
-                     static_cast<const uint16_t*>(x), x_row_stride, batch, w, p.wp, nnz, m, (int)K, rbk, gg);
+  GatherArgs ga = gather_args(x, nullptr, x_row_stride, batch, w, p.wp, nnz, m, K, rbk);
+  ga.g = gg;
+  launch_gather<true, false>(dtype, ga, n, st);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return (int)e;
   const int bt = batch <= 16 ? 0 : (batch <= 32 ? 1 : (batch <= 64 ? 2 : 3));
@@ -972,6 +1145,96 @@ int nm_spmm_mc_group(int dtype, const void* x, long long x_row_stride, int batch
   hipLaunchKernelGGL(fn, dim3(p.blocks), dim3(mc_block(16 << bt, kMcTileCols[p.cfg], p.cfg >= 3)), 0, st, g);
   e = hipGetLastError();
   return e == hipSuccess ? NM_OK : (int)e;
+}
+
+size_t nm_spmm_rows_scratch_bytes(int rows, int n, const int* h, int w, int nnz, int m, int splits) {
+  RowsPlan p;
+  return make_rows_plan(rows, n, h, w, nnz, m, splits, &p) == NM_OK ? p.scratch : 0;
+}
+
+int nm_spmm_rows_plan(int rows, int n, const int* h, int w, int nnz, int m, int splits, int* out_splits,
+                      int* out_blocks) {
+  RowsPlan p;
+  const int rc = make_rows_plan(rows, n, h, w, nnz, m, splits, &p);
+  if (rc != NM_OK) return rc;
+  if (out_splits) *out_splits = p.splits;
+  if (out_blocks) *out_blocks = p.blocks;
+  return NM_OK;
+}
+
+int nm_spmm_rows(int dtype, const void* x, const void* up, long long x_row_stride, int rows, int n,
+                 const void* const* mat_data, const uint8_t* const* mat_index, void* const* out,
+                 const long long* out_row_stride, const int* h, void* scratch, size_t scratch_bytes, void* workspace,
+                 size_t workspace_bytes, int w, int nnz, int m, int splits, void* stream) {
+  if (dtype != NM_DTYPE_F16 && dtype != NM_DTYPE_BF16) return NM_ERR_BAD_CONFIG;
+  if (!mat_data || !mat_index || !out || !out_row_stride || !h) return NM_ERR_NULL_POINTER;
+  if (up && n != 1) return NM_ERR_BAD_SHAPE;
+  RowsPlan p;
+  const int rc = make_rows_plan(rows, n, h, w, nnz, m, splits, &p);
+  if (rc != NM_OK) return rc;
+  if (!x || !scratch || !workspace) return NM_ERR_NULL_POINTER;
+  const long long K = (long long)(w / nnz) * (long long)m;
+  if (x_row_stride < K) return NM_ERR_BAD_SHAPE;
+  for (int i = 0; i < n; ++i) {
+    if (!mat_data[i] || !mat_index[i] || !out[i]) return NM_ERR_NULL_POINTER;
+    if (out_row_stride[i] < h[i]) return NM_ERR_BAD_SHAPE;
+    if (((uintptr_t)mat_data[i] & 15u) != 0 || ((uintptr_t)out[i] & 7u) != 0 || out_row_stride[i] % 4 != 0)
+      return NM_ERR_MISALIGNED;  // 16-B weight loads, 8-B output stores
+  }
+  if (((uintptr_t)workspace & 255u) != 0 || ((uintptr_t)scratch & 255u) != 0) return NM_ERR_MISALIGNED;
+  if (workspace_bytes < (size_t)NM_TICKET_BYTES || scratch_bytes < p.scratch) return NM_ERR_WORKSPACE;
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  const int rbk = ceil_div_mc(rows, 16);
+  McGatherGroup gg;
+  memset(&gg, 0, sizeof(gg));
+  McGroupArgs g;
+  memset(&g, 0, sizeof(g));
+  g.n = n;
+  size_t part_off = 0;
+  int tile_off = 0, block_off = 0;
+  for (int i = 0; i < n; ++i) {
+    uint16_t* xg = reinterpret_cast<uint16_t*>(static_cast<char*>(scratch) + (size_t)i * p.xg_bytes);
+    gg.mat_index[i] = mat_index[i];
+    gg.xg[i] = xg;
+    SpmmArgs& a = g.p[i];
+    const int tiles = h[i] / kRowsTile;
+    a.x = xg;
+    a.x_row_stride = rbk;  // operand-order activations: the row blocks stored
+    a.mat_data = mat_data[i];
+    a.mat_index = mat_index[i];
+    a.out = out[i];
+    a.out_row_stride = out_row_stride[i];
+    a.tickets = static_cast<uint32_t*>(workspace) + (size_t)tile_off * (size_t)p.mt;
+    a.partial = reinterpret_cast<float*>(static_cast<char*>(scratch) + p.part_off) + part_off;
+    a.batch = rows;
+    a.h = h[i];
+    a.tiles = tiles;
+    a.w = w;
+    a.nnz = nnz;
+    a.m = m;
+    a.K = (int)K;
+    a.splits = p.splits;
+    a.rows_per_split = p.rows_per_split;
+    g.first[i] = block_off;
+    tile_off += tiles;
+    block_off += tiles * p.mt * p.splits;
+    part_off += p.splits > 1 ? (size_t)p.splits * (size_t)(tiles * p.mt) * (kRowsPartBytes / 4) : (size_t)0;
+  }
+  GatherArgs ga = gather_args(x, up, x_row_stride, rows, w, p.wp, nnz, m, K, rbk);
+  ga.g = gg;
+  launch_gather<true, true>(dtype, ga, n, st);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return (int)e;
+  launch_rows_product(dtype, g, p.mt, p.blocks, st);
+  e = hipGetLastError();
+  return e == hipSuccess ? NM_OK : (int)e;
+}
+
+int nm_gather_columns_silu_mul(int dtype, const void* gate, const void* up, long long x_row_stride, int rows,
+                               const uint8_t* mat_index, int w, int nnz, int m, void* out, long long out_row_stride,
+                               void* stream) {
+  if (!up) return NM_ERR_NULL_POINTER;
+  return gather_columns_run(dtype, gate, up, x_row_stride, rows, mat_index, w, nnz, m, out, out_row_stride, stream);
 }
 
 }  // extern "C"

@@ -240,6 +240,26 @@ def library_route(rows: int, K: int, h: int) -> bool:
     return rows > _lib.NM_MC_MAX_BATCH or (rows > 64 and h <= 1024)
 
 
+def rows_route(rows: int, w: int, hs) -> bool:
+    """Whether products of one input past NM_MC_MAX_BATCH rows (16-bit, plan
+    left to the library) run on nm_spmm_rows rather than as one BLAS GEMM each:
+    from 160 rows (at 129 rows half of its second row tile is padding), several
+    products up to rows * (sum of outputs) = 12.6M, a lone one up to 768 rows
+    when it is deeper than wide (w >= h) and has more than 1024 outputs. The
+    BLAS library runs a GEMM per product, without splitting its depth, and wins
+    on wide outputs, where its 256-wide tiles read less per multiply.
+    Graph replay, gathers included, nm_spmm_rows / library (us): Llama-3.1-8B down
+    200 / 500 / 1024 rows 41 / 57, 55 / 77, 85 / 91; Qwen3-14B down 200 / 500 /
+    1024 rows 50 / 96, 85 / 99, 158 / 142; q/k/v 200 / 500 / 2048 rows 25 / 48, 29
+    / 59, 85 / 102; gate and up 200 / 333 / 500 rows 57 / 65, 76 / 80, 103 / 99; o
+    200 / 500 rows 23 / 20, 26 / 27; Qwen3-14B gate alone 200 rows 61 / 53."""
+    if rows < 160 or rows > _lib.NM_ROWS_MAX:
+        return False
+    if len(hs) > 1:
+        return rows * sum(hs) <= 3 << 22
+    return rows <= 768 and w >= hs[0] > 1024
+
+
 def nmsparse_spmm_forward_hip(x, mat_data, mat_index, w, h, BLOCK_WIDTH, VEC_WIDTH, *, out=None, config_id=-1,
                               splits=0, matrix_cores=None):
     """out[..., r, :] = W_sparse @ x[..., r, :] for every row of x ([..., rows, K]),
@@ -256,10 +276,11 @@ def nmsparse_spmm_forward_hip(x, mat_data, mat_index, w, h, BLOCK_WIDTH, VEC_WID
     (NM_MC_MAX_BATCH rows per launch; fp32 accumulation in the matrix cores'
     own order, see _lib.spmm_mc_plan). matrix_cores=None takes the matrix
     cores for NM_MAX_BATCH < rows <= NM_MC_MAX_BATCH of a 16-bit type when
-    config_id and splits are left to the library, and the library route
-    instead (library_route) past NM_MC_MAX_BATCH rows: the gathered activations (nm_gather_columns, [rows, w]) times
-    mat_data as one hipBLASLt GEMM (torch.matmul: a plain GEMM over half the
-    input width); else the small-batch kernel. True / False forces one of the
+    config_id and splits are left to the library; past NM_MC_MAX_BATCH rows
+    (library_route) nm_spmm_rows where it is faster (rows_route), elsewhere
+    the gathered activations (nm_gather_columns, [rows, w]) times mat_data as
+    one hipBLASLt GEMM (torch.matmul: a plain GEMM over half the input width);
+    else the small-batch kernel. True / False forces one of the
     two HIP kernels (True needs fp16 or bf16). config_id and splits are those
     of the kernel that runs.
     """
@@ -303,6 +324,9 @@ def nmsparse_spmm_forward_hip(x, mat_data, mat_index, w, h, BLOCK_WIDTH, VEC_WID
         raise TypeError("the matrix-core SpMM takes fp16 or bf16")
     md = _aligned(mat_data)
     lib = _lib.load()
+    if library_gemm and rows_route(rows, w, [h]):
+        _spmm_rows(x2d, [(md, mat_index)], w, BLOCK_WIDTH, VEC_WIDTH, [out])
+        return out
     if library_gemm:
         wp = (w + 7) // 8 * 8
         with torch.cuda.device(x.device):
@@ -342,8 +366,11 @@ def nmsparse_spmm_silu_mul_hip(gate, up, mat_data, mat_index, w, h, BLOCK_WIDTH,
     NM_MC_MAX_BATCH rows on the matrix cores with the SiLU product formed at
     the gathered positions inside the activation gather (nm_spmm_mc_silu_mul:
     no separate SiLU and multiply launches, one rounding, like the GEMV
-    gate/up pair's epilogue), otherwise the product formed in fp32 with one
-    rounding and then nmsparse_spmm_forward_hip. Returns [..., rows, h]."""
+    gate/up pair's epilogue), past them likewise inside the gather of
+    nm_spmm_rows or of the library GEMM (with expf and a division: the bits of
+    the product formed in fp32 with one rounding), otherwise the product formed
+    in fp32 with one rounding and then nmsparse_spmm_forward_hip. Returns
+    [..., rows, h]."""
     if gate.shape != up.shape or gate.dtype != up.dtype or gate.device != up.device:
         raise ValueError("gate and up must have one shape, dtype and device")
     K = gate.shape[-1]
@@ -351,7 +378,9 @@ def nmsparse_spmm_silu_mul_hip(gate, up, mat_data, mat_index, w, h, BLOCK_WIDTH,
     explicit = config_id >= 0 or splits > 0
     fused = (gate.dtype in (torch.float16, torch.bfloat16) and gate.is_cuda and _lib.NM_MAX_BATCH < rows
              <= _lib.NM_MC_MAX_BATCH and (explicit or not library_route(rows, K, h)))
-    if not fused:
+    wide = (gate.dtype in (torch.float16, torch.bfloat16) and gate.is_cuda and not explicit
+            and rows > _lib.NM_MC_MAX_BATCH)
+    if not (fused or wide):
         act = (torch.nn.functional.silu(gate.float()) * up.float()).to(gate.dtype)
         return nmsparse_spmm_forward_hip(act, mat_data, mat_index, w, h, BLOCK_WIDTH, VEC_WIDTH, out=out,
                                          config_id=config_id, splits=splits)
@@ -361,6 +390,10 @@ def nmsparse_spmm_silu_mul_hip(gate, up, mat_data, mat_index, w, h, BLOCK_WIDTH,
         raise TypeError("x and mat_data must have same dtype")
     if mat_index.dtype != torch.uint8:
         raise TypeError("mat_index must be uint8")
+    if h % 128 != 0:
+        raise ValueError("h must be divisible by 128")
+    if VEC_WIDTH < BLOCK_WIDTH or VEC_WIDTH > 256:
+        raise ValueError(f"need N <= M <= 256 (uint8 positions), got N={BLOCK_WIDTH}, M={VEC_WIDTH}")
     if w % BLOCK_WIDTH != 0 or K != (w // BLOCK_WIDTH) * VEC_WIDTH:
         raise ValueError(f"x has {K} columns; w={w}, N={BLOCK_WIDTH}, M={VEC_WIDTH} need {w // BLOCK_WIDTH * VEC_WIDTH}")
     if tuple(mat_data.shape) != (w, h) or not mat_data.is_contiguous():
@@ -375,7 +408,20 @@ def nmsparse_spmm_silu_mul_hip(gate, up, mat_data, mat_index, w, h, BLOCK_WIDTH,
           or out.device != gate.device or out.data_ptr() % 16):
         raise ValueError(f"out must be a contiguous, 16-byte aligned {(*lead, h)} tensor of x.dtype")
     md = _aligned(mat_data)
+    if wide and rows_route(rows, w, [h]):
+        _spmm_rows(g2d, [(md, mat_index)], w, BLOCK_WIDTH, VEC_WIDTH, [out], up2d=u2d)
+        return out
     lib = _lib.load()
+    if wide:
+        wp = (w + 7) // 8 * 8
+        with torch.cuda.device(gate.device):
+            xg = torch.empty(rows, wp, dtype=gate.dtype, device=gate.device)
+            rc = lib.nm_gather_columns_silu_mul(_DTYPE_CODE[gate.dtype], g2d.data_ptr(), u2d.data_ptr(), K, rows,
+                                                mat_index.data_ptr(), w, BLOCK_WIDTH, VEC_WIDTH, xg.data_ptr(), wp,
+                                                torch.cuda.current_stream(gate.device).cuda_stream)
+            _lib.check(rc, "nm_gather_columns_silu_mul")
+            torch.matmul(xg[:, :w], md, out=out.view(rows, h))
+        return out
     need = lib.nm_spmm_mc_workspace_bytes(rows, h, w, BLOCK_WIDTH, VEC_WIDTH, int(config_id), int(splits))
     if need == 0:
         raise ValueError("spmm shape outside what libnmsparse_hip supports")
@@ -399,7 +445,8 @@ def nmsparse_spmm_group_hip(x, mats, BLOCK_WIDTH, VEC_WIDTH, *, outs=None, confi
     NM_MC_MAX_GROUP products of the same w: one gather launch for every
     product's activations and one matrix-core launch over all their tiles
     (nm_spmm_mc_group; each product's rows equal nm_spmm_mc's with the same
-    config_id and splits). Otherwise (fewer or more rows, fp32, more
+    config_id and splits), and past them likewise on nm_spmm_rows where that
+    is faster (rows_route). Otherwise (fewer or more rows, fp32, more
     products, or with the plan left to the library past 64 rows of products
     of at most 1024 outputs: library_route) each product runs through
     nmsparse_spmm_forward_hip on its own.
@@ -417,10 +464,13 @@ def nmsparse_spmm_group_hip(x, mats, BLOCK_WIDTH, VEC_WIDTH, *, outs=None, confi
     elif len(outs) != len(mats):
         raise ValueError(f"{len(outs)} outputs for {len(mats)} products")
     explicit = config_id >= 0 or splits > 0  # a matrix-core plan named by the caller
+    one_w = all(md.shape[0] == w for md, _ in mats)
     grouped = (x.dtype in (torch.float16, torch.bfloat16) and _lib.NM_MAX_BATCH < rows <= _lib.NM_MC_MAX_BATCH
                and (explicit or not library_route(rows, K, max(hs))) and 1 < len(mats) <= _lib.NM_MC_MAX_GROUP
-               and all(md.shape[0] == w for md, _ in mats))
-    if not grouped:
+               and one_w)
+    wide = (x.dtype in (torch.float16, torch.bfloat16) and not explicit and rows > _lib.NM_MC_MAX_BATCH
+            and 1 < len(mats) <= _lib.NM_MC_MAX_GROUP and one_w and rows_route(rows, w, hs))
+    if not (grouped or wide):
         return [nmsparse_spmm_forward_hip(x, md, mi, w, h, BLOCK_WIDTH, VEC_WIDTH, out=o, config_id=config_id,
                                           splits=splits)
                 for (md, mi), h, o in zip(mats, hs, outs)]
@@ -447,6 +497,8 @@ def nmsparse_spmm_group_hip(x, mats, BLOCK_WIDTH, VEC_WIDTH, *, outs=None, confi
               or o.data_ptr() % 16):
             raise ValueError(f"out must be a contiguous, 16-byte aligned {(*lead, h)} tensor of x.dtype")
         res.append(o)
+    if wide:
+        return _spmm_rows(x2d, mats, w, BLOCK_WIDTH, VEC_WIDTH, res)
     mds = [_aligned(md) for md, _ in mats]
     n = len(mats)
     per = _lib.NM_MC_MAX_BATCH
@@ -471,6 +523,36 @@ def nmsparse_spmm_group_hip(x, mats, BLOCK_WIDTH, VEC_WIDTH, *, outs=None, confi
                                       VEC_WIDTH, int(config_id), int(splits), stream)
             _lib.check(rc, "nm_spmm_mc_group")
     return res
+
+
+def _spmm_rows(x2d, mats, w, BLOCK_WIDTH, VEC_WIDTH, outs, *, up2d=None, splits=0):
+    """nm_spmm_rows on checked operands: outs[i] [rows, h_i] = mats[i] applied
+    to every row of x2d [rows, K] (of round(silu(x2d) * up2d) with up2d), one
+    gather launch and one matrix-core launch for any number of rows. The
+    gathered activations and split partials live in a tensor of this call, the
+    arrival counters in the stream's workspace."""
+    n = len(mats)
+    rows, K = x2d.shape
+    hs = [int(md.shape[1]) for md, _ in mats]
+    lib = _lib.load()
+    harr = (ctypes.c_int * n)(*hs)
+    need = lib.nm_spmm_rows_scratch_bytes(rows, n, harr, w, BLOCK_WIDTH, VEC_WIDTH, int(splits))
+    if need == 0:
+        raise ValueError("spmm shape outside what libnmsparse_hip supports")
+    mds = [_aligned(md) for md, _ in mats]
+    mds_arr = (ctypes.c_void_p * n)(*[md.data_ptr() for md in mds])
+    mis_arr = (ctypes.c_void_p * n)(*[mi.data_ptr() for _, mi in mats])
+    outs_arr = (ctypes.c_void_p * n)(*[o.data_ptr() for o in outs])
+    ostr = (ctypes.c_longlong * n)(*hs)
+    with torch.cuda.device(x2d.device):
+        stream = torch.cuda.current_stream(x2d.device).cuda_stream
+        ws = workspace_for(x2d.device, _lib.NM_TICKET_BYTES, stream)
+        scratch = torch.empty(need, dtype=torch.uint8, device=x2d.device)
+        rc = lib.nm_spmm_rows(_DTYPE_CODE[x2d.dtype], x2d.data_ptr(), None if up2d is None else up2d.data_ptr(), K,
+                              rows, n, mds_arr, mis_arr, outs_arr, ostr, harr, scratch.data_ptr(), need, ws.data_ptr(),
+                              ws.numel(), w, BLOCK_WIDTH, VEC_WIDTH, int(splits), stream)
+    _lib.check(rc, "nm_spmm_rows")
+    return outs
 
 
 def _check_vector(t, n, like, what):
@@ -922,4 +1004,4 @@ __all__ = ["nmsparse_spmv_forward_hip", "nmsparse_spmv_forward_triton_ptx", "nms
            "nmsparse_gate_up_silu", "nmsparse_gemv_launch", "nmsparse_qkv_decode", "nmsparse_spmm_forward_hip",
            "nmsparse_gemv_partials", "carry_splits", "GemvProblem", "launch_plan", "validate_args", "workspace_for",
            "nmsparse_gemv_accumulate", "nmsparse_gate_up_accumulate", "nmsparse_gemv_silu", "gate_up_ssq_slots",
-           "library_route", "attention_supported", "nmsparse_attention_decode"]
+           "library_route", "rows_route", "attention_supported", "nmsparse_attention_decode"]

@@ -70,7 +70,7 @@ def _spmm_dispatches(rows):
     out = []
     for r in rows:
         n = r["Kernel_Name"]
-        for k in ("nm_spmm_mc_kernel", "nm_gather_mc_kernel", "nm_spmm_kernel"):
+        for k in ("nm_spmm_mc_kernel", "nm_gather_mc_kernel", "nm_gather_mc_lds_kernel", "nm_spmm_kernel"):
             if k + "<" in n:
                 out.append((k + n[n.index("<", n.index(k)):n.index(">", n.index(k)) + 1], float(r["Counter_Value"])))
                 break

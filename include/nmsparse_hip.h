@@ -333,6 +333,25 @@ int nm_spmm_plan(int batch, int h, int w, int nnz, int m, int config_id, int spl
                  int* out_splits, int* out_blocks, int* out_rows_per_block);
 
 /*
+ * Several small-batch SpMMs of the same activations in one launch: product i
+ * (0 <= i < n <= 4) is mat_data[i] / mat_index[i] applied to every row of x,
+ * h[i] outputs, out rows out_row_stride[i] apart; each product's rows are bit
+ * for bit nm_spmm's with the library's plan for its shape. Only products that
+ * run the same kernel share a launch: nm_spmm_group_workspace_bytes returns 0
+ * (and nm_spmm_group NM_ERR_BAD_CONFIG) for others.
+ */
+size_t nm_spmm_group_workspace_bytes(int dtype, int batch, int n, const int* h, int w, int nnz, int m);
+int nm_spmm_group(int dtype, const void* x, long long x_row_stride, int batch, int n, const void* const* mat_data,
+                  const uint8_t* const* mat_index, void* const* out, const long long* out_row_stride, const int* h,
+                  void* workspace, size_t workspace_bytes, int w, int nnz, int m, void* stream);
+
+/*
+ * out = round(silu(gate) * up) over n elements (fp16 / bf16, n a multiple of
+ * 8, 16-byte aligned pointers), in fp32 with expf, a division and one rounding.
+ */
+int nm_silu_mul(int dtype, const void* gate, const void* up, void* out, long long n, void* stream);
+
+/*
  * Matrix-core SpMM: the same product for 1 <= batch <= NM_MC_MAX_BATCH rows
  * in one pass over the packed weights, fp16 and bf16 only
  * (v_mfma_f32_16x16x32_f16 / _bf16: fp32 accumulation, one rounding to the

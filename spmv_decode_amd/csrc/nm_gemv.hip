@@ -523,43 +523,106 @@ int make_spmm_plan(int batch, int h, int w, int nnz, int m, int cfg, int splits,
   return make_plan(1, &h, w, nnz, m, 1, cfg, splits, p, kMaxRowsSpmm, batch);
 }
 
-int launch_spmm(int dtype, const void* x, long long x_row_stride, int batch, const void* mat_data,
-                const uint8_t* mat_index, void* out, long long out_row_stride, void* workspace,
-                size_t workspace_bytes, int h, int w, int nnz, int m, int cfg, int splits, void* stream) {
+// n products of the same activations, each on the plan of its own launch (so
+// its rows keep their bits); one launch when they run the same kernel
+// (configuration and gather width), NM_ERR_BAD_CONFIG otherwise. `need`: only
+// plan, and report the workspace.
+int launch_spmm_group(int dtype, const void* x, long long x_row_stride, int batch, int n, const void* const* mat_data,
+                      const uint8_t* const* mat_index, void* const* out, const long long* out_row_stride, const int* h,
+                      void* workspace, size_t workspace_bytes, int w, int nnz, int m, int cfg, int splits, void* stream,
+                      size_t* need = nullptr) {
   if (dtype < NM_DTYPE_F16 || dtype > NM_DTYPE_F32) return NM_ERR_BAD_CONFIG;
-  Plan p;
-  const int rc = make_spmm_plan(batch, h, w, nnz, m, cfg, splits, &p);
-  if (rc != NM_OK) return rc;
-  if (!x || !mat_data || !mat_index || !out || !workspace) return NM_ERR_NULL_POINTER;
+  if (n < 1 || n > kMaxProblems || !h) return NM_ERR_BAD_SHAPE;
+  Plan p[kMaxProblems];
+  size_t bytes = 0, tickets = 0;
+  long long blocks = 0;
+  for (int i = 0; i < n; ++i) {
+    const int rc = make_spmm_plan(batch, h[i], w, nnz, m, cfg, splits, &p[i]);
+    if (rc != NM_OK) return rc;
+    if (p[i].cfg != p[0].cfg || gather_slot(p[i].rows_per_split) != gather_slot(p[0].rows_per_split))
+      return NM_ERR_BAD_CONFIG;
+    bytes += p[i].workspace - NM_TICKET_BYTES;  // its partials
+    tickets += (size_t)p[i].tiles[0];
+    blocks += p[i].blocks;
+  }
+  if (tickets > (size_t)kMaxTickets || blocks > 0x7fffffffLL) return NM_ERR_BAD_SHAPE;
+  if (need) {
+    *need = NM_TICKET_BYTES + bytes;
+    return NM_OK;
+  }
+  if (!x || !mat_data || !mat_index || !out || !out_row_stride || !workspace) return NM_ERR_NULL_POINTER;
   const long long K = (long long)(w / nnz) * (long long)m;
-  if (batch > 1 && (x_row_stride < K || out_row_stride < h)) return NM_ERR_BAD_SHAPE;
-  if (((uintptr_t)mat_data & 15u) != 0 || ((uintptr_t)out & 15u) != 0) return NM_ERR_MISALIGNED;
+  if (batch > 1 && x_row_stride < K) return NM_ERR_BAD_SHAPE;
+  for (int i = 0; i < n; ++i) {
+    if (!mat_data[i] || !mat_index[i] || !out[i]) return NM_ERR_NULL_POINTER;
+    if (batch > 1 && out_row_stride[i] < h[i]) return NM_ERR_BAD_SHAPE;
+    if (((uintptr_t)mat_data[i] & 15u) != 0 || ((uintptr_t)out[i] & 15u) != 0) return NM_ERR_MISALIGNED;
+  }
   if (((uintptr_t)workspace & 255u) != 0) return NM_ERR_MISALIGNED;
-  if (workspace_bytes < p.workspace) return NM_ERR_WORKSPACE;
-  SpmmArgs a;
-  memset(&a, 0, sizeof(a));
-  a.x = x;
-  a.x_row_stride = x_row_stride;
-  a.mat_data = mat_data;
-  a.mat_index = mat_index;
-  a.out = out;
-  a.out_row_stride = out_row_stride;
-  a.tickets = reinterpret_cast<uint32_t*>(workspace) + p.ticket_off[0];
-  a.partial = reinterpret_cast<float*>(static_cast<char*>(workspace) + p.partial_off[0]);
-  a.batch = batch;
-  a.h = h;
-  a.tiles = p.tiles[0];
-  a.w = w;
-  a.nnz = nnz;
-  a.m = m;
-  a.K = (int)K;
-  a.splits = p.splits;
-  a.rows_per_split = p.rows_per_split;
-  const int gslot = gather_slot(p.rows_per_split);  // <= 2: rows_per_split <= kMaxRowsSpmm
-  const SpmmFn fn = spmm_table(dtype)[p.cfg].fn[spmm_nb_slot(batch)][gslot];
-  hipLaunchKernelGGL(fn, dim3(p.blocks), dim3(kBlock), 0, static_cast<hipStream_t>(stream), a);
+  if (workspace_bytes < NM_TICKET_BYTES + bytes) return NM_ERR_WORKSPACE;
+  SpmmGroupArgs g;
+  memset(&g, 0, sizeof(g));
+  g.n = n;
+  size_t part = NM_TICKET_BYTES, tick = 0;
+  int first = 0;
+  for (int i = 0; i < n; ++i) {
+    SpmmArgs& a = g.p[i];
+    a.x = x;
+    a.x_row_stride = x_row_stride;
+    a.mat_data = mat_data[i];
+    a.mat_index = mat_index[i];
+    a.out = out[i];
+    a.out_row_stride = out_row_stride[i];
+    a.tickets = reinterpret_cast<uint32_t*>(workspace) + tick;
+    a.partial = reinterpret_cast<float*>(static_cast<char*>(workspace) + part);
+    a.batch = batch;
+    a.h = h[i];
+    a.tiles = p[i].tiles[0];
+    a.w = w;
+    a.nnz = nnz;
+    a.m = m;
+    a.K = (int)K;
+    a.splits = p[i].splits;
+    a.rows_per_split = p[i].rows_per_split;
+    g.first[i] = first;
+    first += p[i].blocks;
+    tick += (size_t)p[i].tiles[0];
+    part += p[i].workspace - NM_TICKET_BYTES;
+  }
+  const int gslot = gather_slot(p[0].rows_per_split);  // <= 2: rows_per_split <= kMaxRowsSpmm
+  const SpmmFn fn = spmm_table(dtype)[p[0].cfg].fn[spmm_nb_slot(batch)][gslot];
+  hipLaunchKernelGGL(fn, dim3((unsigned)blocks), dim3(kBlock), 0, static_cast<hipStream_t>(stream), g);
   hipError_t e = hipGetLastError();
   return e == hipSuccess ? NM_OK : (int)e;
+}
+
+// round_T(silu(gate) * up) of n elements, n a multiple of 8 (16-byte words),
+// in fp32 with expf, a division and one rounding: PyTorch's arithmetic in one
+// pass. Bound by its launch at the sizes of a small batch (4 x 14336: 2.6 us in
+// a graph, where the casts, SiLU, product and cast back took 12).
+template <int DT>
+__global__ __launch_bounds__(kBlock) void nm_silu_mul_kernel(const u32x4* __restrict__ gate,
+                                                            const u32x4* __restrict__ up, u32x4* __restrict__ out,
+                                                            long long words) {
+  using E = Elem<DT>;
+  typedef typename E::scalar T;
+  typedef T t8 __attribute__((ext_vector_type(8)));
+  const long long i = (long long)blockIdx.x * kBlock + threadIdx.x;
+  if (i >= words) return;
+  const u32x4 gw[1] = {gate[i]}, uw[1] = {up[i]};
+  float g[8], u[8];
+  E::unpack(gw, g);
+  E::unpack(uw, u);
+  t8 r;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    float y = g[e] / (1.0f + expf(-g[e])) * u[e];
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm volatile("" : "+v"(y));  // the fp32 product is rounded before the element type
+#endif
+    r[e] = E::from_f32(y);
+  }
+  out[i] = __builtin_bit_cast(u32x4, r);
 }
 
 }  // namespace
@@ -768,8 +831,35 @@ size_t nm_spmm_workspace_bytes(int batch, int h, int w, int nnz, int m, int conf
 int nm_spmm(int dtype, const void* x, long long x_row_stride, int batch, const void* mat_data,
             const uint8_t* mat_index, void* out, long long out_row_stride, void* workspace, size_t workspace_bytes,
             int h, int w, int nnz, int m, int config_id, int splits, void* stream) {
-  return launch_spmm(dtype, x, x_row_stride, batch, mat_data, mat_index, out, out_row_stride, workspace,
-                     workspace_bytes, h, w, nnz, m, config_id, splits, stream);
+  return launch_spmm_group(dtype, x, x_row_stride, batch, 1, &mat_data, &mat_index, &out, &out_row_stride, &h,
+                           workspace, workspace_bytes, w, nnz, m, config_id, splits, stream);
+}
+
+size_t nm_spmm_group_workspace_bytes(int dtype, int batch, int n, const int* h, int w, int nnz, int m) {
+  size_t need = 0;
+  return launch_spmm_group(dtype, nullptr, 0, batch, n, nullptr, nullptr, nullptr, nullptr, h, nullptr, 0, w, nnz, m,
+                           -1, 0, nullptr, &need) == NM_OK
+             ? need
+             : 0;
+}
+
+int nm_spmm_group(int dtype, const void* x, long long x_row_stride, int batch, int n, const void* const* mat_data,
+                  const uint8_t* const* mat_index, void* const* out, const long long* out_row_stride, const int* h,
+                  void* workspace, size_t workspace_bytes, int w, int nnz, int m, void* stream) {
+  return launch_spmm_group(dtype, x, x_row_stride, batch, n, mat_data, mat_index, out, out_row_stride, h, workspace,
+                           workspace_bytes, w, nnz, m, -1, 0, stream);
+}
+
+int nm_silu_mul(int dtype, const void* gate, const void* up, void* out, long long n, void* stream) {
+  if (dtype != NM_DTYPE_F16 && dtype != NM_DTYPE_BF16) return NM_ERR_BAD_CONFIG;
+  if (!gate || !up || !out) return NM_ERR_NULL_POINTER;
+  if (n <= 0 || n % 8 != 0 || n / 8 > (long long)kBlock * 0x7fffffffLL) return NM_ERR_BAD_SHAPE;
+  if ((((uintptr_t)gate | (uintptr_t)up | (uintptr_t)out) & 15u) != 0) return NM_ERR_MISALIGNED;
+  hipLaunchKernelGGL((dtype == NM_DTYPE_F16 ? nm_silu_mul_kernel<NM_DTYPE_F16> : nm_silu_mul_kernel<NM_DTYPE_BF16>),
+                     dim3((unsigned)((n / 8 + kBlock - 1) / kBlock)), dim3(kBlock), 0, static_cast<hipStream_t>(stream),
+                     static_cast<const u32x4*>(gate), static_cast<const u32x4*>(up), static_cast<u32x4*>(out), n / 8);
+  const hipError_t e = hipGetLastError();
+  return e == hipSuccess ? NM_OK : (int)e;
 }
 
 int nm_spmm_plan(int batch, int h, int w, int nnz, int m, int config_id, int splits, int* out_config_id,

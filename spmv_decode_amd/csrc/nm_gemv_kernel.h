@@ -953,8 +953,17 @@ struct SpmmArgs {
   int rows_per_split;
 };
 
+// Several products of the same activations in one grid (sibling Linears):
+// product i owns workgroups first[i] .. first[i + 1] - 1, with its own weights,
+// outputs, plan, partials and arrival counters.
+struct SpmmGroupArgs {
+  SpmmArgs p[kMaxProblems];
+  int first[kMaxProblems];
+  int n;
+};
+
 template <int DT, int TH, int U, int G, bool NT, int NB>
-__global__ __launch_bounds__(kBlock) void nm_spmm_kernel(SpmmArgs a) {
+__global__ __launch_bounds__(kBlock) void nm_spmm_kernel(SpmmGroupArgs g) {
   using E = Elem<DT>;
   typedef typename E::scalar T;
   constexpr int W = E::kWords;
@@ -970,12 +979,18 @@ __global__ __launch_bounds__(kBlock) void nm_spmm_kernel(SpmmArgs a) {
   __shared__ __attribute__((aligned(16))) float red[NB][TK * HT];
   __shared__ int is_last;
 
+  int pi = 0;
+#pragma unroll
+  for (int q = 1; q < kMaxProblems; ++q)
+    if (q < g.n && (int)blockIdx.x >= g.first[q]) pi = q;
+  const SpmmArgs& a = g.p[pi];
+  const int local = (int)blockIdx.x - g.first[pi];
   const int h = a.h;
   const int tid = threadIdx.x;
   const int th = tid % TH;
   const int tk = tid / TH;
-  const int tile = (int)blockIdx.x % a.tiles;
-  const int split = (int)blockIdx.x / a.tiles;
+  const int tile = local % a.tiles;
+  const int split = local / a.tiles;
   const int c0 = split * a.rows_per_split;
   const int cw = min(a.rows_per_split, a.w - c0);
   const int nch = (cw + CH - 1) / CH;
@@ -1250,7 +1265,7 @@ struct KernelRow {
 #define NM_SPMM_CONFIGS(X) X(16, 4, true) X(16, 8, true) X(32, 4, true) X(32, 8, true)
 constexpr int kNumSpmmConfigs = 4;
 
-typedef void (*SpmmFn)(SpmmArgs);
+typedef void (*SpmmFn)(SpmmGroupArgs);
 
 // fn[batch rows per launch: 2, 4, 8][gather slot: 256, 512, 1024 columns per split].
 struct SpmmRow {

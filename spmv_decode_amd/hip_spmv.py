@@ -369,8 +369,8 @@ def nmsparse_spmm_silu_mul_hip(gate, up, mat_data, mat_index, w, h, BLOCK_WIDTH,
     gate/up pair's epilogue), past them likewise inside the gather of
     nm_spmm_rows or of the library GEMM (with expf and a division: the bits of
     the product formed in fp32 with one rounding), otherwise the product formed
-    in fp32 with one rounding and then nmsparse_spmm_forward_hip. Returns
-    [..., rows, h]."""
+    in fp32 with one rounding (nm_silu_mul, the same bits, where it can) and
+    then nmsparse_spmm_forward_hip. Returns [..., rows, h]."""
     if gate.shape != up.shape or gate.dtype != up.dtype or gate.device != up.device:
         raise ValueError("gate and up must have one shape, dtype and device")
     K = gate.shape[-1]
@@ -381,7 +381,16 @@ def nmsparse_spmm_silu_mul_hip(gate, up, mat_data, mat_index, w, h, BLOCK_WIDTH,
     wide = (gate.dtype in (torch.float16, torch.bfloat16) and gate.is_cuda and not explicit
             and rows > _lib.NM_MC_MAX_BATCH)
     if not (fused or wide):
-        act = (torch.nn.functional.silu(gate.float()) * up.float()).to(gate.dtype)
+        if (gate.is_cuda and gate.dtype in (torch.float16, torch.bfloat16) and gate.numel() and gate.numel() % 8 == 0
+                and gate.is_contiguous() and up.is_contiguous()
+                and gate.data_ptr() % 16 == 0 and up.data_ptr() % 16 == 0):
+            act = torch.empty_like(gate)
+            with torch.cuda.device(gate.device):
+                rc = _lib.load().nm_silu_mul(_DTYPE_CODE[gate.dtype], gate.data_ptr(), up.data_ptr(), act.data_ptr(),
+                                             gate.numel(), torch.cuda.current_stream(gate.device).cuda_stream)
+            _lib.check(rc, "nm_silu_mul")
+        else:
+            act = (torch.nn.functional.silu(gate.float()) * up.float()).to(gate.dtype)
         return nmsparse_spmm_forward_hip(act, mat_data, mat_index, w, h, BLOCK_WIDTH, VEC_WIDTH, out=out,
                                          config_id=config_id, splits=splits)
     if not (mat_data.is_cuda and mat_index.is_cuda) or mat_data.device != gate.device:
@@ -446,8 +455,10 @@ def nmsparse_spmm_group_hip(x, mats, BLOCK_WIDTH, VEC_WIDTH, *, outs=None, confi
     product's activations and one matrix-core launch over all their tiles
     (nm_spmm_mc_group; each product's rows equal nm_spmm_mc's with the same
     config_id and splits), and past them likewise on nm_spmm_rows where that
-    is faster (rows_route). Otherwise (fewer or more rows, fp32, more
-    products, or with the plan left to the library past 64 rows of products
+    is faster (rows_route); up to NM_MAX_BATCH rows of any dtype one
+    small-batch launch for products that run the same kernel (nm_spmm_group:
+    the bits of one launch each). Otherwise (more rows, fp32, more products, or
+    with the plan left to the library past 64 rows of products
     of at most 1024 outputs: library_route) each product runs through
     nmsparse_spmm_forward_hip on its own.
     """
@@ -470,7 +481,12 @@ def nmsparse_spmm_group_hip(x, mats, BLOCK_WIDTH, VEC_WIDTH, *, outs=None, confi
                and one_w)
     wide = (x.dtype in (torch.float16, torch.bfloat16) and not explicit and rows > _lib.NM_MC_MAX_BATCH
             and 1 < len(mats) <= _lib.NM_MC_MAX_GROUP and one_w and rows_route(rows, w, hs))
-    if not (grouped or wide):
+    small = 0  # the workspace of one small-batch launch for all products, 0: one launch each
+    if (0 < rows <= _lib.NM_MAX_BATCH and not explicit and 1 < len(mats) <= 4 and one_w and x.dtype in _DTYPE_CODE
+            and w % BLOCK_WIDTH == 0):
+        small = _lib.load().nm_spmm_group_workspace_bytes(_DTYPE_CODE[x.dtype], rows, len(hs),
+                                                          (ctypes.c_int * len(hs))(*hs), w, BLOCK_WIDTH, VEC_WIDTH)
+    if not (grouped or wide or small):
         return [nmsparse_spmm_forward_hip(x, md, mi, w, h, BLOCK_WIDTH, VEC_WIDTH, out=o, config_id=config_id,
                                           splits=splits)
                 for (md, mi), h, o in zip(mats, hs, outs)]
@@ -504,8 +520,8 @@ def nmsparse_spmm_group_hip(x, mats, BLOCK_WIDTH, VEC_WIDTH, *, outs=None, confi
     per = _lib.NM_MC_MAX_BATCH
     lib = _lib.load()
     harr = (ctypes.c_int * n)(*hs)
-    need = lib.nm_spmm_mc_group_workspace_bytes(min(rows, per), n, harr, w, BLOCK_WIDTH, VEC_WIDTH, int(config_id),
-                                                int(splits))
+    need = small or lib.nm_spmm_mc_group_workspace_bytes(min(rows, per), n, harr, w, BLOCK_WIDTH, VEC_WIDTH,
+                                                         int(config_id), int(splits))
     if need == 0:
         raise ValueError("spmm group shape outside what libnmsparse_hip supports")
     esize = x.element_size()
@@ -515,6 +531,12 @@ def nmsparse_spmm_group_hip(x, mats, BLOCK_WIDTH, VEC_WIDTH, *, outs=None, confi
     with torch.cuda.device(x.device):
         stream = torch.cuda.current_stream(x.device).cuda_stream
         ws = workspace_for(x.device, need, stream)
+        if small:
+            outs_arr = (ctypes.c_void_p * n)(*[o.data_ptr() for o in res])
+            rc = lib.nm_spmm_group(_DTYPE_CODE[x.dtype], x2d.data_ptr(), K, rows, n, mds_arr, mis_arr, outs_arr, ostr,
+                                   harr, ws.data_ptr(), ws.numel(), w, BLOCK_WIDTH, VEC_WIDTH, stream)
+            _lib.check(rc, "nm_spmm_group")
+            return res
         for r0 in range(0, rows, per):
             b = min(per, rows - r0)
             outs_arr = (ctypes.c_void_p * n)(*[o.data_ptr() + r0 * h * esize for o, h in zip(res, hs)])

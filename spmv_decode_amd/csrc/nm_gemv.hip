@@ -75,6 +75,13 @@ int auto_config(long long h_total, int nmat, bool carried) {
   return h_total > 16384 ? 6 : (h_total > 4096 ? 3 : 1);
 }
 
+// fp32 on 256- and 512-row tiles: the same configuration with cached loads. An
+// fp32 lane reads its 32 bytes of a row in two loads, each half of every cache
+// line; read past the cache, a line came from memory for each half (graph
+// replay, non-temporal / cached: 4096 -> 14336 27.3 / 23.1 us, 5120 -> 17408 38.4 /
+// 33.4; 128-row tiles measured the same either way).
+int cached_twin(int cfg) { return cfg == 3 ? 11 : (cfg == 6 ? 12 : cfg); }
+
 // Workgroups that run at once, one per CU: an MI355X has 256 CUs. The split
 // count below is chosen for this many; it changes speed only, never results.
 constexpr int kPlanCUs = 256;
@@ -458,7 +465,8 @@ int launch(const nm_gemv_launch_desc& d, void* workspace, size_t workspace_bytes
   const int variant = silu_in    ? kVarSilu
                       : carry_in ? (d.carry_splits == 1 ? kVarCarry1 : (d.carry_splits <= 8 ? kVarCarry8 : kVarCarry16))
                                  : (d.norm_weight ? kVarNorm : kVarPlain);
-  const KernelFn fn = kernel_table(d.dtype, pair)[p.cfg].fn[gather_slot(p.rows_per_split)][variant];
+  const int kcfg = d.dtype == NM_DTYPE_F32 && !pair && d.config_id < 0 ? cached_twin(p.cfg) : p.cfg;
+  const KernelFn fn = kernel_table(d.dtype, pair)[kcfg].fn[gather_slot(p.rows_per_split)][variant];
   if (!fn) return NM_ERR_BAD_EPILOGUE;
   hipLaunchKernelGGL(fn, dim3(p.blocks), dim3(kBlock), 0, static_cast<hipStream_t>(stream), a);
   hipError_t e = hipGetLastError();

@@ -464,6 +464,15 @@ int nm_gemv_plan(int h, int w, int nnz, int m, int config_id, int splits,
                  int* out_rows_per_block);
 
 /*
+ * y[r] = sum_k weight[r * row_stride + k] * x[k] for r < n: one row of
+ * activations through a dense weight (a decode step's output head). fp16 and
+ * bf16, fp32 sums, one rounding; K a multiple of 8 up to 8192, row_stride a
+ * multiple of 8, x and weight 16-byte aligned.
+ */
+int nm_dense_gemv(int dtype, const void* x, const void* weight, long long row_stride, void* y, int n, int K,
+                  void* stream);
+
+/*
  * The attention of one decode token over the transposed static caches:
  * out[h, :] = softmax over positions p <= *pos of q[h, :] . K[h / g, :, p] /
  * sqrt(head_dim), times V[h / g, :, p], with g = n_heads / kv_heads query heads

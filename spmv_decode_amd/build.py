@@ -22,7 +22,8 @@ ROOT = PKG.parent
 CSRC = PKG / "csrc"
 # (source, extra defines): the host side, then the kernels of each element type.
 UNITS = [(CSRC / "nm_gemv.hip", []), *[(CSRC / "nm_gemv_inst.hip", [f"-DNM_INST_DTYPE={dt}"]) for dt in (0, 1, 2)],
-         (CSRC / "nm_spmm_mc.hip", []), (CSRC / "nm_spmm_rows.hip", []), (CSRC / "nm_attention.hip", [])]
+         (CSRC / "nm_spmm_mc.hip", []), (CSRC / "nm_spmm_rows.hip", []), (CSRC / "nm_attention.hip", []),
+         (CSRC / "nm_dense_gemv.hip", [])]
 LIB_PATH = PKG / "libnmsparse_hip.so"
 # Measurement-only streaming-read kernel used by the microbenchmark.
 PROBE_SOURCES = [PKG / "csrc" / "roofline_probe.hip"]

@@ -232,6 +232,15 @@ def project(lin: nn.Module, x: torch.Tensor) -> torch.Tensor:
     return lin(x)
 
 
+def project_head(lin: nn.Module, x: torch.Tensor, kernel: bool) -> torch.Tensor:
+    """The output head on one row x [..., dim] -> [1, vocab]: in the library's
+    dense GEMV when `kernel` (Decoder.setup_cache found it to take the weight),
+    else project."""
+    if kernel and type(lin) is nn.Linear and lin.bias is None and lin.weight.dtype == x.dtype:
+        return torch.ops.nmsparse.dense_gemv(x.reshape(1, -1), lin.weight)
+    return project(lin, x).view(1, -1)
+
+
 def project_rows(lin: nn.Module, x2d: torch.Tensor) -> torch.Tensor:
     """lin(x) for every row of x2d [rows, K] -> [rows, h]: an NmSparseLinear
     through the SpMM on its packed weights (the small-batch kernel up to 8
@@ -710,6 +719,7 @@ class Decoder(nn.Module):
         self.lm_head = nn.Linear(cfg.dim, cfg.vocab, bias=False)
         self.max_seq = 0
         self.attention_kernel = False  # setup_cache: the layers' decode_kernel
+        self.head_kernel = False  # setup_cache: lm_head in the library's dense GEMV (project_head)
         self.gemv_forms = {}  # (n_out, n_in) -> dense_gemv form, filled by tune_dense_gemv
         self.dense_fusion = "none"  # set_dense_fusion's mode
 
@@ -834,12 +844,15 @@ class Decoder(nn.Module):
         self.rope = torch.polar(torch.ones_like(ang), ang).to(torch.complex64).to(device)
         self.rope_real = torch.view_as_real(self.rope)  # the same table as fp32 (cos, sin) pairs
         self.positions = torch.arange(max_seq, device=device)
-        kernel = False
+        kernel = head = False
         if self.q_pad.is_cuda:
-            from ..hip_spmv import attention_supported
+            from ..hip_spmv import attention_supported, dense_gemv_supported
 
+            head = (type(self.lm_head) is nn.Linear and self.lm_head.bias is None
+                    and dense_gemv_supported(torch.empty(1, c.dim, device=self.q_pad.device, dtype=dtype),
+                                             self.lm_head.weight))
             kernel = attention_supported(self.q_pad, self.k_cache_t[0], self.v_cache_t[0], hd)
-        self.attention_kernel = kernel
+        self.attention_kernel, self.head_kernel = kernel, head
         for blk in self.layers:
             (blk.self_attn if isinstance(blk, Block) else blk.attention).decode_kernel = kernel
         self._carry = None
@@ -949,7 +962,7 @@ class Decoder(nn.Module):
             h = ln2(x)
             g_out, u_out = project_rows_group((gate, up), h)
             x = x + project_rows_silu_mul(down, g_out, u_out)
-        return project(self.lm_head, self.norm(x[-1:].view(1, 1, -1))).view(1, -1)
+        return project_head(self.lm_head, self.norm(x[-1:].view(1, 1, -1)), self.head_kernel)
 
     def forward_step(self, token: torch.Tensor, pos: torch.Tensor) -> torch.Tensor:
         """One decode step: token [1, 1] int64 and pos [1] int64 on the device
@@ -971,15 +984,15 @@ class Decoder(nn.Module):
                 run = fused_layers_accumulated if len(bufs) == 4 else fused_layers_carried
                 h2d = run(self.layers, x2d, *bufs, self.k_cache_t, self.v_cache_t, pos, self.q_pad, self.zero,
                           self.rope_real)
-                return project(self.lm_head, self.norm(h2d.view(1, 1, -1))).view(1, -1)
+                return project_head(self.lm_head, self.norm(h2d.view(1, 1, -1)), self.head_kernel)
             for i, blk in enumerate(self.layers):
                 fused_block_step(blk, x2d, self.k_cache_t[i], self.v_cache_t[i], pos, self.q_pad, self.zero,
                                  self.rope_real)
-            return project(self.lm_head, self.norm(x)).view(1, -1)
+            return project_head(self.lm_head, self.norm(x), self.head_kernel)
         freqs = (self.rope_real if torch.compiler.is_compiling() else self.rope).index_select(0, pos)
         for i, layer in enumerate(self.layers):
             x = layer(x, freqs, self.k_cache_t[i], self.v_cache_t[i], pos, self.q_pad, self.zero)
-        return project(self.lm_head, self.norm(x)).view(1, -1)
+        return project_head(self.lm_head, self.norm(x), self.head_kernel)
 
 
 def _graph_median_us(launches, reps: int, warmup: int) -> float:

@@ -1022,8 +1022,38 @@ def nmsparse_attention_decode(q, k_cache_t, v_cache_t, pos, head_dim, *, out=Non
     return out
 
 
+def dense_gemv_supported(x: torch.Tensor, weight: torch.Tensor) -> bool:
+    """Whether nmsparse_dense_gemv takes x [..., K] (one row) and weight [n, K]:
+    fp16 / bf16 on one GPU, unit strides along K, K a multiple of 8 up to 8192,
+    rows at 16-byte boundaries. No GPU work."""
+    if weight.dim() != 2 or x.dim() == 0:
+        return False
+    n, K = weight.shape
+    return (x.is_cuda and weight.device == x.device and x.dtype == weight.dtype
+            and x.dtype in (torch.float16, torch.bfloat16) and x.shape[-1] == K and x.numel() == K and n > 0
+            and 0 < K <= 8192 and K % 8 == 0 and x.is_contiguous() and weight.stride(1) == 1
+            and weight.stride(0) >= K and weight.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0
+            and weight.data_ptr() % 16 == 0)
+
+
+def nmsparse_dense_gemv(x, weight):
+    """weight [n, K] applied to the one row x [..., K] -> [1, n], fp32 sums, one
+    rounding (dense_gemv_supported says which operands are taken)."""
+    if not dense_gemv_supported(x, weight):
+        raise ValueError(f"dense gemv of x {tuple(x.shape)} {x.dtype} and weight {tuple(weight.shape)} {weight.dtype} "
+                         "is not supported")
+    n, K = weight.shape
+    y = torch.empty(1, n, dtype=x.dtype, device=x.device)
+    with torch.cuda.device(x.device):
+        rc = _lib.load().nm_dense_gemv(_DTYPE_CODE[x.dtype], x.data_ptr(), weight.data_ptr(), weight.stride(0),
+                                       y.data_ptr(), n, K, torch.cuda.current_stream(x.device).cuda_stream)
+    _lib.check(rc, "nm_dense_gemv")
+    return y
+
+
 __all__ = ["nmsparse_spmv_forward_hip", "nmsparse_spmv_forward_triton_ptx", "nmsparse_gemv_grouped",
            "nmsparse_gate_up_silu", "nmsparse_gemv_launch", "nmsparse_qkv_decode", "nmsparse_spmm_forward_hip",
            "nmsparse_gemv_partials", "carry_splits", "GemvProblem", "launch_plan", "validate_args", "workspace_for",
            "nmsparse_gemv_accumulate", "nmsparse_gate_up_accumulate", "nmsparse_gemv_silu", "gate_up_ssq_slots",
-           "library_route", "rows_route", "attention_supported", "nmsparse_attention_decode"]
+           "library_route", "rows_route", "attention_supported", "nmsparse_attention_decode",
+           "dense_gemv_supported", "nmsparse_dense_gemv"]

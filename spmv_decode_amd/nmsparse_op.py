@@ -28,7 +28,8 @@ run to run) adds `nmsparse::gemv_accumulate_`, `nmsparse::gate_up_accumulate_`
 `nmsparse::gemv_silu_add_` (down_proj taking the pair's SiLU product as it
 gathers its input), and the `zero` argument of the q/k/v ops (an accumulator
 cleared by the launch). `nmsparse::attention_decode` is the attention between
-the q/k/v launch and o_proj: one launch over the caches' positions up to pos.
+the q/k/v launch and o_proj: one launch over the caches' positions up to pos; `nmsparse::dense_gemv` the
+decode step's dense output head.
 
 `nmsparse::gemv_grouped` (one launch for 1-4 gemv calls on the same input),
 `nmsparse::gemv_silu_mul` (silu(gemv gate) * gemv up in one launch), both
@@ -58,8 +59,8 @@ import torch
 
 from typing import Optional
 
-from .hip_spmv import (GemvProblem, nmsparse_attention_decode, nmsparse_gate_up_accumulate, nmsparse_gate_up_silu,
-                       nmsparse_gemv_accumulate, nmsparse_gemv_grouped, nmsparse_gemv_launch, nmsparse_gemv_partials,
+from .hip_spmv import (GemvProblem, nmsparse_attention_decode, nmsparse_dense_gemv, nmsparse_gate_up_accumulate,
+                       nmsparse_gate_up_silu, nmsparse_gemv_accumulate, nmsparse_gemv_grouped, nmsparse_gemv_launch, nmsparse_gemv_partials,
                        nmsparse_gemv_silu, nmsparse_qkv_decode, nmsparse_spmm_forward_hip, nmsparse_spmv_forward_hip)
 
 _kernel = os.environ.get("NM_KERNEL", "")
@@ -378,6 +379,18 @@ def _(q, k_cache_t, v_cache_t, pos, head_dim):
     return q.new_empty((1, q.shape[0] * int(head_dim)))
 
 
-__all__ = ["attention_decode", "gemv", "spmm", "gemv_grouped", "gemv_silu_mul", "gemv_residual", "qkv_decode", "gemv_add_", "gate_up_silu", "gemv_partials_",
+@torch.library.custom_op("nmsparse::dense_gemv", mutates_args=())
+def dense_gemv(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
+    """A dense weight [n, K] applied to one row x [..., K] -> [1, n]
+    (hip_spmv.nmsparse_dense_gemv)."""
+    return nmsparse_dense_gemv(x, weight)
+
+
+@dense_gemv.register_fake
+def _(x, weight):
+    return x.new_empty((1, weight.shape[0]))
+
+
+__all__ = ["attention_decode", "dense_gemv", "gemv", "spmm", "gemv_grouped", "gemv_silu_mul", "gemv_residual", "qkv_decode", "gemv_add_", "gate_up_silu", "gemv_partials_",
            "qkv_decode_carried", "gate_up_silu_carried", "gemv_accumulate_", "gate_up_accumulate_",
            "gemv_silu_accumulate_", "gemv_silu_add_"]

@@ -464,6 +464,33 @@ int nm_gemv_plan(int h, int w, int nnz, int m, int config_id, int splits,
                  int* out_rows_per_block);
 
 /*
+ * A prompt's keys, values and queries, one launch: for positions 0 .. P-1 the
+ * optional per-head RMSNorm (q_norm, k_norm [head_dim], fp32) and the rotary
+ * embedding (rope_table fp32 [>= P, head_dim / 2, 2]: cos, sin of (even, odd)
+ * pairs) of q [P, n_heads * head_dim] into q_out [P, n_heads, head_dim] and of
+ * k [P, kv_heads * head_dim] into k_cache_t [kv_heads, >= head_dim, cache_len];
+ * v into v_cache_t [kv_heads, head_dim, cache_len]; rows *_row_stride elements
+ * apart, one rounding each. Positions from P on are untouched. fp16 and bf16;
+ * head_dim 64 or 128; cache_len and every stride multiples of 8, pointers
+ * 16-byte aligned.
+ */
+int nm_prefill_rope(int dtype, const void* q, long long q_row_stride, const void* k, long long k_row_stride,
+                    const void* v, long long v_row_stride, const void* q_norm, const void* k_norm, float eps,
+                    const float* rope_table, int P, int n_heads, int kv_heads, int head_dim, void* q_out,
+                    void* k_cache_t, long long k_head_stride, void* v_cache_t, long long v_head_stride, int cache_len,
+                    void* stream);
+
+/*
+ * Causal attention of a prompt over the caches nm_prefill_rope wrote: position
+ * p < P of q [P, n_heads, head_dim] over positions 0 .. p, into out [P, n_heads,
+ * head_dim]; scores, softmax and sums in fp32, probabilities and outputs
+ * rounded to the element type. Layouts as nm_attention_decode's.
+ */
+int nm_attention_prefill(int dtype, const void* q, const void* k_cache_t, long long k_head_stride,
+                         const void* v_cache_t, long long v_head_stride, void* out, int P, int n_heads, int kv_heads,
+                         int head_dim, int cache_len, void* stream);
+
+/*
  * y[r] = sum_k weight[r * row_stride + k] * x[k] for r < n: one row of
  * activations through a dense weight (a decode step's output head). fp16 and
  * bf16, fp32 sums, one rounding; K a multiple of 8 up to 8192, row_stride a

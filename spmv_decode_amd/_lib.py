@@ -102,6 +102,9 @@ ABI = {
     "nm_spmm_rows_plan": (_i, [_i, _i, _ip, _i, _i, _i, _i, _ip, _ip]),
     "nm_spmm_rows": (_i, [_i, _vp, _vp, _ll, _i, _i, ctypes.POINTER(_vp), ctypes.POINTER(_vp), ctypes.POINTER(_vp),
                           ctypes.POINTER(_ll), _ip, _vp, _sz, _vp, _sz, _i, _i, _i, _i, _vp]),
+    "nm_prefill_rope": (_i, [_i, _vp, _ll, _vp, _ll, _vp, _ll, _vp, _vp, ctypes.c_float, _vp, _i, _i, _i, _i, _vp, _vp,
+                             _ll, _vp, _ll, _i, _vp]),
+    "nm_attention_prefill": (_i, [_i, _vp, _vp, _ll, _vp, _ll, _vp, _i, _i, _i, _i, _i, _vp]),
     "nm_dense_gemv": (_i, [_i, _vp, _vp, _ll, _vp, _i, _i, _vp]),
     "nm_attention_decode_workspace_bytes": (_sz, [_i, _i, _i, _i, _i]),
     "nm_attention_decode": (_i, [_i, _vp, _ll, _vp, _ll, _vp, _ll, _vp, _vp, _vp, _sz, _i, _i, _i, _i, _i, _vp]),

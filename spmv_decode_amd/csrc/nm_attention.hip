@@ -1,5 +1,7 @@
-// nm_attention.hip — the attention of one decode token over the transposed
-// static caches, in one launch (nm_attention_decode, include/nmsparse_hip.h):
+// nm_attention.hip — attention over the transposed static caches
+// (include/nmsparse_hip.h): one decode token in one launch
+// (nm_attention_decode), and a whole prompt (nm_prefill_rope,
+// nm_attention_prefill; at the end of this file). The decode token:
 //
 //   out[h, :] = softmax_p( q[h, :] . K[:, p] / sqrt(hd) ) V[:, p]^T,  p <= pos
 //
@@ -410,6 +412,242 @@ typedef void (*AttnFn)(AttnArgs);
 const AttnFn kAttnKernels[2][2][3] = {NM_ATTN_ROW(NM_DTYPE_F16), NM_ATTN_ROW(NM_DTYPE_BF16)};
 #undef NM_ATTN_ROW
 
+// ---------------------------------------------------------------------------
+// A whole prompt (nm_prefill_rope, nm_attention_prefill): the rotary embedding
+// with the cache writes, and causal attention of every position over the
+// caches.
+// ---------------------------------------------------------------------------
+struct RopeArgs {
+  const void *q, *k, *v;            // [P, heads * hd], rows *_stride elements apart
+  long long q_stride, k_stride, v_stride;
+  const void *q_norm, *k_norm;      // optional [hd] per-head RMSNorm weights
+  const float2* rope;               // [>= P, hd / 2] (cos, sin)
+  void* q_out;                      // [P, n_heads, hd]
+  void* k_cache;                    // [kv_heads, >= hd, S]
+  void* v_cache;                    // [kv_heads, hd, S]
+  long long k_head, v_head;
+  float eps;
+  int P, nh, kvh, S;
+};
+
+// A workgroup takes 64 positions of one head: blockIdx.y < nh a query head
+// (norm, rotation, to q_out), then the key heads (the same, transposed into the
+// cache through LDS) and the value heads (transposed only). Lane (row, part)
+// holds a quarter of a row's head. One pass over q, k and v where the norms, the
+// casts, the complex product and the strided cache copies took twelve launches
+// per layer. Bound by its launch and one memory round trip.
+template <int DT, int HD>
+__global__ __launch_bounds__(kBlock) void nm_prefill_rope_kernel(RopeArgs a) {
+  using E = Elem<DT>;
+  typedef typename E::scalar T;
+  constexpr int Q = HD / 4;        // elements per lane
+  constexpr int TS = 64 + 8;       // LDS row stride of the transposed tile
+  __shared__ __attribute__((aligned(16))) T tile[HD * TS];
+  const int tid = threadIdx.x, row = tid >> 2, part = tid & 3;
+  const int p0 = (int)blockIdx.x * 64, head = (int)blockIdx.y;
+  const int pos = min(p0 + row, a.P - 1);
+  const int kind = head < a.nh ? 0 : (head < a.nh + a.kvh ? 1 : 2);
+  const int hi = kind == 0 ? head : (kind == 1 ? head - a.nh : head - a.nh - a.kvh);
+  const T* src = static_cast<const T*>(kind == 0 ? a.q : (kind == 1 ? a.k : a.v)) +
+                 (long long)pos * (kind == 0 ? a.q_stride : (kind == 1 ? a.k_stride : a.v_stride)) + hi * HD + part * Q;
+  u32x4 raw[Q / 8];
+#pragma unroll
+  for (int i = 0; i < Q / 8; ++i) raw[i] = *reinterpret_cast<const u32x4*>(src + 8 * i);
+  float x[Q];
+#pragma unroll
+  for (int i = 0; i < Q / 8; ++i) {
+    const u32x4 one[1] = {raw[i]};
+    float f[8];
+    E::unpack(one, f);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) x[8 * i + e] = f[e];
+  }
+  const T* norm = static_cast<const T*>(kind == 0 ? a.q_norm : a.k_norm);
+  if (kind < 2) {
+    if (norm) {
+      float s = 0.0f;
+#pragma unroll
+      for (int e = 0; e < Q; ++e) s = __builtin_fmaf(x[e], x[e], s);
+      s += dpp<0xB1>(s);
+      s += dpp<0x4E>(s);  // the row's four lanes
+      const float r = rsqrtf(s / (float)HD + a.eps);
+#pragma unroll
+      for (int e = 0; e < Q; ++e) x[e] *= r * E::to_f32(norm[part * Q + e]);
+    }
+    const float2* cs = a.rope + (size_t)pos * (HD / 2) + part * (Q / 2);
+#pragma unroll
+    for (int e = 0; e < Q / 2; ++e) {
+      const float2 c = cs[e];
+      const float x0 = x[2 * e], x1 = x[2 * e + 1];
+      x[2 * e] = x0 * c.x - x1 * c.y;
+      x[2 * e + 1] = x0 * c.y + x1 * c.x;
+    }
+  }
+  typedef T t8 __attribute__((ext_vector_type(8)));
+  if (kind == 0) {
+    if (p0 + row >= a.P) return;
+    T* out = static_cast<T*>(a.q_out) + ((long long)pos * a.nh + hi) * HD + part * Q;
+#pragma unroll
+    for (int i = 0; i < Q / 8; ++i) {
+      t8 v;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] = E::from_f32(x[8 * i + e]);
+      *reinterpret_cast<t8*>(out + 8 * i) = v;
+    }
+    return;
+  }
+#pragma unroll
+  for (int e = 0; e < Q; ++e) tile[(part * Q + e) * TS + row] = E::from_f32(x[e]);
+  __syncthreads();
+  T* cache = static_cast<T*>(kind == 1 ? a.k_cache : a.v_cache) + (long long)hi * (kind == 1 ? a.k_head : a.v_head);
+#pragma unroll
+  for (int i = 0; i < HD / 32; ++i) {  // 8 positions of a dimension per lane
+    const int d = i * 32 + (tid >> 3), p = 8 * (tid & 7);
+    T* dst = cache + (long long)d * a.S + p0 + p;
+    if (p0 + p + 8 <= a.P) {  // S and so every row of the cache is a multiple of 8 (host)
+      *reinterpret_cast<u32x4*>(dst) = *reinterpret_cast<const u32x4*>(&tile[d * TS + p]);
+    } else {
+      for (int e = 0; e < 8; ++e)
+        if (p0 + p + e < a.P) dst[e] = tile[d * TS + p + e];
+    }
+  }
+}
+
+struct PrefillArgs {
+  const void* q;   // [P, n_heads, hd]
+  const void* k;   // [kv_heads, >= hd, S]
+  const void* v;   // [kv_heads, hd, S]
+  void* out;       // [P, n_heads, hd]
+  long long k_head, v_head;
+  int P, nh, kvh, g, S, tiles;
+  float scale;     // log2(e) / sqrt(hd)
+};
+
+// A workgroup takes 64 positions of one query head, 16 per wave, and goes over
+// the cached positions up to its last in blocks of 64: scores as in
+// nm_attention_kernel (K through LDS, read transposed), a running maximum and
+// sum per row, values from LDS rows of positions; the next block's K and V are
+// requested before the current one is multiplied. Workgroups of one key/value
+// head share an XCD's L2 (id modulo kv_heads), the longest rows first. The
+// library's fused kernel with its transposes took 41.6 us for 500 positions of 32
+// heads over 8 (128 workgroups), this one takes 22.5; at 128 / 1024 / 8000
+// positions 17.5 / 59.7 / 1388 and 9.1 / 42.9 / 1229.
+template <int DT, int HD>
+__global__ __launch_bounds__(kBlock) void nm_attention_prefill_kernel(PrefillArgs a) {
+  using E = Elem<DT>;
+  typedef typename E::scalar T;
+  constexpr int PB = 64;
+  constexpr int NK = HD / 32;   // 16-B loads per lane of K (and of V)
+  constexpr int KQ = HD / 32;   // MFMA steps over the head dimension
+  constexpr int DB = HD / 16;   // 16-column output blocks
+  constexpr int VS = PB + 8, PSTR = PB + 8;
+  __shared__ __attribute__((aligned(16))) T ks[HD * PB];
+  __shared__ __attribute__((aligned(16))) T vs[HD * VS];
+  __shared__ __attribute__((aligned(16))) T ps[4][16 * PSTR];
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, lg = lane >> 4, li = lane & 15;
+  const int id = (int)blockIdx.x;
+  const int kh = id % a.kvh, head = kh * a.g + (id / a.kvh) % a.g, qt = a.tiles - 1 - id / a.nh;
+  const int r0 = qt * PB + 16 * wave;  // the wave's first position
+
+  u32x4 qr[KQ];
+  const T* q = static_cast<const T*>(a.q) + ((long long)min(r0 + li, a.P - 1) * a.nh + head) * HD;
+#pragma unroll
+  for (int i = 0; i < KQ; ++i) qr[i] = *reinterpret_cast<const u32x4*>(q + 32 * i + 8 * lg);
+  const int krow = tid >> 3, kslot = tid & 7;  // 16 B of row krow + 32 i
+  const T* kb = static_cast<const T*>(a.k) + (long long)kh * a.k_head;
+  const T* vb = static_cast<const T*>(a.v) + (long long)kh * a.v_head;
+  u32x4 kr[NK], vr[NK];
+  auto load = [&](int blk) {
+    const int p = min(blk * PB + 8 * kslot, a.S - 8);
+#pragma unroll
+    for (int i = 0; i < NK; ++i) {
+      kr[i] = *reinterpret_cast<const u32x4*>(kb + (long long)(krow + 32 * i) * a.S + p);
+      vr[i] = *reinterpret_cast<const u32x4*>(vb + (long long)(krow + 32 * i) * a.S + p);
+    }
+  };
+  load(0);
+  f4 o[DB];
+#pragma unroll
+  for (int d = 0; d < DB; ++d) o[d] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+  float m[4], l[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) m[j] = -INFINITY, l[j] = 0.0f;
+  const int rr = 8 * lg + (li >> 2);
+
+  for (int blk = 0; blk <= qt; ++blk) {
+    __syncthreads();  // the previous block's reads are done
+    const int left = a.P - (blk * PB + 8 * kslot);  // cached positions past the prompt stay out of the sums
+    u32x4 keep;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) keep[e] = (left > 2 * e ? 0xffffu : 0u) | (left > 2 * e + 1 ? 0xffff0000u : 0u);
+#pragma unroll
+    for (int i = 0; i < NK; ++i) {
+      const int r = krow + 32 * i;
+      *reinterpret_cast<u32x4*>(&ks[r * PB + 8 * (kslot ^ (2 * (r & 3)))]) = kr[i];
+      *reinterpret_cast<u32x4*>(&vs[r * VS + 8 * kslot]) = vr[i] & keep;
+    }
+    __syncthreads();
+    if (blk < qt) load(blk + 1);
+
+    float sc[4][4];  // [16-position block][row 4 lg + j]
+#pragma unroll
+    for (int b = 0; b < 4; ++b) {
+      const int slot = 2 * b + ((li & 3) >> 1);
+      const T* kp = &ks[rr * PB + 8 * (slot ^ (2 * (rr & 3))) + 4 * (li & 1)];
+      f4 acc = f4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+      for (int i = 0; i < KQ; ++i) {
+        const s4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4*)(kp + 32 * i * PB));
+        const s4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4*)(kp + (32 * i + 4) * PB));
+        const s8 kf = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+        acc = mfma16x16x32<DT>(__builtin_bit_cast(s8, qr[i]), kf, acc);
+      }
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        sc[b][j] = blk < qt || 16 * b + li <= 16 * wave + 4 * lg + j ? acc[j] * a.scale : -INFINITY;
+    }
+    float alpha[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      float mx = max_nan(max_nan(sc[0][j], sc[1][j]), max_nan(sc[2][j], sc[3][j]));
+      mx = max_nan(m[j], row16(mx, [](float x, float y) { return max_nan(x, y); }));
+      alpha[j] = __builtin_amdgcn_exp2f(m[j] - mx);  // 0 at the first block
+      m[j] = mx;
+      float s = 0.0f;
+#pragma unroll
+      for (int b = 0; b < 4; ++b) {
+        const float p = __builtin_amdgcn_exp2f(sc[b][j] - mx);
+        s += p;
+        ps[wave][(4 * lg + j) * PSTR + 16 * b + li] = E::from_f32(p);
+      }
+      l[j] = l[j] * alpha[j] + row16(s, [](float x, float y) { return x + y; });
+    }
+#pragma unroll
+    for (int d = 0; d < DB; ++d)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) o[d][j] *= alpha[j];
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int i = 0; i < PB / 32; ++i) {
+      const s8 pa = __builtin_bit_cast(s8, *reinterpret_cast<const u32x4*>(&ps[wave][li * PSTR + 32 * i + 8 * lg]));
+#pragma unroll
+      for (int d = 0; d < DB; ++d)
+        o[d] = mfma16x16x32<DT>(
+            pa, __builtin_bit_cast(s8, *reinterpret_cast<const u32x4*>(&vs[(16 * d + li) * VS + 32 * i + 8 * lg])), o[d]);
+    }
+    __builtin_amdgcn_wave_barrier();
+  }
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int r = r0 + 4 * lg + j;
+    if (r >= a.P) continue;
+    T* out = static_cast<T*>(a.out) + ((long long)r * a.nh + head) * HD + li;
+    const float inv = 1.0f / l[j];
+#pragma unroll
+    for (int d = 0; d < DB; ++d) out[16 * d] = E::from_f32(o[d][j] * inv);
+  }
+}
+
 }  // namespace
 }  // namespace nm_hip
 
@@ -459,6 +697,74 @@ int nm_attention_decode(int dtype, const void* q, long long q_row_stride, const 
   a.scale = 1.44269504088896340736f / sqrtf((float)head_dim);
   const AttnFn fn = kAttnKernels[dtype == NM_DTYPE_F16 ? 0 : 1][head_dim / 128][p.npb / 2];
   hipLaunchKernelGGL(fn, dim3((unsigned)(p.splits * kv_heads)), dim3(kBlock), 0, static_cast<hipStream_t>(stream), a);
+  const hipError_t e = hipGetLastError();
+  return e == hipSuccess ? NM_OK : (int)e;
+}
+
+int nm_prefill_rope(int dtype, const void* q, long long q_row_stride, const void* k, long long k_row_stride,
+                    const void* v, long long v_row_stride, const void* q_norm, const void* k_norm, float eps,
+                    const float* rope_table, int P, int n_heads, int kv_heads, int head_dim, void* q_out,
+                    void* k_cache_t, long long k_head_stride, void* v_cache_t, long long v_head_stride, int cache_len,
+                    void* stream) {
+  if (dtype != NM_DTYPE_F16 && dtype != NM_DTYPE_BF16) return NM_ERR_BAD_CONFIG;
+  if (P <= 0 || n_heads <= 0 || kv_heads <= 0 || (head_dim != 64 && head_dim != 128) || cache_len < P ||
+      cache_len % 8 != 0 || n_heads + 2LL * kv_heads > 65535)
+    return NM_ERR_BAD_SHAPE;
+  const long long qd = (long long)n_heads * head_dim, kd = (long long)kv_heads * head_dim;
+  const long long row = (long long)head_dim * cache_len;
+  if (q_row_stride < qd || k_row_stride < kd || v_row_stride < kd || k_head_stride < row || v_head_stride < row)
+    return NM_ERR_BAD_SHAPE;
+  if (!q || !k || !v || !rope_table || !q_out || !k_cache_t || !v_cache_t) return NM_ERR_NULL_POINTER;
+  if (((q_row_stride | k_row_stride | v_row_stride | k_head_stride | v_head_stride) & 7) != 0 ||
+      ((uintptr_t)q | (uintptr_t)k | (uintptr_t)v | (uintptr_t)q_out | (uintptr_t)k_cache_t | (uintptr_t)v_cache_t) %
+              16 != 0 ||
+      (uintptr_t)rope_table % 8 != 0)
+    return NM_ERR_MISALIGNED;
+  if ((q_norm || k_norm) && !(eps >= 0.0f)) return NM_ERR_BAD_EPILOGUE;
+  RopeArgs a;
+  memset(&a, 0, sizeof(a));
+  a.q = q, a.k = k, a.v = v;
+  a.q_stride = q_row_stride, a.k_stride = k_row_stride, a.v_stride = v_row_stride;
+  a.q_norm = q_norm, a.k_norm = k_norm, a.eps = eps;
+  a.rope = reinterpret_cast<const float2*>(rope_table);
+  a.q_out = q_out, a.k_cache = k_cache_t, a.v_cache = v_cache_t;
+  a.k_head = k_head_stride, a.v_head = v_head_stride;
+  a.P = P, a.nh = n_heads, a.kvh = kv_heads, a.S = cache_len;
+  typedef void (*Fn)(RopeArgs);
+  const Fn fns[2][2] = {{&nm_prefill_rope_kernel<NM_DTYPE_F16, 64>, &nm_prefill_rope_kernel<NM_DTYPE_F16, 128>},
+                        {&nm_prefill_rope_kernel<NM_DTYPE_BF16, 64>, &nm_prefill_rope_kernel<NM_DTYPE_BF16, 128>}};
+  hipLaunchKernelGGL(fns[dtype == NM_DTYPE_F16 ? 0 : 1][head_dim / 128],
+                     dim3((unsigned)((P + 63) / 64), (unsigned)(n_heads + 2 * kv_heads)), dim3(kBlock), 0,
+                     static_cast<hipStream_t>(stream), a);
+  const hipError_t e = hipGetLastError();
+  return e == hipSuccess ? NM_OK : (int)e;
+}
+
+int nm_attention_prefill(int dtype, const void* q, const void* k_cache_t, long long k_head_stride,
+                         const void* v_cache_t, long long v_head_stride, void* out, int P, int n_heads, int kv_heads,
+                         int head_dim, int cache_len, void* stream) {
+  if (dtype != NM_DTYPE_F16 && dtype != NM_DTYPE_BF16) return NM_ERR_BAD_CONFIG;
+  if (P <= 0 || n_heads <= 0 || kv_heads <= 0 || n_heads % kv_heads != 0 || (head_dim != 64 && head_dim != 128) ||
+      cache_len < P || cache_len % 8 != 0)
+    return NM_ERR_BAD_SHAPE;
+  const long long row = (long long)head_dim * cache_len, tiles = (P + 63) / 64;
+  if (k_head_stride < row || v_head_stride < row || tiles * n_heads > 0x7fffffffLL) return NM_ERR_BAD_SHAPE;
+  if (!q || !k_cache_t || !v_cache_t || !out) return NM_ERR_NULL_POINTER;
+  if (((k_head_stride | v_head_stride) & 7) != 0 ||
+      ((uintptr_t)q | (uintptr_t)k_cache_t | (uintptr_t)v_cache_t | (uintptr_t)out) % 16 != 0)
+    return NM_ERR_MISALIGNED;
+  PrefillArgs a;
+  memset(&a, 0, sizeof(a));
+  a.q = q, a.k = k_cache_t, a.v = v_cache_t, a.out = out;
+  a.k_head = k_head_stride, a.v_head = v_head_stride;
+  a.P = P, a.nh = n_heads, a.kvh = kv_heads, a.g = n_heads / kv_heads, a.S = cache_len, a.tiles = (int)tiles;
+  a.scale = 1.44269504088896340736f / sqrtf((float)head_dim);
+  typedef void (*Fn)(PrefillArgs);
+  const Fn fns[2][2] = {
+      {&nm_attention_prefill_kernel<NM_DTYPE_F16, 64>, &nm_attention_prefill_kernel<NM_DTYPE_F16, 128>},
+      {&nm_attention_prefill_kernel<NM_DTYPE_BF16, 64>, &nm_attention_prefill_kernel<NM_DTYPE_BF16, 128>}};
+  hipLaunchKernelGGL(fns[dtype == NM_DTYPE_F16 ? 0 : 1][head_dim / 128], dim3((unsigned)(tiles * n_heads)),
+                     dim3(kBlock), 0, static_cast<hipStream_t>(stream), a);
   const hipError_t e = hipGetLastError();
   return e == hipSuccess ? NM_OK : (int)e;
 }

@@ -305,6 +305,30 @@ def causal_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, n_kv_hea
     return o.squeeze(0).transpose(0, 1).reshape(P, nh * d)
 
 
+def prompt_attention(at, q, k, v, freqs, rope, k_cache_t, v_cache_t) -> torch.Tensor:
+    """The attention of a whole prompt from its projections q [P, q], k and v
+    [P, kv] (at: the attention module): head norms, rotary embedding (freqs
+    complex64 [P, 1, head_dim / 2] or the same as the fp32 table rope), keys and
+    values into the caches at positions 0 .. P-1, causal attention. Where the
+    layer decodes on the library's attention kernel (attend_at), the library's
+    two prompt launches. Returns [P, q]."""
+    c = at.cfg
+    hd, P = c.head_dim, q.shape[0]
+    if at.decode_kernel and q.dtype == k_cache_t.dtype:
+        from ..hip_spmv import nmsparse_prefill_attention
+
+        return nmsparse_prefill_attention(q, k, v, k_cache_t, v_cache_t, rope, hd,
+                                          q_norm=at.q_norm.weight if c.qk_norm else None,
+                                          k_norm=at.k_norm.weight if c.qk_norm else None, norm_eps=c.norm_eps)
+    q, k, v = q.reshape(P, c.n_heads, hd), k.reshape(P, c.n_kv_heads, hd), v.reshape(P, c.n_kv_heads, hd)
+    if c.qk_norm:
+        q, k = at.q_norm(q), at.k_norm(k)
+    q, k = rotate(q, freqs), rotate(k, freqs)
+    k_cache_t[:, :hd, :P].copy_(k.permute(1, 2, 0))
+    v_cache_t[:, :, :P].copy_(v.permute(1, 2, 0))
+    return causal_attention(q, k, v, c.n_kv_heads)
+
+
 def grouped_sparse(mods) -> bool:
     """True when every module is an NmSparseLinear with the same w and N:M, so
     they can share one launch (grouped GEMV, or the gate/up pair)."""
@@ -925,8 +949,8 @@ class Decoder(nn.Module):
         """The prompt in one pass: tokens [P] int64 at positions 0 .. P-1 on
         the device. Every Linear sees all P rows (sparse ones through the SpMM:
         project_rows; q/k/v and gate/up as one grouped SpMM each,
-        project_rows_group), causal attention over the prompt in PyTorch
-        (causal_attention), keys and values written to the static caches at
+        project_rows_group), causal attention over the prompt
+        (prompt_attention), keys and values written to the static caches at
         positions 0 .. P-1 as the decode steps write them. Returns the logits
         of position P-1 [1, vocab]; decoding continues at position P (each
         step rewrites the mask rows itself)."""
@@ -952,13 +976,8 @@ class Decoder(nn.Module):
                 gate, up, down = ff.w1, ff.w3, ff.w2
                 h = ln1(x)
                 q, k, v = project_rows(at.wqkv, h).split([qd, kvd, kvd], dim=-1)
-            q, k, v = q.reshape(P, c.n_heads, hd), k.reshape(P, c.n_kv_heads, hd), v.reshape(P, c.n_kv_heads, hd)
-            if c.qk_norm:
-                q, k = at.q_norm(q), at.k_norm(k)
-            q, k = rotate(q, freqs), rotate(k, freqs)
-            self.k_cache_t[i][:, :hd, :P].copy_(k.permute(1, 2, 0))
-            self.v_cache_t[i][:, :, :P].copy_(v.permute(1, 2, 0))
-            x = x + project_rows(o_proj, causal_attention(q, k, v, c.n_kv_heads))
+            y = prompt_attention(at, q, k, v, freqs, self.rope_real, self.k_cache_t[i], self.v_cache_t[i])
+            x = x + project_rows(o_proj, y)
             h = ln2(x)
             g_out, u_out = project_rows_group((gate, up), h)
             x = x + project_rows_silu_mul(down, g_out, u_out)

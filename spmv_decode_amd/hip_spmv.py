@@ -1022,6 +1022,52 @@ def nmsparse_attention_decode(q, k_cache_t, v_cache_t, pos, head_dim, *, out=Non
     return out
 
 
+def nmsparse_prefill_attention(q, k, v, k_cache_t, v_cache_t, rope_table, head_dim, *, q_norm=None, k_norm=None,
+                               norm_eps=0.0):
+    """A prompt's attention in two launches: q [P, n_heads * head_dim], k and v
+    [P, kv_heads * head_dim] (the projections' rows, unit last stride) get
+    their optional per-head RMSNorms ([head_dim] weights) and rotary embedding
+    (rope_table fp32 [>= P, head_dim / 2, 2]), keys and values go into the
+    caches at positions 0 .. P-1, and every position attends causally. Returns
+    [P, n_heads * head_dim]. The caches must be ones attention_supported takes."""
+    P = q.shape[0]
+    kvh, kd, S = k_cache_t.shape
+    nh = q.shape[1] // head_dim
+    if nh % kvh or not attention_supported(q.new_empty(nh, head_dim), k_cache_t, v_cache_t, head_dim):
+        raise ValueError(f"prompt attention over q {tuple(q.shape)} {q.dtype}, k {tuple(k_cache_t.shape)}, "
+                         f"v {tuple(v_cache_t.shape)} with head_dim {head_dim} is not supported")
+    for name, t, heads in (("q", q, nh), ("k", k, kvh), ("v", v, kvh)):
+        if (t.dim() != 2 or tuple(t.shape) != (P, heads * head_dim) or t.stride(1) != 1 or t.stride(0) % 8
+                or t.dtype != q.dtype or t.device != q.device or t.data_ptr() % 16):
+            raise ValueError(f"{name} must be 16-byte aligned rows [{P}, {heads * head_dim}] of {q.dtype}")
+    if P < 1 or P > S:
+        raise ValueError(f"prompt of {P} positions for a cache of {S}")
+    rt = torch.view_as_real(rope_table) if rope_table.is_complex() else rope_table
+    if (rt.dtype != torch.float32 or rt.ndim != 3 or rt.shape[0] < P or rt.shape[1:] != (head_dim // 2, 2)
+            or not rt.is_contiguous() or rt.device != q.device):
+        raise ValueError(f"rope_table must be contiguous fp32 [>= {P}, {head_dim // 2}, 2] (or complex64) on the device")
+    for norm in (q_norm, k_norm):
+        if norm is not None:
+            _check_vector(norm, head_dim, q, "head norm")
+    lib = _lib.load()
+    code = _DTYPE_CODE[q.dtype]
+    qr = torch.empty(P, nh * head_dim, dtype=q.dtype, device=q.device)
+    out = torch.empty_like(qr)
+    with torch.cuda.device(q.device):
+        stream = torch.cuda.current_stream(q.device).cuda_stream
+        rc = lib.nm_prefill_rope(code, q.data_ptr(), q.stride(0), k.data_ptr(), k.stride(0), v.data_ptr(), v.stride(0),
+                                 None if q_norm is None else q_norm.data_ptr(),
+                                 None if k_norm is None else k_norm.data_ptr(), float(norm_eps), rt.data_ptr(), P, nh,
+                                 kvh, int(head_dim), qr.data_ptr(), k_cache_t.data_ptr(), k_cache_t.stride(0),
+                                 v_cache_t.data_ptr(), v_cache_t.stride(0), S, stream)
+        _lib.check(rc, "nm_prefill_rope")
+        rc = lib.nm_attention_prefill(code, qr.data_ptr(), k_cache_t.data_ptr(), k_cache_t.stride(0),
+                                      v_cache_t.data_ptr(), v_cache_t.stride(0), out.data_ptr(), P, nh, kvh,
+                                      int(head_dim), S, stream)
+        _lib.check(rc, "nm_attention_prefill")
+    return out
+
+
 def dense_gemv_supported(x: torch.Tensor, weight: torch.Tensor) -> bool:
     """Whether nmsparse_dense_gemv takes x [..., K] (one row) and weight [n, K]:
     fp16 / bf16 on one GPU, unit strides along K, K a multiple of 8 up to 8192,
@@ -1056,4 +1102,4 @@ __all__ = ["nmsparse_spmv_forward_hip", "nmsparse_spmv_forward_triton_ptx", "nms
            "nmsparse_gemv_partials", "carry_splits", "GemvProblem", "launch_plan", "validate_args", "workspace_for",
            "nmsparse_gemv_accumulate", "nmsparse_gate_up_accumulate", "nmsparse_gemv_silu", "gate_up_ssq_slots",
            "library_route", "rows_route", "attention_supported", "nmsparse_attention_decode",
-           "dense_gemv_supported", "nmsparse_dense_gemv"]
+           "dense_gemv_supported", "nmsparse_dense_gemv", "nmsparse_prefill_attention"]

@@ -70,3 +70,51 @@ def test_attention_decode_edges(gpu):
         assert not hip_spmv.attention_supported(*bad, 128)
         with pytest.raises(ValueError):
             hip_spmv.nmsparse_attention_decode(*bad, torch.tensor([3], device="cuda"), 128)
+
+
+# (positions, query heads, key/value heads, head_dim, cache length, padded key rows, norms, row padding)
+PROMPTS = [(1, 4, 2, 64, 8, 32, False, 0), (63, 32, 8, 128, 640, 32, False, 0), (64, 16, 8, 128, 128, 0, True, 0),
+           (65, 6, 2, 128, 72, 32, True, 64), (200, 40, 8, 128, 256, 32, True, 0), (333, 4, 4, 64, 336, 0, False, 8),
+           (520, 16, 1, 128, 1024, 32, False, 0)]
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16], ids=str)
+@pytest.mark.parametrize("case", PROMPTS, ids=str)
+def test_prompt_attention_matches_exact(gpu, case, dtype):
+    P, nh, kvh, hd, S, pad, norms, rowpad = case
+    gen = torch.Generator(device="cuda").manual_seed(P + nh)
+
+    def rows(heads):
+        return torch.randn(P, heads * hd + rowpad, device="cuda", generator=gen).to(dtype)[:, :heads * hd]
+
+    q, k, v = rows(nh), rows(kvh), rows(kvh)
+    qn, kn = ((1 + 0.1 * torch.randn(2, hd, device="cuda", generator=gen)).to(dtype).unbind(0) if norms
+              else (None, None))
+    ang = torch.rand(S, hd // 2, device="cuda", generator=gen, dtype=torch.float64) * 6.28
+    table = torch.view_as_real(torch.polar(torch.ones_like(ang), ang).to(torch.complex64)).contiguous()
+    kc = torch.full((kvh, hd + pad, S), float("nan"), device="cuda", dtype=dtype)  # stale contents stay out
+    vc = torch.full((kvh, hd, S), float("nan"), device="cuda", dtype=dtype)
+    y = hip_spmv.nmsparse_prefill_attention(q, k, v, kc, vc, table, hd, q_norm=qn, k_norm=kn, norm_eps=1e-6)
+
+    def turned(t, heads, norm):
+        t = t.double().view(P, heads, hd)
+        if norm is not None:
+            t = t * torch.rsqrt(t.square().mean(-1, keepdim=True) + 1e-6) * norm.double()
+        c, s = table[:P, None, :, 0].double(), table[:P, None, :, 1].double()
+        a, b = t[..., 0::2], t[..., 1::2]
+        return torch.stack((a * c - b * s, a * s + b * c), dim=-1).flatten(-2)
+
+    eps = torch.finfo(dtype).eps
+    kr = turned(k, kvh, kn)
+    assert float((kc[:, :hd, :P].double() - kr.permute(1, 2, 0)).norm() / kr.norm()) <= eps  # one rounding
+    assert torch.equal(vc[:, :, :P], v.reshape(P, kvh, hd).permute(1, 2, 0))
+    assert bool(torch.isnan(kc[:, hd:]).all()) and bool(torch.isnan(kc[:, :, P:]).all())
+    assert bool(torch.isnan(vc[:, :, P:]).all())
+    # attention of the rounded queries and keys in 64 bits
+    qr, kr = turned(q, nh, qn).to(dtype).double(), kc[:, :hd, :P].double()
+    s = torch.bmm(qr.transpose(0, 1).contiguous(), kr.repeat_interleave(nh // kvh, 0).contiguous()) / math.sqrt(hd)
+    s = s.masked_fill(torch.ones(P, P, dtype=torch.bool, device="cuda").triu(1), -math.inf)
+    ref = torch.bmm(torch.softmax(s, -1), vc[:, :, :P].double().transpose(1, 2).repeat_interleave(nh // kvh, 0)
+                    .contiguous()).transpose(0, 1).reshape(P, nh * hd)
+    rel = float((y.double() - ref).norm() / ref.norm())
+    assert rel <= 2 * eps, rel

@@ -28,6 +28,7 @@ capture id, so two graphs never share one.
 """
 from __future__ import annotations
 
+import contextlib
 import ctypes
 import warnings
 
@@ -49,6 +50,22 @@ _retired: list[torch.Tensor] = []
 # active: the graph's pool then keeps the memory for its replays, as it does
 # for every intermediate tensor of the capture.
 _capture_workspaces: dict[tuple[int, int], list[torch.Tensor]] = {}
+
+
+_HERE = contextlib.nullcontext()
+
+
+def _on_device(device: torch.device):
+    """A guard that makes `device` current: nothing to do when it is (the
+    device guard's round trip is 1.4 us of a 12.7 us call, this test 0.3)."""
+    return _HERE if torch.cuda.current_device() == device.index else torch.cuda.device(device)
+
+
+def _raw_stream(device: torch.device) -> int:
+    """Handle of `device`'s current stream, without the stream object around it
+    (0.1 us against 1.9)."""
+    index = device.index
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
 
 
 def capture_id(stream_ptr: int) -> int:
@@ -194,8 +211,8 @@ def nmsparse_spmv_forward_hip(
     if need == 0:
         raise ValueError(f"shape h={h}, w={w}, N={nnz}, M={m} (config {config_id}, splits {splits}) "
                          "is outside what libnmsparse_hip supports")
-    with torch.cuda.device(device):
-        stream = torch.cuda.current_stream(device).cuda_stream
+    with _on_device(device):
+        stream = _raw_stream(device)
         ws = workspace_for(device, need, stream)
         args = (vec.data_ptr(), vec.stride(1), mat_data.data_ptr(), mat_index.data_ptr(), out.data_ptr(),
                 ws.data_ptr(), ws.numel(), h, w, nnz, m)
@@ -329,11 +346,11 @@ def nmsparse_spmm_forward_hip(x, mat_data, mat_index, w, h, BLOCK_WIDTH, VEC_WID
         return out
     if library_gemm:
         wp = (w + 7) // 8 * 8
-        with torch.cuda.device(x.device):
+        with _on_device(x.device):
             xg = torch.empty(rows, wp, dtype=x.dtype, device=x.device)
             rc = lib.nm_gather_columns(_DTYPE_CODE[x.dtype], x2d.data_ptr(), K, rows, mat_index.data_ptr(), w,
                                        BLOCK_WIDTH, VEC_WIDTH, xg.data_ptr(), wp,
-                                       torch.cuda.current_stream(x.device).cuda_stream)
+                                       _raw_stream(x.device))
             _lib.check(rc, "nm_gather_columns")
             torch.matmul(xg[:, :w], md, out=out.view(rows, h))
         return out
@@ -347,8 +364,8 @@ def nmsparse_spmm_forward_hip(x, mat_data, mat_index, w, h, BLOCK_WIDTH, VEC_WID
     o2d = out.view(rows, h)
     esize = x.element_size()
     device = x.device
-    with torch.cuda.device(device):
-        stream = torch.cuda.current_stream(device).cuda_stream
+    with _on_device(device):
+        stream = _raw_stream(device)
         ws = workspace_for(device, need, stream)
         for r0 in range(0, rows, per):
             b = min(per, rows - r0)
@@ -385,9 +402,9 @@ def nmsparse_spmm_silu_mul_hip(gate, up, mat_data, mat_index, w, h, BLOCK_WIDTH,
                 and gate.is_contiguous() and up.is_contiguous()
                 and gate.data_ptr() % 16 == 0 and up.data_ptr() % 16 == 0):
             act = torch.empty_like(gate)
-            with torch.cuda.device(gate.device):
+            with _on_device(gate.device):
                 rc = _lib.load().nm_silu_mul(_DTYPE_CODE[gate.dtype], gate.data_ptr(), up.data_ptr(), act.data_ptr(),
-                                             gate.numel(), torch.cuda.current_stream(gate.device).cuda_stream)
+                                             gate.numel(), _raw_stream(gate.device))
             _lib.check(rc, "nm_silu_mul")
         else:
             act = (torch.nn.functional.silu(gate.float()) * up.float()).to(gate.dtype)
@@ -423,19 +440,19 @@ def nmsparse_spmm_silu_mul_hip(gate, up, mat_data, mat_index, w, h, BLOCK_WIDTH,
     lib = _lib.load()
     if wide:
         wp = (w + 7) // 8 * 8
-        with torch.cuda.device(gate.device):
+        with _on_device(gate.device):
             xg = torch.empty(rows, wp, dtype=gate.dtype, device=gate.device)
             rc = lib.nm_gather_columns_silu_mul(_DTYPE_CODE[gate.dtype], g2d.data_ptr(), u2d.data_ptr(), K, rows,
                                                 mat_index.data_ptr(), w, BLOCK_WIDTH, VEC_WIDTH, xg.data_ptr(), wp,
-                                                torch.cuda.current_stream(gate.device).cuda_stream)
+                                                _raw_stream(gate.device))
             _lib.check(rc, "nm_gather_columns_silu_mul")
             torch.matmul(xg[:, :w], md, out=out.view(rows, h))
         return out
     need = lib.nm_spmm_mc_workspace_bytes(rows, h, w, BLOCK_WIDTH, VEC_WIDTH, int(config_id), int(splits))
     if need == 0:
         raise ValueError("spmm shape outside what libnmsparse_hip supports")
-    with torch.cuda.device(gate.device):
-        stream = torch.cuda.current_stream(gate.device).cuda_stream
+    with _on_device(gate.device):
+        stream = _raw_stream(gate.device)
         ws = workspace_for(gate.device, need, stream)
         rc = lib.nm_spmm_mc_silu_mul(_DTYPE_CODE[gate.dtype], g2d.data_ptr(), u2d.data_ptr(), K, rows, md.data_ptr(),
                                      mat_index.data_ptr(), out.data_ptr(), h, ws.data_ptr(), ws.numel(), h, w,
@@ -528,8 +545,8 @@ def nmsparse_spmm_group_hip(x, mats, BLOCK_WIDTH, VEC_WIDTH, *, outs=None, confi
     mds_arr = (ctypes.c_void_p * n)(*[md.data_ptr() for md in mds])
     mis_arr = (ctypes.c_void_p * n)(*[mi.data_ptr() for _, mi in mats])
     ostr = (ctypes.c_longlong * n)(*hs)
-    with torch.cuda.device(x.device):
-        stream = torch.cuda.current_stream(x.device).cuda_stream
+    with _on_device(x.device):
+        stream = _raw_stream(x.device)
         ws = workspace_for(x.device, need, stream)
         if small:
             outs_arr = (ctypes.c_void_p * n)(*[o.data_ptr() for o in res])
@@ -566,8 +583,8 @@ def _spmm_rows(x2d, mats, w, BLOCK_WIDTH, VEC_WIDTH, outs, *, up2d=None, splits=
     mis_arr = (ctypes.c_void_p * n)(*[mi.data_ptr() for _, mi in mats])
     outs_arr = (ctypes.c_void_p * n)(*[o.data_ptr() for o in outs])
     ostr = (ctypes.c_longlong * n)(*hs)
-    with torch.cuda.device(x2d.device):
-        stream = torch.cuda.current_stream(x2d.device).cuda_stream
+    with _on_device(x2d.device):
+        stream = _raw_stream(x2d.device)
         ws = workspace_for(x2d.device, _lib.NM_TICKET_BYTES, stream)
         scratch = torch.empty(need, dtype=torch.uint8, device=x2d.device)
         rc = lib.nm_spmm_rows(_DTYPE_CODE[x2d.dtype], x2d.data_ptr(), None if up2d is None else up2d.data_ptr(), K,
@@ -807,8 +824,8 @@ def nmsparse_gemv_launch(vec, problems, BLOCK_WIDTH, VEC_WIDTH, *, gate_up=False
     if need == 0:
         raise ValueError("launch shape outside what libnmsparse_hip supports")
     device = vec.device
-    with torch.cuda.device(device):
-        stream = torch.cuda.current_stream(device).cuda_stream
+    with _on_device(device):
+        stream = _raw_stream(device)
         ws = workspace_for(device, need, stream)
         rc = lib.nm_gemv_launch(ctypes.byref(desc), ws.data_ptr(), ws.numel(), stream)
     _lib.check(rc, "nm_gemv_launch")
@@ -1011,8 +1028,8 @@ def nmsparse_attention_decode(q, k_cache_t, v_cache_t, pos, head_dim, *, out=Non
     need = lib.nm_attention_decode_workspace_bytes(nh, kvh, int(head_dim), S, int(span))
     if need == 0:
         raise ValueError(f"span {span} is outside what libnmsparse_hip supports for {S} positions")
-    with torch.cuda.device(q.device):
-        stream = torch.cuda.current_stream(q.device).cuda_stream
+    with _on_device(q.device):
+        stream = _raw_stream(q.device)
         ws = workspace_for(q.device, need, stream)
         rc = lib.nm_attention_decode(_DTYPE_CODE[q.dtype], q.data_ptr(), q.stride(0), k_cache_t.data_ptr(),
                                      k_cache_t.stride(0), v_cache_t.data_ptr(), v_cache_t.stride(0), out.data_ptr(),
@@ -1053,8 +1070,8 @@ def nmsparse_prefill_attention(q, k, v, k_cache_t, v_cache_t, rope_table, head_d
     code = _DTYPE_CODE[q.dtype]
     qr = torch.empty(P, nh * head_dim, dtype=q.dtype, device=q.device)
     out = torch.empty_like(qr)
-    with torch.cuda.device(q.device):
-        stream = torch.cuda.current_stream(q.device).cuda_stream
+    with _on_device(q.device):
+        stream = _raw_stream(q.device)
         rc = lib.nm_prefill_rope(code, q.data_ptr(), q.stride(0), k.data_ptr(), k.stride(0), v.data_ptr(), v.stride(0),
                                  None if q_norm is None else q_norm.data_ptr(),
                                  None if k_norm is None else k_norm.data_ptr(), float(norm_eps), rt.data_ptr(), P, nh,
@@ -1090,9 +1107,9 @@ def nmsparse_dense_gemv(x, weight):
                          "is not supported")
     n, K = weight.shape
     y = torch.empty(1, n, dtype=x.dtype, device=x.device)
-    with torch.cuda.device(x.device):
+    with _on_device(x.device):
         rc = _lib.load().nm_dense_gemv(_DTYPE_CODE[x.dtype], x.data_ptr(), weight.data_ptr(), weight.stride(0),
-                                       y.data_ptr(), n, K, torch.cuda.current_stream(x.device).cuda_stream)
+                                       y.data_ptr(), n, K, _raw_stream(x.device))
     _lib.check(rc, "nm_dense_gemv")
     return y
 

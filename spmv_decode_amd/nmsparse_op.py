@@ -86,8 +86,9 @@ def gemv(x: torch.Tensor, mat_data: torch.Tensor, mat_index: torch.Tensor,
     md = mat_data if mat_data.dtype == torch.float16 else mat_data.to(torch.float16)
     out = nmsparse_spmv_forward_hip(xh, md, mat_index, int(w), int(h), int(block_width), 128,
                                     int(vec_width), 1, int(K))
-    out = out.to(dtype=x.dtype)
-    return out.reshape(*x.shape[:-1], int(h))
+    if x.dtype != torch.float16:
+        out = out.to(dtype=x.dtype)
+    return out.view(*x.shape[:-1], int(h))
 
 
 @gemv.register_fake

@@ -232,12 +232,22 @@ def project(lin: nn.Module, x: torch.Tensor) -> torch.Tensor:
     return lin(x)
 
 
+def records_grad(*tensors) -> bool:
+    """Whether autograd records what is computed from these tensors."""
+    return torch.is_grad_enabled() and any(t.requires_grad for t in tensors)
+
+
 def project_head(lin: nn.Module, x: torch.Tensor, kernel: bool) -> torch.Tensor:
     """The output head on one row x [..., dim] -> [1, vocab]: in the library's
-    dense GEMV when `kernel` (Decoder.setup_cache found it to take the weight),
-    else project."""
-    if kernel and type(lin) is nn.Linear and lin.bias is None and lin.weight.dtype == x.dtype:
-        return torch.ops.nmsparse.dense_gemv(x.reshape(1, -1), lin.weight)
+    dense GEMV when `kernel` (Decoder.setup_cache found it to take the weight)
+    and it takes these operands, else, and where autograd records, project."""
+    if (kernel and type(lin) is nn.Linear and lin.bias is None and lin.weight.dtype == x.dtype
+            and not records_grad(x, lin.weight)):
+        from ..hip_spmv import dense_gemv_supported
+
+        row = x.reshape(1, -1)
+        if torch.compiler.is_compiling() or dense_gemv_supported(row, lin.weight):
+            return torch.ops.nmsparse.dense_gemv(row, lin.weight)
     return project(lin, x).view(1, -1)
 
 
@@ -310,11 +320,15 @@ def prompt_attention(at, q, k, v, freqs, rope, k_cache_t, v_cache_t) -> torch.Te
     [P, kv] (at: the attention module): head norms, rotary embedding (freqs
     complex64 [P, 1, head_dim / 2] or the same as the fp32 table rope), keys and
     values into the caches at positions 0 .. P-1, causal attention. Where the
-    layer decodes on the library's attention kernel (attend_at), the library's
-    two prompt launches. Returns [P, q]."""
+    layer decodes on the library's attention kernel (attend_at) and these
+    operands are within its forms, the library's two prompt launches. Returns
+    [P, q]."""
     c = at.cfg
     hd, P = c.head_dim, q.shape[0]
-    if at.decode_kernel and q.dtype == k_cache_t.dtype:
+    rows = at.decode_kernel and all(t.stride(1) == 1 and t.stride(0) % 8 == 0 and t.data_ptr() % 16 == 0
+                                    and t.dtype == k_cache_t.dtype for t in (q, k, v))
+    norms = (at.q_norm.weight, at.k_norm.weight) if c.qk_norm else ()
+    if rows and all(t.dtype == q.dtype and t.is_contiguous() for t in norms):
         from ..hip_spmv import nmsparse_prefill_attention
 
         return nmsparse_prefill_attention(q, k, v, k_cache_t, v_cache_t, rope, hd,

@@ -46,3 +46,42 @@ def test_dense_gemv_special_values_and_refusals(gpu):
     assert lib.nm_dense_gemv(0, x.data_ptr(), w.data_ptr(), 1032, y.data_ptr(), 40, 8200, None) == -2
     assert lib.nm_dense_gemv(2, x.data_ptr(), w.data_ptr(), 1032, y.data_ptr(), 40, 64, None) == -7
     assert lib.nm_dense_gemv(0, None, w.data_ptr(), 1032, y.data_ptr(), 40, 64, None) == -1
+
+
+def test_decode_step_keeps_the_heads_gradient(gpu):
+    """Where autograd records the output head, a decode step takes the
+    differentiable product: the weight gets its gradient, the logits are those
+    of the step without gradients to fp16 rounding."""
+    from dataclasses import replace
+
+    from spmv_decode_amd.decode.model import CONFIGS, Decoder
+
+    cfg = replace(CONFIGS["qwen3-0.6b"], n_layers=1, vocab=520)
+    torch.manual_seed(0)
+    model = Decoder(cfg).to("cuda", torch.float16).requires_grad_(False)
+    model.lm_head.weight.requires_grad_(True)
+    model.setup_cache(64, torch.device("cuda"))
+    assert model.head_kernel
+    token, pos = torch.tensor([[3]], device="cuda"), torch.tensor([0], device="cuda")
+    with torch.no_grad():
+        plain = model.forward_step(token, pos).double()
+    hidden = {}
+    model.norm.register_forward_hook(lambda m, a, out: hidden.setdefault("x", out.detach()))
+    logits = model.forward_step(token, pos)
+    # one rounding each
+    assert float((logits.double() - plain).norm() / plain.norm()) <= 2 * 2.0 ** -11
+    seed = torch.randn_like(logits)
+    grad, = torch.autograd.grad(logits, model.lm_head.weight, seed)
+    ref = seed.double().t() @ hidden["x"].double().view(1, -1)
+    assert float((grad.double() - ref).norm() / ref.norm()) <= 2.0 ** -10
+
+
+def test_head_takes_a_replaced_weight(gpu):
+    """A head whose weight the kernel does not take goes to the general product."""
+    from spmv_decode_amd.decode.model import project_head
+
+    head = torch.nn.Linear(64, 24, bias=False, device="cuda", dtype=torch.float16).requires_grad_(False)
+    head.weight.data = torch.randn(64, 24, device="cuda", dtype=torch.float16).t()
+    x = torch.randn(1, 1, 64, device="cuda", dtype=torch.float16)
+    y, ref = project_head(head, x, True).double(), x.view(1, -1).double() @ head.weight.double().t()
+    assert float((y - ref).norm() / ref.norm()) <= 2.0 ** -10

@@ -500,6 +500,16 @@ int nm_dense_gemv(int dtype, const void* x, const void* weight, long long row_st
                   void* stream);
 
 /*
+ * sum = x + d and out = sum / sqrt(mean(sum^2) + eps) * weight for rows of dim
+ * elements ([rows, dim] contiguous; weight [dim]): a residual add and the
+ * RMSNorm behind it. fp16 and bf16, fp32 arithmetic, one rounding of the sum
+ * and one of its norm; dim a multiple of 8 up to 8192, every pointer 16-byte
+ * aligned, sum and out apart from each other and from the inputs.
+ */
+int nm_add_rms_norm(int dtype, const void* x, const void* d, const void* weight, float eps, void* sum, void* out,
+                    int rows, int dim, void* stream);
+
+/*
  * The attention of one decode token over the transposed static caches:
  * out[h, :] = softmax over positions p <= *pos of q[h, :] . K[h / g, :, p] /
  * sqrt(head_dim), times V[h / g, :, p], with g = n_heads / kv_heads query heads

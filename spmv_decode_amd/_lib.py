@@ -105,6 +105,7 @@ ABI = {
     "nm_prefill_rope": (_i, [_i, _vp, _ll, _vp, _ll, _vp, _ll, _vp, _vp, ctypes.c_float, _vp, _i, _i, _i, _i, _vp, _vp,
                              _ll, _vp, _ll, _i, _vp]),
     "nm_attention_prefill": (_i, [_i, _vp, _vp, _ll, _vp, _ll, _vp, _i, _i, _i, _i, _i, _vp]),
+    "nm_add_rms_norm": (_i, [_i, _vp, _vp, _vp, ctypes.c_float, _vp, _vp, _i, _i, _vp]),
     "nm_dense_gemv": (_i, [_i, _vp, _vp, _ll, _vp, _i, _i, _vp]),
     "nm_attention_decode_workspace_bytes": (_sz, [_i, _i, _i, _i, _i]),
     "nm_attention_decode": (_i, [_i, _vp, _ll, _vp, _ll, _vp, _ll, _vp, _vp, _vp, _sz, _i, _i, _i, _i, _i, _vp]),

@@ -4,8 +4,9 @@
 
 The library is a plain C-ABI shared object (include/nmsparse_hip.h) compiled
 by hipcc from spmv_decode_amd/csrc/: nm_gemv.hip (host side and C ABI) and
-nm_gemv_inst.hip once per element type (the kernels) and nm_spmm_mc.hip (the
-matrix-core SpMM), compiled in parallel and linked; nothing links against torch.
+nm_gemv_inst.hip once per element type (the kernels), nm_spmm_mc.hip and
+nm_spmm_rows.hip (the matrix-core products), nm_attention.hip,
+nm_dense_gemv.hip and nm_norm.hip, compiled in parallel and linked; nothing links against torch.
 """
 from __future__ import annotations
 
@@ -23,7 +24,7 @@ CSRC = PKG / "csrc"
 # (source, extra defines): the host side, then the kernels of each element type.
 UNITS = [(CSRC / "nm_gemv.hip", []), *[(CSRC / "nm_gemv_inst.hip", [f"-DNM_INST_DTYPE={dt}"]) for dt in (0, 1, 2)],
          (CSRC / "nm_spmm_mc.hip", []), (CSRC / "nm_spmm_rows.hip", []), (CSRC / "nm_attention.hip", []),
-         (CSRC / "nm_dense_gemv.hip", [])]
+         (CSRC / "nm_dense_gemv.hip", []), (CSRC / "nm_norm.hip", [])]
 LIB_PATH = PKG / "libnmsparse_hip.so"
 # Measurement-only streaming-read kernel used by the microbenchmark.
 PROBE_SOURCES = [PKG / "csrc" / "roofline_probe.hip"]

@@ -251,6 +251,19 @@ def project_head(lin: nn.Module, x: torch.Tensor, kernel: bool) -> torch.Tensor:
     return project(lin, x).view(1, -1)
 
 
+def add_norm(norm: nn.Module, x: torch.Tensor, d: torch.Tensor) -> tuple:
+    """(x + d, norm(x + d)) for the rows x, d [rows, dim] of a prompt: one
+    launch of the library where it takes them (500 rows of 4096: 3.7 us where the
+    two calls take 8.8), the two calls elsewhere and for a norm that is not an RMSNorm or has hooks."""
+    if type(norm) is RMSNorm and x.is_cuda and not (norm._forward_hooks or norm._forward_pre_hooks):
+        from ..hip_spmv import add_rms_norm_supported, nmsparse_add_rms_norm
+
+        if add_rms_norm_supported(x, d, norm.weight) and not records_grad(x, d, norm.weight):
+            return nmsparse_add_rms_norm(x, d, norm.weight, norm.eps)
+    x = x + d
+    return x, norm(x)
+
+
 def project_rows(lin: nn.Module, x2d: torch.Tensor) -> torch.Tensor:
     """lin(x) for every row of x2d [rows, K] -> [rows, h]: an NmSparseLinear
     through the SpMM on its packed weights (the small-batch kernel up to 8
@@ -977,24 +990,26 @@ class Decoder(nn.Module):
         x = self.embed_tokens(ids)  # [P, dim]
         freqs = self.rope[:P].view(P, 1, -1)
         qd, kvd = c.n_heads * hd, c.n_kv_heads * hd
+        norms = [blk.input_layernorm if isinstance(blk, Block) else blk.attention_norm for blk in self.layers]
+        h = norms[0](x) if norms else x
         for i, blk in enumerate(self.layers):
             if isinstance(blk, Block):
                 at, mlp = blk.self_attn, blk.mlp
-                ln1, ln2, o_proj = blk.input_layernorm, blk.post_attention_layernorm, at.o_proj
+                ln2, o_proj = blk.post_attention_layernorm, at.o_proj
                 gate, up, down = mlp.gate_proj, mlp.up_proj, mlp.down_proj
-                h = ln1(x)
                 q, k, v = project_rows_group((at.q_proj, at.k_proj, at.v_proj), h)
             else:  # gpt-fast names
                 at, ff = blk.attention, blk.feed_forward
-                ln1, ln2, o_proj = blk.attention_norm, blk.ffn_norm, at.wo
+                ln2, o_proj = blk.ffn_norm, at.wo
                 gate, up, down = ff.w1, ff.w3, ff.w2
-                h = ln1(x)
                 q, k, v = project_rows(at.wqkv, h).split([qd, kvd, kvd], dim=-1)
             y = prompt_attention(at, q, k, v, freqs, self.rope_real, self.k_cache_t[i], self.v_cache_t[i])
-            x = x + project_rows(o_proj, y)
-            h = ln2(x)
-            g_out, u_out = project_rows_group((gate, up), h)
-            x = x + project_rows_silu_mul(down, g_out, u_out)
+            x, h = add_norm(ln2, x, project_rows(o_proj, y))
+            d = project_rows_silu_mul(down, *project_rows_group((gate, up), h))
+            if i + 1 < len(norms):
+                x, h = add_norm(norms[i + 1], x, d)
+            else:
+                x = x + d
         return project_head(self.lm_head, self.norm(x[-1:].view(1, 1, -1)), self.head_kernel)
 
     def forward_step(self, token: torch.Tensor, pos: torch.Tensor) -> torch.Tensor:

@@ -1085,6 +1085,35 @@ def nmsparse_prefill_attention(q, k, v, k_cache_t, v_cache_t, rope_table, head_d
     return out
 
 
+def add_rms_norm_supported(x: torch.Tensor, d: torch.Tensor, weight: torch.Tensor) -> bool:
+    """Whether nmsparse_add_rms_norm takes these operands: fp16 / bf16 on one
+    GPU, x and d contiguous [rows, dim], weight contiguous [dim], dim a
+    multiple of 8 up to 8192, 16-byte aligned. No GPU work."""
+    ts = (x, d, weight)
+    return (x.is_cuda and x.dtype in (torch.float16, torch.bfloat16) and x.dim() == 2 and x.shape == d.shape
+            and tuple(weight.shape) == (x.shape[1],) and 0 < x.shape[0] < 1 << 31 and 0 < x.shape[1] <= 8192
+            and x.shape[1] % 8 == 0
+            and all(t.dtype == x.dtype and t.device == x.device and t.is_contiguous() and t.data_ptr() % 16 == 0
+                    for t in ts))
+
+
+def nmsparse_add_rms_norm(x, d, weight, eps):
+    """(x + d, RMSNorm(x + d) * weight) of rows [rows, dim] in one launch, in
+    the arithmetic of the two PyTorch calls (add_rms_norm_supported says which
+    operands are taken)."""
+    if not add_rms_norm_supported(x, d, weight):
+        raise ValueError(f"add and RMSNorm of x {tuple(x.shape)} {x.dtype}, d {tuple(d.shape)} {d.dtype} and weight "
+                         f"{tuple(weight.shape)} {weight.dtype} is not supported")
+    rows, dim = x.shape
+    total, out = torch.empty_like(x), torch.empty_like(x)
+    with _on_device(x.device):
+        rc = _lib.load().nm_add_rms_norm(_DTYPE_CODE[x.dtype], x.data_ptr(), d.data_ptr(), weight.data_ptr(),
+                                         float(eps), total.data_ptr(), out.data_ptr(), rows, dim,
+                                         _raw_stream(x.device))
+    _lib.check(rc, "nm_add_rms_norm")
+    return total, out
+
+
 def dense_gemv_supported(x: torch.Tensor, weight: torch.Tensor) -> bool:
     """Whether nmsparse_dense_gemv takes x [..., K] (one row) and weight [n, K]:
     fp16 / bf16 on one GPU, unit strides along K, K a multiple of 8 up to 8192,

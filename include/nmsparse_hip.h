@@ -440,9 +440,13 @@ int nm_gather_columns_silu_mul(int dtype, const void* gate, const void* up, long
  * (nm_spmm_rows_scratch_bytes, any contents, 256-byte aligned) holds the
  * gathered activations and the split partials; of `workspace` (256-byte
  * aligned) only the zeroed arrival counters are used. splits 1 to 8, 0 = the
- * library's choice. fp32 accumulation, one rounding; splits summed in order.
+ * library's choice, plus NM_ROWS_SHORT or NM_ROWS_TALL for tiles of 128 or 256
+ * rows (neither: its choice). fp32 accumulation, one rounding; splits summed in
+ * order.
  */
 #define NM_ROWS_MAX 65536
+#define NM_ROWS_SHORT 256
+#define NM_ROWS_TALL 512
 size_t nm_spmm_rows_scratch_bytes(int rows, int n, const int* h, int w, int nnz, int m, int splits);
 int nm_spmm_rows_plan(int rows, int n, const int* h, int w, int nnz, int m, int splits, int* out_splits,
                       int* out_blocks);

@@ -31,6 +31,7 @@ NM_MAX_BATCH = 8
 NM_MC_MAX_BATCH = 128
 NM_MC_MAX_GROUP = 4
 NM_ROWS_MAX = 65536
+NM_ROWS_SHORT, NM_ROWS_TALL = 256, 512  # added to a split count: tiles of 128 / 256 rows
 NM_STATIC_SCRATCH_BYTES = NM_TICKET_BYTES + (16 << 20)
 
 _vp = ctypes.c_void_p

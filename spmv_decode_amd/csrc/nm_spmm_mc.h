@@ -17,11 +17,10 @@ struct McGroupArgs {
   int n;
 };
 
-// nm_spmm_rows: tiles of kRowsTile rows x kRowsTile outputs, fp32 partials of a
-// split's tile.
-constexpr int kRowsTile = 128;
-constexpr int kRowsPartBytes = kRowsTile * kRowsTile * 4;
+// nm_spmm_rows: tiles of kRowsTile or kRowsTallTile rows x kRowsTile outputs,
+// fp32 partials of a split's tile.
+constexpr int kRowsTile = 128, kRowsTallTile = 256;
 
-void launch_rows_product(int dtype, const McGroupArgs& g, int mt, int blocks, hipStream_t st);
+void launch_rows_product(int dtype, const McGroupArgs& g, int bm, int mt, int blocks, hipStream_t st);
 
 }  // namespace nm_hip

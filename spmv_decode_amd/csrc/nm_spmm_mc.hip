@@ -890,14 +890,21 @@ int make_mc_plan(int batch, int h, int w, int nnz, int m, int cfg, int splits, M
   return make_mc_plan(batch, 1, &h, w, nnz, m, cfg, splits, p);
 }
 
-// The plan of nm_spmm_rows: the split count whose rounds of workgroups (one per
-// CU) take the fewest chunk times, a split's handoff counted as 6 + 3 per split
-// (fitted to graph-replay sweeps of 1-6 splits at the Llama-3.1-8B and Qwen3
-// shapes, 129-2048 rows: a chunk takes about 0.5 us, 2 / 4 splits' handoffs 6 / 9). Scratch layout: the products' gathered
-// activations in operand order, then their partial tiles [splits, tiles] when
-// splits > 1.
+// The plan of nm_spmm_rows: the tile height and split count whose rounds of
+// workgroups (one per CU) take the fewest chunk times of a 128-row tile (about
+// 0.75 us). A 256-row tile's chunk takes 1.5 of them for twice the rows. A
+// split's handoff counts 6 + 3 per split, at least 10 per round; of a tall tile,
+// whose partials are twice as large, 17 + 3 per split, at least 19 per round.
+// From graph-replay sweeps of 1-6 splits at the Llama-3.1-8B and Qwen3 shapes,
+// 200-2048 rows (us, 128- / 256-row tiles, each at its best split count): Llama
+// gate and up 200 / 500 / 1024 rows 56 / 46, 105 / 83, 175 / 155; q, k, v 500 / 1024 rows
+// 36 / 39, 59 / 45; down 200 / 500 / 1024 rows 43 / 47, 61 / 63, 97 / 93; Qwen3-14B gate
+// and up 256 / 500 rows 97 / 100, 151 / 135, down 500 rows 94 / 83. Scratch layout: the
+// products' gathered activations in operand order, then their partial tiles
+// [splits, tiles] when splits > 1.
 struct RowsPlan {
-  int mt, splits, rows_per_split, blocks, wp;
+  int bm, mt, splits, rows_per_split, blocks, wp;  // bm rows per tile
+  size_t part_bytes;  // of a split's tile
   size_t xg_bytes, part_off, scratch;
 };
 
@@ -917,30 +924,43 @@ int make_rows_plan(int rows, int n, const int* hs, int w, int nnz, int m, int sp
   const int rbk = ceil_div_mc(rows, 16);
   p->wp = ceil_div_mc(w, kMcCK) * kMcCK;
   if (16LL * rbk * (p->wp / 8) > 0x7fffffffLL) return NM_ERR_BAD_SHAPE;
-  p->mt = ceil_div_mc(rows, kRowsTile);
-  const long long tiles = hsum / kRowsTile * p->mt;
-  if (tiles > kMaxTickets) return NM_ERR_BAD_SHAPE;
+  const int forced = splits & (NM_ROWS_TALL | NM_ROWS_SHORT);
+  splits &= ~forced;
   const int chunks = p->wp / kMcCK;
   double best = 0.0;
+  long long best_tiles = 0;
   p->splits = 0;
-  for (int s = 1; s <= 8; ++s) {
-    if (splits > 0 && s != splits) continue;
-    const int per = ceil_div_mc(chunks, s < chunks ? s : chunks);
-    const int eff = ceil_div_mc(chunks, per);
-    if (splits <= 0 && eff != s) continue;
-    const long long rounds = (tiles * eff + kMcCUs - 1) / kMcCUs;
-    const double cost = (double)rounds * per + (eff > 1 ? 6.0 + 3.0 * eff : 0.0);
-    if (p->splits == 0 || cost < best) {
-      best = cost;
-      p->splits = eff;
-      p->rows_per_split = per * kMcCK;
+  for (int tall = 0; tall < 2; ++tall) {
+    if (forced == (tall ? NM_ROWS_SHORT : NM_ROWS_TALL)) continue;
+    const int bm = tall ? kRowsTallTile : kRowsTile, mt = ceil_div_mc(rows, bm);
+    const long long tiles = hsum / kRowsTile * mt;
+    if (tiles > kMaxTickets) continue;
+    for (int s = 1; s <= 8; ++s) {
+      if (splits > 0 && s != splits) continue;
+      const int per = ceil_div_mc(chunks, s < chunks ? s : chunks);
+      const int eff = ceil_div_mc(chunks, per);
+      if (splits <= 0 && eff != s) continue;
+      const double rounds = (double)((tiles * eff + kMcCUs - 1) / kMcCUs);
+      const double once = (tall ? 17.0 : 6.0) + 3.0 * eff, handoff = (tall ? 19.0 : 10.0) * rounds;
+      const double cost = rounds * per * (tall ? 1.5 : 1.0) + (eff > 1 ? (once > handoff ? once : handoff) : 0.0);
+      if (p->splits == 0 || cost < best) {
+        best = cost;
+        best_tiles = tiles;
+        p->bm = bm;
+        p->mt = mt;
+        p->splits = eff;
+        p->rows_per_split = per * kMcCK;
+      }
     }
   }
-  if (p->splits == 0) return NM_ERR_BAD_CONFIG;
+  if (p->splits == 0)
+    return hsum / kRowsTile * ceil_div_mc(rows, kRowsTile) > kMaxTickets ? NM_ERR_BAD_SHAPE : NM_ERR_BAD_CONFIG;
+  const long long tiles = best_tiles;
+  p->part_bytes = (size_t)p->bm * kRowsTile * 4;
   p->blocks = (int)(tiles * p->splits);
   p->xg_bytes = (size_t)rbk * 16 * (size_t)p->wp * 2;  // a multiple of 2 KB
   p->part_off = (size_t)n * p->xg_bytes;
-  p->scratch = p->part_off + (p->splits > 1 ? (size_t)p->splits * (size_t)tiles * kRowsPartBytes : (size_t)0);
+  p->scratch = p->part_off + (p->splits > 1 ? (size_t)p->splits * (size_t)tiles * p->part_bytes : (size_t)0);
   return NM_OK;
 }
 
@@ -1218,14 +1238,14 @@ int nm_spmm_rows(int dtype, const void* x, const void* up, long long x_row_strid
     g.first[i] = block_off;
     tile_off += tiles;
     block_off += tiles * p.mt * p.splits;
-    part_off += p.splits > 1 ? (size_t)p.splits * (size_t)(tiles * p.mt) * (kRowsPartBytes / 4) : (size_t)0;
+    part_off += p.splits > 1 ? (size_t)p.splits * (size_t)(tiles * p.mt) * (p.part_bytes / 4) : (size_t)0;
   }
   GatherArgs ga = gather_args(x, up, x_row_stride, rows, w, p.wp, nnz, m, K, rbk);
   ga.g = gg;
   launch_gather<true, true>(dtype, ga, n, st);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return (int)e;
-  launch_rows_product(dtype, g, p.mt, p.blocks, st);
+  launch_rows_product(dtype, g, p.bm, p.mt, p.blocks, st);
   e = hipGetLastError();
   return e == hipSuccess ? NM_OK : (int)e;
 }

@@ -261,19 +261,21 @@ def rows_route(rows: int, w: int, hs) -> bool:
     """Whether products of one input past NM_MC_MAX_BATCH rows (16-bit, plan
     left to the library) run on nm_spmm_rows rather than as one BLAS GEMM each:
     from 160 rows (at 129 rows half of its second row tile is padding), several
-    products up to rows * (sum of outputs) = 12.6M, a lone one up to 768 rows
-    when it is deeper than wide (w >= h) and has more than 1024 outputs. The
-    BLAS library runs a GEMM per product, without splitting its depth, and wins
-    on wide outputs, where its 256-wide tiles read less per multiply.
+    products up to rows * (sum of outputs) = 12.6M, and up to 512 rows (two tall
+    row tiles) of up to 36864 outputs; a lone one up to 768 rows when it is
+    deeper than wide (w >= h) and has more than 1024 outputs. The BLAS library
+    runs a GEMM per product, without splitting its depth, and wins on wide
+    outputs of many rows, where its 256-wide tiles read less per multiply.
     Graph replay, gathers included, nm_spmm_rows / library (us): Llama-3.1-8B down
-    200 / 500 / 1024 rows 41 / 57, 55 / 77, 85 / 91; Qwen3-14B down 200 / 500 /
-    1024 rows 50 / 96, 85 / 99, 158 / 142; q/k/v 200 / 500 / 2048 rows 25 / 48, 29
-    / 59, 85 / 102; gate and up 200 / 333 / 500 rows 57 / 65, 76 / 80, 103 / 99; o
-    200 / 500 rows 23 / 20, 26 / 27; Qwen3-14B gate alone 200 rows 61 / 53."""
+    200 / 500 / 1024 rows 43 / 57, 61 / 77, 93 / 107; Qwen3-14B down 200 / 500 /
+    1024 rows 50 / 96, 83 / 99, 158 / 142; q/k/v 200 / 500 / 1024 rows 25 / 48, 29
+    / 59, 45 / 67; Llama-3.1-8B gate and up 200 / 500 / 512 / 1024 rows 46 / 65, 83 / 109,
+    83 / 96, 155 / 139, Qwen3-14B's at 500 rows 135 / 163; o 200 / 500 rows 23 / 20, 26 / 27;
+    Qwen3-32B gate alone 500 / 2048 rows 92 / 77, 298 / 279."""
     if rows < 160 or rows > _lib.NM_ROWS_MAX:
         return False
     if len(hs) > 1:
-        return rows * sum(hs) <= 3 << 22
+        return rows * sum(hs) <= 3 << 22 or (rows <= 512 and sum(hs) <= 9 << 12)
     return rows <= 768 and w >= hs[0] > 1024
 
 

@@ -43,6 +43,27 @@ def test_rows_products(gpu, dtype, shape):
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16], ids=str)
+@pytest.mark.parametrize("shape", SHAPES, ids=str)
+def test_rows_products_tall_tiles(gpu, dtype, shape):
+    """The 256-row tiles at their edges; both tile heights add a split's
+    products in the same order, so their results are the same bits."""
+    K, hs, nnz, m = shape
+    cases = [make_case(K, h, nnz, m, seed=K + 5 * h + i, dtype=dtype) for i, h in enumerate(hs)]
+    mats = [(md, mi) for _, md, mi in cases]
+    w = mats[0][0].shape[0]
+    for rows in (1, 129, 255, 256, 257, 500):
+        X = torch.randn(rows, K, generator=torch.Generator(device="cuda").manual_seed(rows), device="cuda").to(dtype)
+        for splits in (1, 2, 3, 8):
+            say(f"spmm rows tall {dtype} K{K} h{hs} {nnz}:{m} rows {rows} splits {splits}")
+            outs, short = ([torch.full((rows, h), 7.0, dtype=dtype, device="cuda") for h in hs] for _ in range(2))
+            hip_spmv._spmm_rows(X, mats, w, nnz, m, outs, splits=_lib.NM_ROWS_TALL + splits)
+            hip_spmv._spmm_rows(X, mats, w, nnz, m, short, splits=_lib.NM_ROWS_SHORT + splits)
+            for (md, mi), o, f in zip(mats, outs, short):
+                check_rows(o, X, md, mi, nnz, m, f"tall {dtype} {K}x{md.shape[1]} r{rows} s{splits}")
+                assert torch.equal(o, f)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16], ids=str)
 def test_rows_silu_product(gpu, dtype):
     """The product formed in the gather is PyTorch's fp32 one, bit for bit, on
     every path (library GEMM, nm_spmm_rows), so the outputs are those of the
@@ -104,7 +125,8 @@ def test_rows_route_and_arguments(gpu):
     """Routes agree with each other's results (the oracle bar on both sides of
     each line of rows_route), and what nm_spmm_rows refuses is refused."""
     for K, hs, rows, own in ((4096, [4096, 1024, 1024], 159, False), (4096, [4096, 1024, 1024], 160, True),
-                             (4096, [14336, 14336], 438, True), (4096, [14336, 14336], 439, False),
+                             (4096, [14336, 14336], 512, True), (4096, [14336, 14336], 513, False),
+                             (256, [18432, 18432], 512, True), (256, [18560, 18432], 512, False),
                              (14336, [4096], 768, True), (14336, [4096], 769, False), (4096, [1024], 300, False),
                              (4096, [4096], 300, False)):
         assert hip_spmv.rows_route(rows, K // 2, hs) == own

@@ -313,6 +313,10 @@ done:
 // stages, at least three steps in flight: before step k every wave's loads of
 // step k + 1 have landed and its reads of step k - 1, whose stage the loads of
 // step k + 5 then fill, have been multiplied.
+// Graph replay, gathers included, against the 128-row tiles (us): Llama-3.1-8B
+// gate and up at 200 / 500 / 1024 rows 46 / 83 / 155 (56 / 105 / 175), q, k and v at
+// 1024 rows 45 (59); a split deep product of few rows stays with those (down at 200
+// rows 47 against 43).
 constexpr int kTallBM = kRowsTallTile, kTallCK = 32, kTallStages = 6;
 constexpr int kTallW = kTallCK * kBN * 2;                // weights of a stage
 constexpr int kTallStage = kTallW + kTallBM * kTallCK * 2;

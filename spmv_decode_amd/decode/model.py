@@ -180,6 +180,13 @@ def attend_at(at, q: torch.Tensor, k_cache_t: torch.Tensor, v_cache_t: torch.Ten
     return attend(q, k_cache_t, v_cache_t, c, zero)
 
 
+def reads_position(layer: nn.Module) -> bool:
+    """Whether the layer's attention takes the position itself (attend_at on the
+    library's kernel); any other reads the mask rows of the key caches."""
+    at = layer.self_attn if isinstance(layer, Block) else getattr(layer, "attention", None)
+    return getattr(at, "decode_kernel", False)
+
+
 def linear_into(lin: nn.Module, x2d: torch.Tensor, out: torch.Tensor) -> torch.Tensor:
     """y = lin(x) written into `out` ([1, h] contiguous slice): the sparse GEMV's
     `out=` for NmSparseLinear, torch.mm (hipBLASLt) for a dense nn.Linear, the
@@ -769,7 +776,6 @@ class Decoder(nn.Module):
         self.norm = RMSNorm(cfg.dim, cfg.norm_eps)
         self.lm_head = nn.Linear(cfg.dim, cfg.vocab, bias=False)
         self.max_seq = 0
-        self.attention_kernel = False  # setup_cache: the layers' decode_kernel
         self.head_kernel = False  # setup_cache: lm_head in the library's dense GEMV (project_head)
         self.gemv_forms = {}  # (n_out, n_in) -> dense_gemv form, filled by tune_dense_gemv
         self.dense_fusion = "none"  # set_dense_fusion's mode
@@ -903,7 +909,7 @@ class Decoder(nn.Module):
                     and dense_gemv_supported(torch.empty(1, c.dim, device=self.q_pad.device, dtype=dtype),
                                              self.lm_head.weight))
             kernel = attention_supported(self.q_pad, self.k_cache_t[0], self.v_cache_t[0], hd)
-        self.attention_kernel, self.head_kernel = kernel, head
+        self.head_kernel = head
         for blk in self.layers:
             (blk.self_attn if isinstance(blk, Block) else blk.attention).decode_kernel = kernel
         self._carry = None
@@ -1016,7 +1022,7 @@ class Decoder(nn.Module):
         """One decode step: token [1, 1] int64 and pos [1] int64 on the device
         -> logits [1, vocab]. No host synchronisation."""
         x = self.embed_tokens(token)  # [1, 1, dim]
-        if not self.attention_kernel:
+        if not all(reads_position(b) for b in self.layers):  # one put in place since setup_cache does not
             # causal mask of this step in every layer's key cache: 0 up to pos, -inf after
             keep = (self.positions <= pos).expand_as(self.k_mask)
             if torch.compiler.is_compiling():  # the tracer takes no strided out=; the compiler fuses the copy

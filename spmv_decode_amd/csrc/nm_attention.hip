@@ -34,6 +34,7 @@
 //    sums in the workspace; the last to arrive at the head (the GEMV's split-K
 //    handoff: agent-scope atomics, no fence) merges them in split order. The
 //    result does not depend on the arrival order.
+#include <float.h>
 #include <math.h>
 
 #include "nm_mfma.h"
@@ -68,6 +69,11 @@ __device__ inline float row16(float v, F f) {  // f over the 16 lanes of a row, 
 }
 // A maximum that keeps NaN (a NaN score makes its whole row NaN, as softmax does).
 __device__ inline float max_nan(float a, float b) { return a > b || a != a ? a : b; }
+// What the scores of a split or block are taken relative to: its maximum m, and
+// a finite number where every score is -inf. Their probabilities are then 0
+// (exp2(-inf - -inf) is NaN), so other positions keep their softmax; a row of
+// nothing but -inf ends as 0 / 0.
+__device__ inline float exp_base(float m) { return fmaxf(m, -FLT_MAX); }
 
 template <int DT, int HD, int NPB>
 __global__ __launch_bounds__(kBlock) void nm_attention_kernel(AttnArgs a) {
@@ -190,9 +196,10 @@ __global__ __launch_bounds__(kBlock) void nm_attention_kernel(AttnArgs a) {
     auto at = [&](int w) { return j == 0 ? wm[w].x : (j == 1 ? wm[w].y : (j == 2 ? wm[w].z : wm[w].w)); };
     rowmax[j] = max_nan(max_nan(at(0), at(1)), max_nan(at(2), at(3)));
     rowsum[j] = 0.0f;
+    const float base = exp_base(rowmax[j]);
 #pragma unroll
     for (int b = 0; b < NPB; ++b) {
-      const float p = __builtin_amdgcn_exp2f(sc[b][j] - rowmax[j]);
+      const float p = __builtin_amdgcn_exp2f(sc[b][j] - base);
       rowsum[j] += p;
       ps[(4 * lg + j) * PSTR + 16 * (wave * NPB + b) + li] = E::from_f32(p);
     }
@@ -611,12 +618,13 @@ __global__ __launch_bounds__(kBlock) void nm_attention_prefill_kernel(PrefillArg
     for (int j = 0; j < 4; ++j) {
       float mx = max_nan(max_nan(sc[0][j], sc[1][j]), max_nan(sc[2][j], sc[3][j]));
       mx = max_nan(m[j], row16(mx, [](float x, float y) { return max_nan(x, y); }));
-      alpha[j] = __builtin_amdgcn_exp2f(m[j] - mx);  // 0 at the first block
+      const float base = exp_base(mx);
+      alpha[j] = __builtin_amdgcn_exp2f(m[j] - base);  // 0 at the first block
       m[j] = mx;
       float s = 0.0f;
 #pragma unroll
       for (int b = 0; b < 4; ++b) {
-        const float p = __builtin_amdgcn_exp2f(sc[b][j] - mx);
+        const float p = __builtin_amdgcn_exp2f(sc[b][j] - base);
         s += p;
         ps[wave][(4 * lg + j) * PSTR + 16 * b + li] = E::from_f32(p);
       }

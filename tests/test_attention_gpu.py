@@ -118,3 +118,43 @@ def test_prompt_attention_matches_exact(gpu, case, dtype):
                     .contiguous()).transpose(0, 1).reshape(P, nh * hd)
     rel = float((y.double() - ref).norm() / ref.norm())
     assert rel <= 2 * eps, rel
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16], ids=str)
+def test_attention_decode_over_splits_of_infinite_scores(gpu, dtype):
+    """Whole splits whose every score is -inf weigh nothing and leave the rest
+    its softmax; a row of nothing else is NaN, as a softmax of it is."""
+    hd, S = 128, 640
+    q, k, v = case(8, 2, hd, S, dtype, 0, seed=5)
+    q[:, 0] = 1
+    k[0, 0, :256] = -math.inf
+    bar = 2 * torch.finfo(dtype).eps
+    for span in (0, 64, 128, 256):
+        for pos in (256, 300, 511, 639):
+            y = hip_spmv.nmsparse_attention_decode(q, k, v, torch.tensor([pos], device="cuda"), hd, span=span)
+            ref = exact(q, k, v, hd, pos + 1)
+            assert float((y.double() - ref).norm() / ref.norm()) <= bar, (span, pos)
+        for pos in (63, 255):
+            y = hip_spmv.nmsparse_attention_decode(q, k, v, torch.tensor([pos], device="cuda"), hd, span=span)
+            assert torch.isnan(y[0, :4 * hd]).all() and torch.isfinite(y[0, 4 * hd:]).all(), (span, pos)
+
+
+def test_prompt_attention_over_blocks_of_infinite_scores(gpu):
+    """The same of a row's leading blocks in a prompt: in bf16, scores of
+    -1e60 are -inf in fp32."""
+    P, nh, kvh, hd, S, first = 200, 4, 2, 128, 256, 70
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    q, k, v = (torch.randn(P, h * hd, device="cuda", generator=gen).bfloat16() for h in (nh, kvh, kvh))
+    q[:, ::hd], k[:, ::hd] = 1e30, 0
+    k[:first, ::hd] = -1e30
+    table = torch.zeros(S, hd // 2, 2, device="cuda")
+    table[..., 0] = 1  # no rotation
+    kc, vc = (torch.zeros(kvh, hd, S, device="cuda").bfloat16() for _ in range(2))
+    y = hip_spmv.nmsparse_prefill_attention(q, k, v, kc, vc, table, hd).view(P, nh, hd)
+    qd, kd, vd = (t.double().view(P, -1, hd).transpose(0, 1).contiguous() for t in (q, k, v))
+    kd, vd = kd.repeat_interleave(nh // kvh, 0), vd.repeat_interleave(nh // kvh, 0)
+    s = torch.bmm(qd, kd.transpose(1, 2).contiguous()) / math.sqrt(hd)
+    s = s.masked_fill(torch.ones(P, P, dtype=torch.bool, device="cuda").triu(1), -math.inf)
+    ref = torch.bmm(torch.softmax(s, -1), vd).transpose(0, 1)[first:]
+    assert float((y[first:].double() - ref).norm() / ref.norm()) <= 2 * torch.finfo(torch.bfloat16).eps
+    assert torch.isnan(y[:first]).all()

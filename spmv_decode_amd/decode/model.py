@@ -258,11 +258,20 @@ def project_head(lin: nn.Module, x: torch.Tensor, kernel: bool) -> torch.Tensor:
     return project(lin, x).view(1, -1)
 
 
+def plain_norm(norm: nn.Module) -> bool:
+    """Whether calling this module is an RMSNorm of its weight and eps and
+    nothing else: no other class or forward, no hooks."""
+    hooks = nn.modules.module
+    return (type(norm) is RMSNorm and "forward" not in vars(norm)
+            and not (norm._forward_hooks or norm._forward_pre_hooks or hooks._global_forward_hooks
+                     or hooks._global_forward_pre_hooks))
+
+
 def add_norm(norm: nn.Module, x: torch.Tensor, d: torch.Tensor) -> tuple:
     """(x + d, norm(x + d)) for the rows x, d [rows, dim] of a prompt: one
     launch of the library where it takes them (500 rows of 4096: 3.7 us where the
-    two calls take 8.8), the two calls elsewhere and for a norm that is not an RMSNorm or has hooks."""
-    if type(norm) is RMSNorm and x.is_cuda and not (norm._forward_hooks or norm._forward_pre_hooks):
+    two calls take 8.8), the two calls elsewhere and for a norm that is more than its arithmetic (plain_norm)."""
+    if plain_norm(norm) and x.is_cuda:
         from ..hip_spmv import add_rms_norm_supported, nmsparse_add_rms_norm
 
         if add_rms_norm_supported(x, d, norm.weight) and not records_grad(x, d, norm.weight):
@@ -340,20 +349,21 @@ def prompt_attention(at, q, k, v, freqs, rope, k_cache_t, v_cache_t) -> torch.Te
     [P, kv] (at: the attention module): head norms, rotary embedding (freqs
     complex64 [P, 1, head_dim / 2] or the same as the fp32 table rope), keys and
     values into the caches at positions 0 .. P-1, causal attention. Where the
-    layer decodes on the library's attention kernel (attend_at) and these
-    operands are within its forms, the library's two prompt launches. Returns
-    [P, q]."""
+    layer decodes on the library's attention kernel (attend_at), these operands
+    are within its forms and the head norms are plain ones of one eps, the
+    library's two prompt launches. Returns [P, q]."""
     c = at.cfg
     hd, P = c.head_dim, q.shape[0]
     rows = at.decode_kernel and all(t.stride(1) == 1 and t.stride(0) % 8 == 0 and t.data_ptr() % 16 == 0
                                     and t.dtype == k_cache_t.dtype for t in (q, k, v))
-    norms = (at.q_norm.weight, at.k_norm.weight) if c.qk_norm else ()
-    if rows and all(t.dtype == q.dtype and t.is_contiguous() for t in norms):
+    norms = (at.q_norm, at.k_norm) if c.qk_norm else ()
+    if rows and all(plain_norm(n) and n.weight.dtype == q.dtype and n.weight.is_contiguous() and n.eps == norms[0].eps
+                    for n in norms):
         from ..hip_spmv import nmsparse_prefill_attention
 
+        weights = dict(zip(("q_norm", "k_norm"), (n.weight for n in norms)))
         return nmsparse_prefill_attention(q, k, v, k_cache_t, v_cache_t, rope, hd,
-                                          q_norm=at.q_norm.weight if c.qk_norm else None,
-                                          k_norm=at.k_norm.weight if c.qk_norm else None, norm_eps=c.norm_eps)
+                                          norm_eps=norms[0].eps if norms else 0.0, **weights)
     q, k, v = q.reshape(P, c.n_heads, hd), k.reshape(P, c.n_kv_heads, hd), v.reshape(P, c.n_kv_heads, hd)
     if c.qk_norm:
         q, k = at.q_norm(q), at.k_norm(k)

@@ -259,10 +259,10 @@ def project_head(lin: nn.Module, x: torch.Tensor, kernel: bool) -> torch.Tensor:
 
 
 def plain_norm(norm: nn.Module) -> bool:
-    """Whether calling this module is an RMSNorm of its weight and eps and
-    nothing else: no other class or forward, no hooks."""
+    """Whether calling this module is an RMSNorm of its weight and a given eps
+    (None: PyTorch's own choice) and nothing else: no other class or forward, no hooks."""
     hooks = nn.modules.module
-    return (type(norm) is RMSNorm and "forward" not in vars(norm)
+    return (type(norm) is RMSNorm and norm.eps is not None and norm.eps >= 0 and "forward" not in vars(norm)
             and not (norm._forward_hooks or norm._forward_pre_hooks or hooks._global_forward_hooks
                      or hooks._global_forward_pre_hooks))
 

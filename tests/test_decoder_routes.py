@@ -72,6 +72,20 @@ def test_changed_head_norms_in_a_prompt(gpu, change):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("eps", [None, -1e-6])
+def test_prompt_norms_of_an_eps_the_kernels_do_not_take(gpu, eps):
+    model = decoder(qk_norm=True)
+    model.setup_cache(128, torch.device("cuda"))
+    for m in model.modules():
+        if isinstance(m, RMSNorm):
+            m.eps = eps
+    got = model.prefill(prompt())
+    for blk in model.layers:
+        blk.self_attn.decode_kernel = False
+    close(got, model.prefill(prompt()))
+
+
+@pytest.mark.gpu
 def test_a_layer_put_in_place_after_the_caches_attends_causally(gpu):
     """Its attention reads the mask rows, which the step then has to write."""
     model = decoder()

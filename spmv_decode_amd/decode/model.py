@@ -169,22 +169,27 @@ def attend_at(at, q: torch.Tensor, k_cache_t: torch.Tensor, v_cache_t: torch.Ten
               pos: torch.Tensor) -> torch.Tensor:
     """attend over the positions <= pos (at: the attention module). Where
     Decoder.setup_cache found the caches within the library's attention kernel
-    (at.decode_kernel) one launch reads the position on the device and the
+    (at.decode_kernel; not in forward mode: on_kernel) one launch reads the position on the device and the
     cached positions up to it; the mask row and q's columns past head_dim are
     not read then. Otherwise attend (q the padded query buffer, the mask row
     written for pos)."""
     c = at.cfg
-    if at.decode_kernel:
+    if on_kernel(at):
         y = torch.ops.nmsparse.attention_decode(q, k_cache_t, v_cache_t, pos, c.head_dim)
         return y.view(c.n_kv_heads, c.n_heads // c.n_kv_heads, c.head_dim)
     return attend(q, k_cache_t, v_cache_t, c, zero)
+
+
+def on_kernel(at) -> bool:
+    """Whether this attention module runs on the library's kernels."""
+    return at.decode_kernel and not forward_mode()
 
 
 def reads_position(layer: nn.Module) -> bool:
     """Whether the layer's attention takes the position itself (attend_at on the
     library's kernel); any other reads the mask rows of the key caches."""
     at = layer.self_attn if isinstance(layer, Block) else getattr(layer, "attention", None)
-    return getattr(at, "decode_kernel", False)
+    return hasattr(at, "decode_kernel") and on_kernel(at)
 
 
 def linear_into(lin: nn.Module, x2d: torch.Tensor, out: torch.Tensor) -> torch.Tensor:
@@ -239,17 +244,24 @@ def project(lin: nn.Module, x: torch.Tensor) -> torch.Tensor:
     return lin(x)
 
 
-def records_grad(*tensors) -> bool:
-    """Whether autograd records what is computed from these tensors."""
-    return torch.is_grad_enabled() and any(t.requires_grad for t in tensors)
+def forward_mode() -> bool:
+    """Whether a forward-mode level is open: tangents may then ride on any
+    operand, and the library's launches would drop them."""
+    return not torch.compiler.is_compiling() and torch.autograd.forward_ad._current_level >= 0
+
+
+def differentiated(*tensors) -> bool:
+    """Whether autograd follows what is computed from these tensors, in
+    reverse or in forward mode."""
+    return forward_mode() or (torch.is_grad_enabled() and any(t.requires_grad for t in tensors))
 
 
 def project_head(lin: nn.Module, x: torch.Tensor, kernel: bool) -> torch.Tensor:
     """The output head on one row x [..., dim] -> [1, vocab]: in the library's
     dense GEMV when `kernel` (Decoder.setup_cache found it to take the weight)
-    and it takes these operands, else, and where autograd records, project."""
+    and it takes these operands, else, and where autograd follows, project."""
     if (kernel and type(lin) is nn.Linear and lin.bias is None and lin.weight.dtype == x.dtype
-            and not records_grad(x, lin.weight)):
+            and not differentiated(x, lin.weight)):
         from ..hip_spmv import dense_gemv_supported
 
         row = x.reshape(1, -1)
@@ -274,7 +286,7 @@ def add_norm(norm: nn.Module, x: torch.Tensor, d: torch.Tensor) -> tuple:
     if plain_norm(norm) and x.is_cuda:
         from ..hip_spmv import add_rms_norm_supported, nmsparse_add_rms_norm
 
-        if add_rms_norm_supported(x, d, norm.weight) and not records_grad(x, d, norm.weight):
+        if add_rms_norm_supported(x, d, norm.weight) and not differentiated(x, d, norm.weight):
             return nmsparse_add_rms_norm(x, d, norm.weight, norm.eps)
     x = x + d
     return x, norm(x)
@@ -354,7 +366,7 @@ def prompt_attention(at, q, k, v, freqs, rope, k_cache_t, v_cache_t) -> torch.Te
     library's two prompt launches. Returns [P, q]."""
     c = at.cfg
     hd, P = c.head_dim, q.shape[0]
-    rows = at.decode_kernel and all(t.stride(1) == 1 and t.stride(0) % 8 == 0 and t.data_ptr() % 16 == 0
+    rows = on_kernel(at) and all(t.stride(1) == 1 and t.stride(0) % 8 == 0 and t.data_ptr() % 16 == 0
                                     and t.dtype == k_cache_t.dtype for t in (q, k, v))
     norms = (at.q_norm, at.k_norm) if c.qk_norm else ()
     if rows and all(plain_norm(n) and n.weight.dtype == q.dtype and n.weight.is_contiguous() and n.eps == norms[0].eps
@@ -461,7 +473,7 @@ def attention_core(at, qkv, freqs, k_cache_t, v_cache_t, pos, q_pad, zero):
     qk = rotate(qk, freqs)
     q, k = qk[:c.n_heads], qk[c.n_heads:]
     v = qkv[0, qd + kvd:].view(c.n_kv_heads, c.head_dim, 1)
-    if not at.decode_kernel:
+    if not on_kernel(at):
         q_pad[:, :c.head_dim].copy_(q)
         q = q_pad
     if torch.compiler.is_compiling():

@@ -5,6 +5,7 @@ import copy
 
 import pytest
 import torch
+import torch.autograd.forward_ad as fw
 
 from spmv_decode_amd.decode.model import Decoder, RMSNorm, tiny_config
 
@@ -97,3 +98,51 @@ def test_a_layer_put_in_place_after_the_caches_attends_causally(gpu):
     model.layers[1] = layer
     model.reset_cache()
     close(steps(model, ids), ref)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("call", ["step", "prefill"])
+def test_forward_mode_tangents_of_the_head(gpu, call):
+    """Logits are linear in the head's weight: its tangent 2 W gives 2 logits."""
+    model = decoder()
+    model.setup_cache(128, torch.device("cuda"))
+    token, pos = torch.tensor([[3]], device="cuda"), torch.tensor([0], device="cuda")
+
+    def run():
+        with torch.no_grad():
+            return model.forward_step(token, pos) if call == "step" else model.prefill(token.view(-1))
+
+    plain, w = run(), model.lm_head.weight
+    with fw.dual_level():
+        del model.lm_head._parameters["weight"]
+        model.lm_head.weight = fw.make_dual(w.detach().clone(), 2 * w.detach())
+        tangent = fw.unpack_dual(run()).tangent
+    assert tangent is not None
+    close(tangent, 2 * plain)
+
+
+@pytest.mark.gpu
+def test_forward_mode_tangents_of_the_values(gpu):
+    """The attention of a step is linear in its values, here those of a full
+    cache's last position: their tangents 2 V give 2 y."""
+    from spmv_decode_amd.decode.model import attention_core
+
+    model = decoder(qk_norm=False)
+    model.setup_cache(128, torch.device("cuda"))
+    at, c = model.layers[0].self_attn, model.cfg
+    qd, kvd = c.n_heads * c.head_dim, c.n_kv_heads * c.head_dim
+    qkv = torch.randn(1, qd + 2 * kvd, device="cuda", generator=torch.Generator(device="cuda").manual_seed(2)).half()
+    pos = torch.tensor([127], device="cuda")  # every slot attended to: a mask row of zeros
+
+    def run(qkv):
+        with torch.no_grad():
+            return attention_core(at, qkv, model.rope.index_select(0, pos), model.k_cache_t[0].clone(),
+                                  model.v_cache_t[0].clone(), pos, model.q_pad.clone(), model.zero)
+
+    plain = run(qkv)
+    seed = torch.zeros_like(qkv)
+    seed[:, qd + kvd:] = 2 * qkv[:, qd + kvd:]
+    with fw.dual_level():
+        tangent = fw.unpack_dual(run(fw.make_dual(qkv, seed))).tangent
+    assert tangent is not None
+    close(tangent, 2 * plain)

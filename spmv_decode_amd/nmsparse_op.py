@@ -59,9 +59,10 @@ import torch
 
 from typing import Optional
 
-from .hip_spmv import (GemvProblem, nmsparse_attention_decode, nmsparse_dense_gemv, nmsparse_gate_up_accumulate,
-                       nmsparse_gate_up_silu, nmsparse_gemv_accumulate, nmsparse_gemv_grouped, nmsparse_gemv_launch, nmsparse_gemv_partials,
-                       nmsparse_gemv_silu, nmsparse_qkv_decode, nmsparse_spmm_forward_hip, nmsparse_spmv_forward_hip)
+from .hip_spmv import (GemvProblem, dense_gemv_supported, nmsparse_attention_decode, nmsparse_dense_gemv,
+                       nmsparse_gate_up_accumulate, nmsparse_gate_up_silu, nmsparse_gemv_accumulate,
+                       nmsparse_gemv_grouped, nmsparse_gemv_launch, nmsparse_gemv_partials, nmsparse_gemv_silu,
+                       nmsparse_qkv_decode, nmsparse_spmm_forward_hip, nmsparse_spmv_forward_hip)
 
 _kernel = os.environ.get("NM_KERNEL", "")
 if _kernel not in ("", "hip", "triton_ptx", "guarded", "fp16", "fp16_split"):
@@ -383,8 +384,11 @@ def _(q, k_cache_t, v_cache_t, pos, head_dim):
 @torch.library.custom_op("nmsparse::dense_gemv", mutates_args=())
 def dense_gemv(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
     """A dense weight [n, K] applied to one row x [..., K] -> [1, n]
-    (hip_spmv.nmsparse_dense_gemv)."""
-    return nmsparse_dense_gemv(x, weight)
+    (hip_spmv.nmsparse_dense_gemv; the BLAS product for a weight that it does
+    not take, which a compiled step may meet: it was traced before)."""
+    if dense_gemv_supported(x, weight):
+        return nmsparse_dense_gemv(x, weight)
+    return torch.mm(x.reshape(1, -1), weight.t())
 
 
 @dense_gemv.register_fake

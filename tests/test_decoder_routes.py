@@ -146,3 +146,27 @@ def test_forward_mode_tangents_of_the_values(gpu):
         tangent = fw.unpack_dual(run(fw.make_dual(qkv, seed))).tangent
     assert tangent is not None
     close(tangent, 2 * plain)
+
+
+@pytest.mark.parametrize("device", ["cpu", pytest.param("cuda", marks=pytest.mark.gpu)])
+@pytest.mark.parametrize("form", ["transposed", "shifted"])
+def test_compiled_step_with_a_head_the_kernel_does_not_take(request, device, form):
+    """A head weight of other strides or alignment than setup_cache saw: a
+    compiled step, which checks nothing when traced, multiplies it all the same."""
+    if device == "cuda":
+        request.getfixturevalue("gpu")
+    model = decoder(device, torch.float32 if device == "cpu" else torch.float16)
+    model.setup_cache(128, torch.device(device), model.lm_head.weight.dtype)
+    assert model.head_kernel == (device == "cuda")
+    model.head_kernel = True
+    w = model.lm_head.weight
+    if form == "transposed":
+        w.data = w.data.t().contiguous().t()
+    else:
+        buf = torch.empty(w.numel() + 1, device=device, dtype=w.dtype)[1:].view_as(w)
+        w.data = buf.copy_(w.data)
+    token, pos = torch.tensor([[3]], device=device), torch.tensor([0], device=device)
+    with torch.no_grad():
+        ref = model.forward_step(token, pos)
+        got = torch.compile(model.forward_step, backend="eager", fullgraph=True)(token, pos)
+    close(got, ref)

@@ -484,6 +484,8 @@ def nmsparse_spmm_group_hip(x, mats, BLOCK_WIDTH, VEC_WIDTH, *, outs=None, confi
     mats = list(mats)
     if not mats:
         return []
+    if x.ndim < 2:
+        raise ValueError(f"x must be [..., rows, K], got {tuple(x.shape)}")
     K = x.shape[-1]
     lead = x.shape[:-1]
     rows = x.reshape(-1, K).shape[0]

@@ -57,3 +57,14 @@ def test_silu_mul_is_the_fp32_product(gpu, dtype):
     assert lib.nm_silu_mul(code, gate.data_ptr(), up.data_ptr(), out.data_ptr(), 12, None) == -2
     assert lib.nm_silu_mul(code, gate.data_ptr() + 2, up.data_ptr(), out.data_ptr(), 8, None) == -5
     assert lib.nm_silu_mul(2, gate.data_ptr(), up.data_ptr(), out.data_ptr(), 8, None) == -7
+
+
+def test_group_refuses_a_vector(gpu):
+    """Rows are [..., rows, K], as for one product."""
+    mats = [make_case(128, 128, 2, 4, seed=i)[1:] for i in range(2)]
+    x = torch.randn(128, device="cuda").half()
+    with pytest.raises(ValueError):
+        hip_spmv.nmsparse_spmm_forward_hip(x, *mats[0], 64, 128, 2, 4)
+    for n in (1, 2):
+        with pytest.raises(ValueError):
+            hip_spmv.nmsparse_spmm_group_hip(x, mats[:n], 2, 4)

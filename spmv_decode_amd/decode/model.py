@@ -932,8 +932,9 @@ class Decoder(nn.Module):
                                              self.lm_head.weight))
             kernel = attention_supported(self.q_pad, self.k_cache_t[0], self.v_cache_t[0], hd)
         self.head_kernel = head
-        for blk in self.layers:
-            (blk.self_attn if isinstance(blk, Block) else blk.attention).decode_kernel = kernel
+        for at in self.layers.modules():  # those inside a layer's wrapper as well
+            if isinstance(at, (Attention, GptFastAttention)):
+                at.decode_kernel = kernel
         self._carry = None
         self.prepare_decode()
 

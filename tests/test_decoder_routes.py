@@ -170,3 +170,28 @@ def test_compiled_step_with_a_head_the_kernel_does_not_take(request, device, for
         ref = model.forward_step(token, pos)
         got = torch.compile(model.forward_step, backend="eager", fullgraph=True)(token, pos)
     close(got, ref)
+
+
+class Wrapped(torch.nn.Module):
+    def __init__(self, layer):
+        super().__init__()
+        self.layer = layer
+
+    def forward(self, *args):
+        return self.layer(*args)
+
+
+@pytest.mark.parametrize("device", ["cpu", pytest.param("cuda", marks=pytest.mark.gpu)])
+@pytest.mark.parametrize("wrap", [Wrapped, lambda layer: torch.compile(layer, backend="eager")],
+                         ids=["module", "compiled"])
+def test_wrapped_layers_take_caches(request, device, wrap):
+    if device == "cuda":
+        request.getfixturevalue("gpu")
+    dtype = torch.float32 if device == "cpu" else torch.float16
+    model = decoder(device, dtype)
+    model.setup_cache(128, torch.device(device), dtype)
+    ids = torch.arange(9, device=device)
+    ref = steps(model, ids, device)
+    model.layers[0] = wrap(model.layers[0])
+    model.setup_cache(128, torch.device(device), dtype)
+    close(steps(model, ids, device), ref)

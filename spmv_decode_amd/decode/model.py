@@ -933,8 +933,8 @@ class Decoder(nn.Module):
             kernel = attention_supported(self.q_pad, self.k_cache_t[0], self.v_cache_t[0], hd)
         self.head_kernel = head
         for at in self.layers.modules():  # those inside a layer's wrapper as well
-            if isinstance(at, (Attention, GptFastAttention)):
-                at.decode_kernel = kernel
+            if isinstance(at, (Attention, GptFastAttention)):  # a class of its own may read the mask rows
+                at.decode_kernel = kernel and type(at) in (Attention, GptFastAttention)
         self._carry = None
         self.prepare_decode()
 

@@ -7,7 +7,7 @@ import pytest
 import torch
 import torch.autograd.forward_ad as fw
 
-from spmv_decode_amd.decode.model import Decoder, RMSNorm, tiny_config
+from spmv_decode_amd.decode.model import Attention, Decoder, RMSNorm, attend, rotate, tiny_config
 
 # two fp16 paths of a few layers: rounding in another order, each below 2^-11 of its value, over about 40 roundings
 REL = 2e-2
@@ -195,3 +195,26 @@ def test_wrapped_layers_take_caches(request, device, wrap):
     model.layers[0] = wrap(model.layers[0])
     model.setup_cache(128, torch.device(device), dtype)
     close(steps(model, ids, device), ref)
+
+
+class MaskReader(Attention):
+    """Attention written for the caches' documented layout, mask row included."""
+
+    def forward(self, x, freqs, k_cache_t, v_cache_t, pos, q_pad, zero):
+        c = self.cfg
+        q, k, v = (p(x).view(-1, c.head_dim) for p in (self.q_proj, self.k_proj, self.v_proj))
+        q_pad[:, :c.head_dim] = rotate(q, freqs)
+        k_cache_t[:, :c.head_dim].index_copy_(2, pos, rotate(k, freqs).unsqueeze(-1))
+        v_cache_t.index_copy_(2, pos, v.unsqueeze(-1))
+        return self.o_proj(attend(q_pad, k_cache_t, v_cache_t, c, zero).view(1, 1, -1))
+
+
+@pytest.mark.gpu
+def test_an_attention_class_of_its_own_finds_the_mask_rows_written(gpu):
+    model = decoder()
+    model.setup_cache(128, torch.device("cuda"))
+    ref = steps(model, prompt())
+    for blk in model.layers:
+        blk.self_attn.__class__ = MaskReader
+    model.setup_cache(128, torch.device("cuda"))
+    close(steps(model, prompt()), ref)

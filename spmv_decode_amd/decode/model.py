@@ -930,7 +930,7 @@ class Decoder(nn.Module):
             head = (type(self.lm_head) is nn.Linear and self.lm_head.bias is None
                     and dense_gemv_supported(torch.empty(1, c.dim, device=self.q_pad.device, dtype=dtype),
                                              self.lm_head.weight))
-            kernel = attention_supported(self.q_pad, self.k_cache_t[0], self.v_cache_t[0], hd)
+            kernel = c.n_layers > 0 and attention_supported(self.q_pad, self.k_cache_t[0], self.v_cache_t[0], hd)
         self.head_kernel = head
         for at in self.layers.modules():  # those inside a layer's wrapper as well
             if isinstance(at, (Attention, GptFastAttention)):  # a class of its own may read the mask rows

@@ -218,3 +218,15 @@ def test_an_attention_class_of_its_own_finds_the_mask_rows_written(gpu):
         blk.self_attn.__class__ = MaskReader
     model.setup_cache(128, torch.device("cuda"))
     close(steps(model, prompt()), ref)
+
+
+@pytest.mark.gpu
+def test_a_decoder_without_layers(gpu):
+    model = decoder(n_layers=0)
+    model.setup_cache(128, torch.device("cuda"))
+    token = torch.tensor([[3]], device="cuda")
+    with torch.no_grad():
+        y = model.forward_step(token, torch.tensor([0], device="cuda"))
+        ref = model.norm(model.embed_tokens(token)).double().view(1, -1) @ model.lm_head.weight.double().t()
+    close(y, ref, 2.0 ** -10)  # one rounding
+    close(model.prefill(token.view(-1)), ref, 2.0 ** -10)

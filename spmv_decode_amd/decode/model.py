@@ -283,7 +283,7 @@ def add_norm(norm: nn.Module, x: torch.Tensor, d: torch.Tensor) -> tuple:
     """(x + d, norm(x + d)) for the rows x, d [rows, dim] of a prompt: one
     launch of the library where it takes them (500 rows of 4096: 3.7 us where the
     two calls take 8.8), the two calls elsewhere and for a norm that is more than its arithmetic (plain_norm)."""
-    if plain_norm(norm) and x.is_cuda:
+    if plain_norm(norm) and x.is_cuda and not torch.compiler.is_compiling():  # no op of its own to trace
         from ..hip_spmv import add_rms_norm_supported, nmsparse_add_rms_norm
 
         if add_rms_norm_supported(x, d, norm.weight) and not differentiated(x, d, norm.weight):
@@ -366,8 +366,9 @@ def prompt_attention(at, q, k, v, freqs, rope, k_cache_t, v_cache_t) -> torch.Te
     library's two prompt launches. Returns [P, q]."""
     c = at.cfg
     hd, P = c.head_dim, q.shape[0]
-    rows = on_kernel(at) and all(t.stride(1) == 1 and t.stride(0) % 8 == 0 and t.data_ptr() % 16 == 0
-                                    and t.dtype == k_cache_t.dtype for t in (q, k, v))
+    rows = (on_kernel(at) and not torch.compiler.is_compiling()
+            and all(t.stride(1) == 1 and t.stride(0) % 8 == 0 and t.data_ptr() % 16 == 0
+                    and t.dtype == k_cache_t.dtype for t in (q, k, v)))
     norms = (at.q_norm, at.k_norm) if c.qk_norm else ()
     if rows and all(plain_norm(n) and n.weight.dtype == q.dtype and n.weight.is_contiguous() and n.eps == norms[0].eps
                     for n in norms):

@@ -230,3 +230,13 @@ def test_a_decoder_without_layers(gpu):
         ref = model.norm(model.embed_tokens(token)).double().view(1, -1) @ model.lm_head.weight.double().t()
     close(y, ref, 2.0 ** -10)  # one rounding
     close(model.prefill(token.view(-1)), ref, 2.0 ** -10)
+
+
+@pytest.mark.gpu
+def test_a_dense_prompt_compiles_whole(gpu):
+    model = decoder(qk_norm=True)
+    model.setup_cache(128, torch.device("cuda"))
+    ref, keys = model.prefill(prompt()), model.k_store.clone()
+    got = torch.compile(model.prefill, backend="eager", fullgraph=True)(prompt())
+    close(got, ref)
+    close(model.k_store[:, :, :64, :9], keys[:, :, :64, :9])

@@ -575,15 +575,24 @@ __global__ __launch_bounds__(kBlock) void nm_gather_mc_kernel(GatherArgs a) {
   }
   const bool row_ok = b < a.batch;
   const long long row = (long long)(row_ok ? b : 0) * a.x_row_stride;
-  uint16_t v[8];
+  // All loads, then all products: formed only where they are wanted, each
+  // product was a branch with its own wait (a call of 16 rows, 3072 -> 1024, with
+  // the SiLU product: 11.5 us against 11.05).
+  uint16_t t[8], u[8], v[8];
+  bool ok[8];
 #pragma unroll
   for (int e = 0; e < 8; ++e) {
     const int c = c0 + e;
     const int cc = c < a.w ? c : a.w - 1;  // clamped: the load stays in range
     const int p = (cc / a.nnz) * a.m + (int)mat_index[cc];
-    const uint16_t t = a.x[row + (p < a.K ? p : 0)];
-    const uint16_t u = SDT >= 0 ? a.x2[row + (p < a.K ? p : 0)] : (uint16_t)0;
-    v[e] = (row_ok && c < a.w && p < a.K) ? gathered<SDT, IEEE>(t, u) : (uint16_t)0;
+    t[e] = a.x[row + (p < a.K ? p : 0)];
+    u[e] = SDT >= 0 ? a.x2[row + (p < a.K ? p : 0)] : (uint16_t)0;
+    ok[e] = row_ok && c < a.w && p < a.K;
+  }
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const uint16_t y = gathered<SDT, IEEE>(t[e], u[e]);
+    v[e] = ok[e] ? y : (uint16_t)0;
   }
   *reinterpret_cast<u32x4*>(a.g.xg[blockIdx.z] + (FRAG ? (long long)i * 8 : (long long)b * a.wp + c0)) = pack8(v);
 }

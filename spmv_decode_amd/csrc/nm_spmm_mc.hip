@@ -54,14 +54,18 @@ static_assert(NM_MC_MAX_BATCH == 128, "batch tiles of 16, 32, 64 and 128 rows");
 // up to 8% slower, two stages up to 30%). At most 65 KB of LDS per
 // workgroup.
 constexpr int mc_stages(int ht) { return ht == 64 ? 4 : 3; }
-// Lanes per workgroup: 4 wave64, 8 for the DMA tiles that give each a
-// 16-column block. The ring's reads and multiplies run back to back within a
-// wave (each read block ends with its wait), so with one wave per SIMD every
-// LDS round trip was exposed; a second wave multiplies meanwhile. Calls with
-// the gather, 4 -> 8 waves (graph replay): gate/up 4096 -> 2 x 14336 at 128 rows
-// 37.8 -> 35.0 us, 5120 -> 2 x 17408 at 33 / 128 rows 50.1 -> 45.9 / 79.1 -> 68.9,
-// down 17408 -> 5120 30.8 -> 28.5 at 33; up to 16 rows level (the weight stream).
-constexpr int mc_block(int bt, int ht, bool dma) { return dma && ht / (bt < 32 ? 8 : 4) >= 16 ? 512 : 256; }
+// Lanes per workgroup: 4 wave64, 8 for the DMA tiles of 64 and more rows, and
+// of 32 rows x 128 and more columns. The ring's reads and multiplies run back to
+// back within a wave (each read block ends with its wait), so with one wave per
+// SIMD every LDS round trip was exposed; a second wave multiplies meanwhile.
+// Calls with the gather, 4 -> 8 waves (graph replay, us): gate/up 4096 -> 2 x 14336
+// at 128 rows 40.3 -> 36.0, 5120 -> 2 x 17408 at 33 / 128 rows 54.0 -> 49.7 / 79.8 ->
+// 69.3, down 17408 -> 5120 at 33 31.2 -> 29.2; of 32 x 128 q/k/v 4096 at 17 rows 16.1
+// -> 15.2. The smaller tiles multiply too little per chunk to hide anything and
+// wait at the ring's barriers for twice the waves: 32 x 64 4096 -> 4096 at 24 rows
+// 12.0 -> 12.6, 14336 -> 4096 at 32 20.7 -> 21.4; 16 x 128 17408 -> 5120 at 9 24.7 ->
+// 25.1.
+constexpr int mc_block(int bt, int ht, bool dma) { return dma && (bt >= 64 || (bt == 32 && ht >= 128)) ? 512 : 256; }
 inline int ceil_div_mc(int a, int b) { return (a + b - 1) / b; }
 constexpr int kMcNtAux = 2;  // cache policy of the weight DMA: non-temporal
 

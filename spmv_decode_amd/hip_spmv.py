@@ -259,24 +259,47 @@ def library_route(rows: int, K: int, h: int) -> bool:
 
 def rows_route(rows: int, w: int, hs) -> bool:
     """Whether products of one input past NM_MC_MAX_BATCH rows (16-bit, plan
-    left to the library) run on nm_spmm_rows rather than as one BLAS GEMM each:
-    from 160 rows (at 129 rows half of its second row tile is padding), several
-    products up to rows * (sum of outputs) = 12.6M, and up to 512 rows (two tall
-    row tiles) of up to 36864 outputs; a lone one up to 768 rows when it is
-    deeper than wide (w >= h) and has more than 1024 outputs. The BLAS library
-    runs a GEMM per product, without splitting its depth, and wins on wide
-    outputs of many rows, where its 256-wide tiles read less per multiply.
-    Graph replay, gathers included, nm_spmm_rows / library (us): Llama-3.1-8B down
-    200 / 500 / 1024 rows 43 / 57, 61 / 77, 93 / 107; Qwen3-14B down 200 / 500 /
-    1024 rows 50 / 96, 83 / 99, 158 / 142; q/k/v 200 / 500 / 1024 rows 25 / 48, 29
-    / 59, 45 / 67; Llama-3.1-8B gate and up 200 / 500 / 512 / 1024 rows 46 / 65, 83 / 109,
-    83 / 96, 155 / 139, Qwen3-14B's at 500 rows 135 / 163; o 200 / 500 rows 23 / 20, 26 / 27;
-    Qwen3-32B gate alone 500 / 2048 rows 92 / 77, 298 / 279."""
+    left to the library) run on nm_spmm_rows rather than as one BLAS GEMM each.
+    Never below 160 rows: at 129 half of its second row tile is padding.
+
+    The BLAS library runs a GEMM per product, without splitting its depth; it
+    wins where its 256-wide tiles read less per multiply (wide outputs of many
+    rows) and where the row tiles of nm_spmm_rows are mostly padding (257 to 384
+    rows in tiles of 256, 160 rows of outputs just past two rounds of the chip).
+    The lines lie where the faster side changes in graph replays, gathers
+    included, over 30 shapes and 160-2048 rows (us, nm_spmm_rows / library; a line's other
+    side in brackets; bf16 as fp16):
+
+    * One product needs compressed columns to split: 5120 -> 2048 at 160 / 768 rows 25 /
+      28, 37 / 44, 8192 -> 4096 40 / 85, 83 / 90, 12800 -> 1280 34 / 51, 59 / 94 [2048 ->
+      1152 at 160 / 768 rows 18 / 15, 25 / 22; 3072 -> 2048 at 160 / 400 rows 22 / 21, 27 /
+      25; 4096 -> 1152 at 160 23 / 20].
+    * Several, of s outputs in all (1024-4096 compressed columns). Up to 256 rows: s =
+      32768 at 160 / 256 rows 46 / 58, 49 / 68; wider from 200 rows, s = 34816 at 208 / 256 74 /
+      85, 81 / 87, s = 51200 at 200 / 224 97 / 109, 99 / 106 [34816 at 160 81 / 78].
+    * Up to 384 rows: s = 22528 at 257 / 384 rows 60 / 69, 71 / 78 [s = 28672 at 300 70 / 66;
+      34816 at 400 126 / 112].
+    * Up to 512 rows, three tiles of 128 giving way to two of 256: s = 15360 at 385 / 512
+      rows 27 / 38, 28 / 39; s = 20480 at 385 / 416 rows 43 / 54, 44 / 54 [at 480 76 / 66]; s =
+      28672 at 385 / 512 75 / 89, 82 / 93; s = 34816 at 500 / 512 134 / 147, 134 / 141 [at 480
+      132 / 119].
+    * More rows: s = 12288 at 513 / 768 rows 54 / 61, 78 / 83; s = 10240 at 1024
+      82 / 85 [s = 15360 at 640 65 / 54; s = 8192 at 1536 147 / 133]; with a narrow
+      product among them, which the library serves badly (q/k/v), s = 6144 at 2048 83 /
+      93, s = 10240 at 1200 137 / 196."""
     if rows < 160 or rows > _lib.NM_ROWS_MAX:
         return False
-    if len(hs) > 1:
-        return rows * sum(hs) <= 3 << 22 or (rows <= 512 and sum(hs) <= 9 << 12)
-    return rows <= 768 and w >= hs[0] > 1024
+    if len(hs) == 1:
+        return rows <= 768 and w >= max(hs[0], 5120) and hs[0] > 1024 and w + hs[0] >= 6400
+    s = sum(hs)
+    if rows <= 256:
+        return s <= 32768 or (rows >= 200 and s <= 51200 and rows * s <= 3 << 22)
+    if rows <= 384:
+        return s <= 22528
+    if rows <= 512:
+        return (s <= 16384 or (s <= 25600 and rows <= 416) or 25600 < s <= 32768
+                or (32768 < s <= 36864 and rows >= 500))
+    return s <= 12288 and rows * s <= (3 << 22 if min(hs) <= 1024 else 5 << 21)
 
 
 def nmsparse_spmm_forward_hip(x, mat_data, mat_index, w, h, BLOCK_WIDTH, VEC_WIDTH, *, out=None, config_id=-1,

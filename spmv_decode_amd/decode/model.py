@@ -356,17 +356,33 @@ def causal_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, n_kv_hea
     return o.squeeze(0).transpose(0, 1).reshape(P, nh * d)
 
 
+def prompt_kernel_positions(n_heads: int, kv_heads: int, head_dim: int) -> int:
+    """The longest prompt whose attention runs in the library's prompt launches.
+    The work grows with the square of the length and PyTorch's fused attention
+    does it at the higher rate (32 heads, 16384 positions: 0.45 PFLOP/s against 0.39); its transposes and the
+    separate rotation and copies, which grow with the length, weigh less and less. bf16,
+    graph replay (us, general path / launches): 64 heads over 8 of 128 at 6144 /
+    8192 positions 1700 / 1683, 2735 / 2914; 32 over 8 at 8192 / 10240 1508 / 1471, 2174 /
+    2260; 16 over 8 at 8192 / 16384 890 / 778, 2727 / 2863; 32 over 4 of 64 at 3072 / 4096 179 /
+    156, 250 / 258."""
+    if head_dim < 128 and n_heads != kv_heads:
+        return 3072
+    return 8192 if n_heads <= 32 else 6144
+
+
 def prompt_attention(at, q, k, v, freqs, rope, k_cache_t, v_cache_t) -> torch.Tensor:
     """The attention of a whole prompt from its projections q [P, q], k and v
     [P, kv] (at: the attention module): head norms, rotary embedding (freqs
     complex64 [P, 1, head_dim / 2] or the same as the fp32 table rope), keys and
     values into the caches at positions 0 .. P-1, causal attention. Where the
     layer decodes on the library's attention kernel (attend_at), these operands
-    are within its forms and the head norms are plain ones of one eps, the
-    library's two prompt launches. Returns [P, q]."""
+    are within its forms, the head norms are plain ones of one eps and the prompt
+    is not too long (prompt_kernel_positions), the library's two prompt launches.
+    Returns [P, q]."""
     c = at.cfg
     hd, P = c.head_dim, q.shape[0]
-    rows = (on_kernel(at) and not torch.compiler.is_compiling()
+    rows = (on_kernel(at) and P <= prompt_kernel_positions(c.n_heads, c.n_kv_heads, hd)
+            and not torch.compiler.is_compiling()
             and all(t.stride(1) == 1 and t.stride(0) % 8 == 0 and t.data_ptr() % 16 == 0
                     and t.dtype == k_cache_t.dtype for t in (q, k, v)))
     norms = (at.q_norm, at.k_norm) if c.qk_norm else ()

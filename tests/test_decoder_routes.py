@@ -240,3 +240,21 @@ def test_a_dense_prompt_compiles_whole(gpu):
     got = torch.compile(model.prefill, backend="eager", fullgraph=True)(prompt())
     close(got, ref)
     close(model.k_store[:, :, :64, :9], keys[:, :, :64, :9])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("P", [3072, 3073])
+def test_long_prompts_take_the_faster_attention(gpu, monkeypatch, P):
+    """Both sides of the length at which PyTorch's attention is faster (4 heads
+    over 2 of 64: 3072 positions) agree."""
+    from spmv_decode_amd.decode import model as dm
+
+    model = decoder(n_layers=1)
+    model.setup_cache(3200, torch.device("cuda"))
+    calls = []
+    plain = dm.causal_attention
+    monkeypatch.setattr(dm, "causal_attention", lambda *a: calls.append(1) or plain(*a))
+    got = model.prefill(prompt(P))
+    assert len(calls) == (P > 3072)
+    monkeypatch.setattr(dm, "prompt_kernel_positions", lambda *a: 0 if P == 3072 else 1 << 20)
+    close(got, model.prefill(prompt(P)))

@@ -46,14 +46,17 @@ static_assert(kBM == kRowsTile && kBN == kRowsTile, "tile shape");
 static_assert(kStages * kStage <= 160 * 1024, "LDS");
 static_assert(kStages * kOps < 64, "vmcnt is a 6-bit counter");
 
-// One DMA of 1 KB: lane l's 16 B at base + off to LDS byte lds + 16 l. M0 (the
-// LDS address) is set where it is used; nothing else in this file needs it.
+// One DMA of 1 KB: lane l's 16 B at base + off to LDS byte lds + 16 l (M0, which
+// the compiler is told it loses; the warning is that nothing restores it).
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
 __device__ __forceinline__ void dma16(const void* base, uint32_t off, uint32_t lds) {
 #if defined(__HIP_DEVICE_COMPILE__)
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(base)
-               : "memory");
+               : "m0", "memory");
 #endif
 }
+#pragma clang diagnostic pop
 
 // This wave's loads but for the last VM have landed and its LDS reads but for
 // the last LGKM have returned; then the workgroup's barrier.

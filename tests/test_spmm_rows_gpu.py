@@ -3,7 +3,7 @@ and of the gathers through LDS: against the oracle bar at ragged depths (a last
 chunk shorter than 64 columns, a single chunk, fewer chunks than splits), row
 counts at the edges of its 128-row tiles, every split count, groups of products
 of different widths, the SiLU-product input, and masks that name positions of
-another group or outside x."""
+another group or outside x; and infinite weights at the end of a ragged depth."""
 import ctypes
 
 import pytest
@@ -150,3 +150,34 @@ def test_rows_route_and_arguments(gpu):
     assert call(dtype=2) == -7 and call(x=None) == -1 and call(stride_x=127) == -2 and call(rows=0) == -2
     assert call(w=63) == -4 and call(splits=9) == -7 and call(nbytes=need - 1) == -6
     assert call(scratch=X.data_ptr() + 16) == -5 and call(out=(ctypes.c_void_p * 1)(X.data_ptr() + 2)) == -5
+
+
+# compressed columns: last chunks of 8 and 32 columns behind 0 to 6 whole ones (every stage of both rings), and of 24 to 62
+DEPTHS = [64 * k + r for k in range(7) for r in (8, 32)] + [24, 500, 62, 254]
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16], ids=str)
+@pytest.mark.parametrize("w", DEPTHS)
+def test_ragged_last_chunks_of_an_infinite_last_row(gpu, dtype, w):
+    """Rows of the last chunk past the split hold copies of its last weight row
+    until they are cleared: an infinite one there, times the zero activations
+    behind it, would turn the outputs to NaN. They are +-Inf, and the others
+    the bits of finite weights."""
+    rows, h = 150, 256
+    _, md, mi = make_case(2 * w, h, 2, 4, seed=w, dtype=dtype)
+    X = torch.randn(rows, 2 * w, generator=torch.Generator(device="cuda").manual_seed(w), device="cuda").to(dtype)
+    last = X[:, (w - 1) // 2 * 4 + int(mi.view(-1)[-1])].float()
+    assert bool((last != 0).all())
+    bad = md.clone()
+    bad[-1, ::7] = float("inf")
+    finite = torch.ones(h, dtype=torch.bool, device="cuda")
+    finite[::7] = False
+    for height in (_lib.NM_ROWS_SHORT, _lib.NM_ROWS_TALL):
+        for splits in (1, 2, 3):
+            say(f"ragged {dtype} w {w} height {height} splits {splits}")
+            plain, got = (torch.full((rows, h), 7.0, dtype=dtype, device="cuda") for _ in range(2))
+            hip_spmv._spmm_rows(X, [(md, mi)], w, 2, 4, [plain], splits=height + splits)
+            hip_spmv._spmm_rows(X, [(bad, mi)], w, 2, 4, [got], splits=height + splits)
+            check_rows(plain, X, md, mi, 2, 4, f"ragged {dtype} {w}")
+            assert torch.equal(got[:, finite], plain[:, finite])
+            assert torch.equal(got[:, ~finite].float(), (last * float("inf"))[:, None].expand(-1, int((~finite).sum())))

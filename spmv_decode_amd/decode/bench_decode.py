@@ -246,7 +246,7 @@ def main(argv=None):
         gc.collect()
         torch.cuda.empty_cache()
         log(f"swapped {n} Linears to {a.m // 2}:{a.m} in {time.time() - t0:.1f} s")
-        if not a.no_tune:  # lm_head stays dense in the sparse model (already tuned if dense ran)
+        if not a.no_tune:  # what stays dense in the sparse model (tuned already if dense ran)
             for shape, r in model.tune_dense_gemv().items():
                 log(f"dense GEMV {shape}: x*W^T {r['mm']} us, W*x {r['mv']} us -> {r['form']}")
                 res.setdefault("dense_gemv_forms", {})[shape] = r

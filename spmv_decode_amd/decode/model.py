@@ -893,12 +893,15 @@ class Decoder(nn.Module):
         GPU: each form is timed over every weight of that shape in the model
         (all layers in order, so the weights stream from HBM as in a decode
         step), captured in one hipGraph and replayed `reps` times; the median
-        replay decides. Shapes already tuned are kept. Returns {"n_out x n_in":
+        replay decides. Shapes already tuned are kept; an output head that
+        decodes in the library's dense GEMV (project_head) is no such product. Returns {"n_out x n_in":
         {"mm": us, "mv": us, "form": ...}} (us per product) for the shapes
         timed now. Changes only how dense products are issued, not their math
         (both forms accumulate in fp32; the roundings can differ in the last bit)."""
         groups = {}
-        for w, _, _ in self._dense_gemv_sites():
+        for w, owner, _ in self._dense_gemv_sites():
+            if owner is self.lm_head and self._head_kernel_takes(w.dtype):
+                continue
             if not w.is_cuda:
                 raise RuntimeError(f"tune_dense_gemv times the products on the GPU; a dense weight is on {w.device}")
             groups.setdefault(tuple(w.shape), {})[w.data_ptr()] = w
@@ -918,6 +921,14 @@ class Decoder(nn.Module):
             report[f"{shape[0]}x{shape[1]}"] = {**{k: round(v, 2) for k, v in us.items()}, "form": best}
         self._apply_gemv_forms()
         return report
+
+    def _head_kernel_takes(self, dtype) -> bool:
+        """Whether the output head of a row of this type runs in the library's dense GEMV."""
+        from ..hip_spmv import dense_gemv_supported
+
+        head = self.lm_head
+        return (type(head) is nn.Linear and head.bias is None and head.weight.is_cuda
+                and dense_gemv_supported(torch.empty(1, self.cfg.dim, device=head.weight.device, dtype=dtype), head.weight))
 
     def setup_cache(self, max_seq: int, device, dtype=torch.float16):
         """Static caches for max_seq positions (see attend for the layouts); the
@@ -940,15 +951,12 @@ class Decoder(nn.Module):
         self.rope = torch.polar(torch.ones_like(ang), ang).to(torch.complex64).to(device)
         self.rope_real = torch.view_as_real(self.rope)  # the same table as fp32 (cos, sin) pairs
         self.positions = torch.arange(max_seq, device=device)
-        kernel = head = False
+        kernel = False
+        self.head_kernel = self.q_pad.is_cuda and self._head_kernel_takes(dtype)
         if self.q_pad.is_cuda:
-            from ..hip_spmv import attention_supported, dense_gemv_supported
+            from ..hip_spmv import attention_supported
 
-            head = (type(self.lm_head) is nn.Linear and self.lm_head.bias is None
-                    and dense_gemv_supported(torch.empty(1, c.dim, device=self.q_pad.device, dtype=dtype),
-                                             self.lm_head.weight))
             kernel = c.n_layers > 0 and attention_supported(self.q_pad, self.k_cache_t[0], self.v_cache_t[0], hd)
-        self.head_kernel = head
         for at in self.layers.modules():  # those inside a layer's wrapper as well
             if isinstance(at, (Attention, GptFastAttention)):  # a class of its own may read the mask rows
                 at.decode_kernel = kernel and type(at) in (Attention, GptFastAttention)

@@ -258,3 +258,18 @@ def test_long_prompts_take_the_faster_attention(gpu, monkeypatch, P):
     assert len(calls) == (P > 3072)
     monkeypatch.setattr(dm, "prompt_kernel_positions", lambda *a: 0 if P == 3072 else 1 << 20)
     close(got, model.prefill(prompt(P)))
+
+
+@pytest.mark.gpu
+def test_tuning_reports_the_products_that_run(gpu):
+    """The head decodes in its own GEMV: neither BLAS form of it is timed or reported."""
+    model = decoder()
+    report = model.tune_dense_gemv(reps=2, warmup=1)
+    assert report and "512x256" not in report
+    with pytest.raises(KeyError):
+        model.gemv_forms[512, 256]
+    model.setup_cache(128, torch.device("cuda"))
+    assert model.head_kernel
+    odd = decoder()
+    odd.lm_head.weight.data = odd.lm_head.weight.data.t().contiguous().t()
+    assert "512x256" in odd.tune_dense_gemv(reps=2, warmup=1)

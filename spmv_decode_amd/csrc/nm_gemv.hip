@@ -598,12 +598,8 @@ int launch_spmm_group(int dtype, const void* x, long long x_row_stride, int batc
     part += p[i].workspace - NM_TICKET_BYTES;
   }
   const int gslot = gather_slot(p[0].rows_per_split);  // <= 2: rows_per_split <= kMaxRowsSpmm
-  const SpmmRow& row = spmm_table(dtype)[p[0].cfg];
-  const int nb = spmm_nb_slot(batch);
-  if (n == 1)
-    hipLaunchKernelGGL(row.fn[nb][gslot], dim3((unsigned)blocks), dim3(kBlock), 0, static_cast<hipStream_t>(stream), g.p[0]);
-  else
-    hipLaunchKernelGGL(row.group[nb][gslot], dim3((unsigned)blocks), dim3(kBlock), 0, static_cast<hipStream_t>(stream), g);
+  const SpmmFn fn = spmm_table(dtype)[p[0].cfg].fn[spmm_nb_slot(batch)][gslot];
+  hipLaunchKernelGGL(fn, dim3((unsigned)blocks), dim3(kBlock), 0, static_cast<hipStream_t>(stream), g);
   hipError_t e = hipGetLastError();
   return e == hipSuccess ? NM_OK : (int)e;
 }

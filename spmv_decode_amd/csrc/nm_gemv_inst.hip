@@ -28,12 +28,10 @@ namespace nm_hip {
 #define NM_PLAIN_ROW(TH, U, NT) NM_ROW(1, TH, U, NT)
 #define NM_PAIR_ROW(TH, U, NT) NM_ROW(2, TH, U, NT)
 
-#define NM_SPMM_G(ARGS, TH, U, NT, NB) \
-  {&nm_spmm_kernel<NM_INST_DTYPE, TH, U, 1, NT, NB, ARGS>, &nm_spmm_kernel<NM_INST_DTYPE, TH, U, 2, NT, NB, ARGS>, \
-   &nm_spmm_kernel<NM_INST_DTYPE, TH, U, 4, NT, NB, ARGS>}
-#define NM_SPMM_NB(ARGS, TH, U, NT) \
-  {NM_SPMM_G(ARGS, TH, U, NT, 2), NM_SPMM_G(ARGS, TH, U, NT, 4), NM_SPMM_G(ARGS, TH, U, NT, 8)}
-#define NM_SPMM_ROW(TH, U, NT) {NM_SPMM_NB(SpmmArgs, TH, U, NT), NM_SPMM_NB(SpmmGroupArgs, TH, U, NT)},
+#define NM_SPMM_G(TH, U, NT, NB) \
+  {&nm_spmm_kernel<NM_INST_DTYPE, TH, U, 1, NT, NB>, &nm_spmm_kernel<NM_INST_DTYPE, TH, U, 2, NT, NB>, \
+   &nm_spmm_kernel<NM_INST_DTYPE, TH, U, 4, NT, NB>}
+#define NM_SPMM_ROW(TH, U, NT) {{NM_SPMM_G(TH, U, NT, 2), NM_SPMM_G(TH, U, NT, 4), NM_SPMM_G(TH, U, NT, 8)}},
 
 #if NM_INST_DTYPE == NM_DTYPE_F16
 #define NM_PLAIN_TABLE kPlainKernelsF16

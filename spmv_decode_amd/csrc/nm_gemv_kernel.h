@@ -962,23 +962,8 @@ struct SpmmGroupArgs {
   int n;
 };
 
-// The product that workgroup `local` of the grid works on; `local` becomes its
-// number within the product. A launch of one product passes its arguments as
-// they are: found among several, they come later, by a dependent scalar load, 2-5%
-// of a call (14336 -> 4096, 8 rows, fp16, M = 64: 20.4 us against 19.4).
-__device__ __forceinline__ const SpmmArgs& spmm_product(const SpmmArgs& a, int&) { return a; }
-__device__ __forceinline__ const SpmmArgs& spmm_product(const SpmmGroupArgs& g, int& local) {
-  int i = 0;
-#pragma unroll
-  for (int q = 1; q < kMaxProblems; ++q)
-    if (q < g.n && local >= g.first[q]) i = q;
-  local -= g.first[i];
-  return g.p[i];
-}
-
-// Args: SpmmArgs or SpmmGroupArgs.
-template <int DT, int TH, int U, int G, bool NT, int NB, class Args>
-__global__ __launch_bounds__(kBlock) void nm_spmm_kernel(Args args) {
+template <int DT, int TH, int U, int G, bool NT, int NB>
+__global__ __launch_bounds__(kBlock) void nm_spmm_kernel(SpmmGroupArgs g) {
   using E = Elem<DT>;
   typedef typename E::scalar T;
   constexpr int W = E::kWords;
@@ -994,8 +979,23 @@ __global__ __launch_bounds__(kBlock) void nm_spmm_kernel(Args args) {
   __shared__ __attribute__((aligned(16))) float red[NB][TK * HT];
   __shared__ int is_last;
 
+  // The first product's arguments are on their way at once, so a launch of one
+  // waits as if it were the only kind; only a workgroup of another product waits
+  // twice. (Chosen before any load, they cost a launch of one 2-5%: 14336 -> 4096, 8
+  // rows, fp16, M = 64 20.4 us against 19.0; two instances of the kernel made a SwiGLU
+  // MLP of 4 rows, whose launches then share no code, 1-2 us slower per pass.)
+  SpmmArgs a = g.p[0];
   int local = (int)blockIdx.x;
-  const SpmmArgs& a = spmm_product(args, local);
+  if (g.n > 1) {
+    int pi = 0;
+#pragma unroll
+    for (int q = 1; q < kMaxProblems; ++q)
+      if (q < g.n && local >= g.first[q]) pi = q;
+    if (pi > 0) {
+      a = g.p[pi];
+      local -= g.first[pi];
+    }
+  }
   const int h = a.h;
   const int tid = threadIdx.x;
   const int th = tid % TH;
@@ -1276,13 +1276,11 @@ struct KernelRow {
 #define NM_SPMM_CONFIGS(X) X(16, 4, true) X(16, 8, true) X(32, 4, true) X(32, 8, true)
 constexpr int kNumSpmmConfigs = 4;
 
-typedef void (*SpmmFn)(SpmmArgs);
-typedef void (*SpmmGroupFn)(SpmmGroupArgs);
+typedef void (*SpmmFn)(SpmmGroupArgs);
 
 // fn[batch rows per launch: 2, 4, 8][gather slot: 256, 512, 1024 columns per split].
 struct SpmmRow {
   SpmmFn fn[3][3];
-  SpmmGroupFn group[3][3];
 };
 
 // Defined in nm_gemv_inst.hip, one object per element type.

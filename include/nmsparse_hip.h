@@ -459,7 +459,10 @@ int nm_spmm_rows(int dtype, const void* x, const void* up, long long x_row_strid
  * Configuration introspection. nm_config_describe writes a short text such as
  * "th32_u8" into buf (ids nm_num_configs() + j describe pair configuration j);
  * nm_gemv_plan reports the configuration and split count the library would
- * use for a single GEMV of a shape (config_id < 0: its own choice).
+ * use for a single GEMV of a shape (config_id < 0: its own choice). An fp32
+ * launch of the library's own choice may run configurations 3 and 6 in their
+ * cached-load forms 11 and 12 (the same plan and bits). nm_gemv_launch_plan
+ * reports the plan likewise.
  */
 int nm_num_configs(void);
 int nm_config_describe(int config_id, char* buf, int buf_len);

@@ -164,7 +164,9 @@ def check(code: int, what: str) -> None:
 
 
 def plan(h: int, w: int, nnz: int, m: int, config_id: int = -1, splits: int = 0) -> dict:
-    """Configuration, split count, grid size and rows per split the library uses."""
+    """Configuration, split count, grid size and rows per split the library uses
+    (fp32 left to its choice may run configurations 3 and 6 as 11 and 12, their
+    cached-load forms)."""
     cfg, sp, blocks, rows = ctypes.c_int(), ctypes.c_int(), ctypes.c_int(), ctypes.c_int()
     rc = load().nm_gemv_plan(h, w, nnz, m, config_id, splits, ctypes.byref(cfg), ctypes.byref(sp),
                              ctypes.byref(blocks), ctypes.byref(rows))

@@ -75,16 +75,28 @@ int auto_config(long long h_total, int nmat, bool carried) {
   return h_total > 16384 ? 6 : (h_total > 4096 ? 3 : 1);
 }
 
-// fp32 on 256- and 512-row tiles: the same configuration with cached loads. An
-// fp32 lane reads its 32 bytes of a row in two loads, each half of every cache
-// line; read past the cache, a line came from memory for each half (graph
-// replay, non-temporal / cached: 4096 -> 14336 27.3 / 23.1 us, 5120 -> 17408 38.4 /
-// 33.4; 128-row tiles measured the same either way).
-int cached_twin(int cfg) { return cfg == 3 ? 11 : (cfg == 6 ? 12 : cfg); }
-
 // Workgroups that run at once, one per CU: an MI355X has 256 CUs. The split
 // count below is chosen for this many; it changes speed only, never results.
 constexpr int kPlanCUs = 256;
+
+// fp32 on 256- and 512-row tiles: the same configuration with cached loads (cfg
+// 3 -> 11, 6 -> 12). An fp32 lane reads its 32 bytes of a row in two loads, each half
+// of every cache line; read past the cache, a line came from memory for each half
+// (graph replay, us, non-temporal / cached: 4096 -> 14336 28.8 / 26.0, 5120 -> 17408 41.3
+// / 37.8, 8192 -> 28672 95.5 / 86.9; 128-row tiles measured the same either way). Not
+// where the workgroups fill the chip in whole rounds over long columns, where the
+// cached form measured slower (2048 -> 8192 10.5 / 11.2, 4096 -> 8192 16.5 / 17.5, 16384 ->
+// 8192 57.7 / 63.2, 8192 -> 16384 53.9 / 55.0; over shorter ones it gains, 1024 -> 8192 8.9 /
+// 8.5, 4096 -> 16384 29.0 / 28.7), nor past 28672 outputs, where it goes either way by
+// 1-4% (2048 -> 32768 29.4 / 30.3, 131072 109.2 / 105.3, 151552 120.2 / 123.4).
+constexpr long long kCachedOutputs = 28672;
+int cached_twin(int cfg, const int* hs, int n, int blocks, int w) {
+  long long h = 0;
+  for (int i = 0; i < n; ++i) h += hs[i];
+  const long long rounds = blocks / kPlanCUs;
+  if (h > kCachedOutputs || (blocks % kPlanCUs == 0 && w >= 1024 * rounds * rounds)) return cfg;
+  return cfg == 3 ? 11 : (cfg == 6 ? 12 : cfg);
+}
 
 // Default split count. About 8 splits of the compressed columns per tile: the
 // cost of a split-K handoff (one partial publish, one arrival atomic on a
@@ -465,7 +477,7 @@ int launch(const nm_gemv_launch_desc& d, void* workspace, size_t workspace_bytes
   const int variant = silu_in    ? kVarSilu
                       : carry_in ? (d.carry_splits == 1 ? kVarCarry1 : (d.carry_splits <= 8 ? kVarCarry8 : kVarCarry16))
                                  : (d.norm_weight ? kVarNorm : kVarPlain);
-  const int kcfg = d.dtype == NM_DTYPE_F32 && !pair && d.config_id < 0 ? cached_twin(p.cfg) : p.cfg;
+  const int kcfg = d.dtype == NM_DTYPE_F32 && !pair && d.config_id < 0 ? cached_twin(p.cfg, hs, nprob, p.blocks, d.w) : p.cfg;
   const KernelFn fn = kernel_table(d.dtype, pair)[kcfg].fn[gather_slot(p.rows_per_split)][variant];
   if (!fn) return NM_ERR_BAD_EPILOGUE;
   hipLaunchKernelGGL(fn, dim3(p.blocks), dim3(kBlock), 0, static_cast<hipStream_t>(stream), a);

@@ -12,9 +12,11 @@
 //
 //  * A workgroup (256 lanes = 4 wave64) owns one key/value head and a split of
 //    PW consecutive positions for all g query heads; splits past pos end at
-//    once, so the work follows the position and not the cache length. At
-//    decode contexts the caches are a few MB: the launch is bound by latency,
-//    so every load of a split is requested before the first is waited for.
+//    once, so the work follows the position. PW follows the cache length
+//    (make_attn_plan): an early position of a long cache runs in the few large
+//    splits that its end needs. At decode contexts the caches are a few MB: the
+//    launch is bound by latency, so every load of a split is requested before
+//    the first is waited for.
 //  * Scores on the matrix cores: A = the queries (g rows of 16), B = K through
 //    LDS, read transposed (ds_read_b64_tr_b16: rows are head dimensions, the
 //    columns positions, as the weights of the matrix-core SpMM); each wave 16

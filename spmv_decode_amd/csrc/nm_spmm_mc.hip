@@ -16,7 +16,7 @@
 //  * A first kernel gathers the activations once per call, Xg[b, c] =
 //    x[b, (c/nnz)*m + mat_index[c]], into the workspace ([batch, wp], wp = w
 //    rounded up to whole 64-column chunks, zero past w).
-//  * The main kernel: a workgroup (4 wave64, 8 in the DMA variant) owns an
+//  * The main kernel: a workgroup (4 wave64, 8 in the larger DMA tiles) owns an
 //    output tile of HT columns r and all BT >= batch rows (16, 32, 64 or 128),
 //    over one split of the compressed columns c. The waves split the tile into
 //    row ranges (one 16-row block each up to 32 rows, two / four blocks each at
@@ -51,8 +51,8 @@ static_assert(NM_MC_MAX_BATCH == 128, "batch tiles of 16, 32, 64 and 128 rows");
 // weights and their activation fragments in flight): 4 / 3 / 3 for 64- /
 // 128- / 256-column tiles, fitted to graph-replay sweeps of 2-8 stages at
 // 16-64 rows over the Llama-3.1-8B and Qwen3 shapes (deeper rings measured
-// up to 8% slower, two stages up to 30%). At most 65 KB of LDS per
-// workgroup.
+// up to 8% slower, two stages up to 30%). 41 to 120 KB of LDS per workgroup
+// (120: 64 rows x 256 columns).
 constexpr int mc_stages(int ht) { return ht == 64 ? 4 : 3; }
 // Lanes per workgroup: 4 wave64, 8 for the DMA tiles of 64 and more rows, and
 // of 32 rows x 128 and more columns. The ring's reads and multiplies run back to

@@ -46,10 +46,12 @@ CACHE_ALIGN = 128
 
 def cache_length(max_seq: int) -> int:
     """Static KV-cache length for `max_seq` positions: rounded up to a
-    multiple of CACHE_ALIGN. The attention products over the cache pick much
-    slower BLAS kernels at other lengths (MI355X, 8 KV heads x 128: the three
-    attention kernels take 17.2 us per layer at 384 positions but 19.8 us at
-    392; 19.4 us at 1024 but 28.2 us at 1032)."""
+    multiple of CACHE_ALIGN. Where attention runs in PyTorch (attend: fp32
+    caches, head sizes other than 64 and 128, more than 16 query heads per
+    key/value head), its products over the cache pick much slower BLAS kernels
+    at other lengths (MI355X, 8 KV heads x 128: its three kernels take 17.2 us
+    per layer at 384 positions but 19.8 us at 392; 19.4 us at 1024 but 28.2 us at
+    1032). The library's attention kernel needs multiples of 8 only."""
     return -(-max_seq // CACHE_ALIGN) * CACHE_ALIGN
 
 

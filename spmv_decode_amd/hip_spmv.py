@@ -267,8 +267,8 @@ def rows_route(rows: int, w: int, hs) -> bool:
     rows) and where the row tiles of nm_spmm_rows are mostly padding (257 to 384
     rows in tiles of 256, 160 rows of outputs just past two rounds of the chip).
     The lines lie where the faster side changes in graph replays, gathers
-    included, over 30 shapes and 160-2048 rows (us, nm_spmm_rows / library; a line's other
-    side in brackets; bf16 as fp16):
+    included, over 123 shapes and 160-2048 rows (us, nm_spmm_rows / library; a line's
+    other side in brackets; bf16 as fp16):
 
     * One product needs compressed columns to split: 5120 -> 2048 at 160 / 768 rows 25 /
       28, 37 / 44, 8192 -> 4096 40 / 85, 83 / 90, 12800 -> 1280 34 / 51, 59 / 94 [2048 ->

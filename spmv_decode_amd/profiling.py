@@ -67,6 +67,8 @@ def spmm_algorithmic(K, h, rows, nnz=32, m=64):
 
 
 def _spmm_dispatches(rows):
+    """The dispatches of SPMM_PROBE_CLASSES: one product each, up to 64 rows (no
+    grouped launch and no nm_spmm_rows kernel among them)."""
     out = []
     for r in rows:
         n = r["Kernel_Name"]

@@ -981,9 +981,8 @@ __global__ __launch_bounds__(kBlock) void nm_spmm_kernel(SpmmGroupArgs g) {
 
   // The first product's arguments are on their way at once, so a launch of one
   // waits as if it were the only kind; only a workgroup of another product waits
-  // twice. (Chosen before any load, they cost a launch of one 2-5%: 14336 -> 4096, 8
-  // rows, fp16, M = 64 20.4 us against 19.0; two instances of the kernel made a SwiGLU
-  // MLP of 4 rows, whose launches then share no code, 1-2 us slower per pass.)
+  // twice. Chosen before any load, they cost a launch of one 2-5% (14336 -> 4096, 8
+  // rows, fp16, M = 64: 20.4 us against 19.0).
   SpmmArgs a = g.p[0];
   int local = (int)blockIdx.x;
   if (g.n > 1) {

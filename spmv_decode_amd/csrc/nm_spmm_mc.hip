@@ -608,8 +608,9 @@ __global__ __launch_bounds__(kBlock) void nm_gather_mc_kernel(GatherArgs a) {
 // Graph replay, fp16 at 32:64, direct / through LDS (us): 4096 columns of input,
 // 500 / 1024 / 2048 rows 4.1 / 5.0, 5.9 / 5.5, 9.5 / 6.9; 14336 columns, 200 / 500
 // / 2048 rows 4.9 / 5.3, 8.6 / 6.6, 28.3 / 22.3; small ones 2.7 / 3.8: so from
-// kGatherLds gathered elements on. Positions outside the window (a mask that
-// names another group) are loaded one by one.
+// kGatherLds gathered elements of a product on (the times are of one product; two
+// or three of them in one launch take the direct form up to the same size).
+// Positions outside the window (a mask that names another group) are loaded one by one.
 constexpr long long kGatherLds = 1 << 21;
 constexpr int kGC = 128, kGR = 32, kGWin = 512;
 template <bool FRAG, int SDT, bool IEEE>

@@ -58,6 +58,8 @@ from dataclasses import dataclass, field
 import torch
 import torch.nn as nn
 import torch.nn.functional as F
+from torch.autograd import forward_ad
+from torch.nn.modules import module as _module
 
 
 @dataclass(frozen=True)
@@ -188,8 +190,8 @@ def on_kernel(at) -> bool:
 def reads_position(layer: nn.Module) -> bool:
     """Whether the layer's attention takes the position itself (attend_at on the
     library's kernel); any other reads the mask rows of the key caches."""
-    at = layer.self_attn if isinstance(layer, Block) else getattr(layer, "attention", None)
-    return hasattr(at, "decode_kernel") and on_kernel(at)
+    at = layer._modules.get("self_attn" if isinstance(layer, Block) else "attention")
+    return getattr(at, "decode_kernel", False) and not forward_mode()
 
 
 def linear_into(lin: nn.Module, x2d: torch.Tensor, out: torch.Tensor) -> torch.Tensor:
@@ -247,7 +249,7 @@ def project(lin: nn.Module, x: torch.Tensor) -> torch.Tensor:
 def forward_mode() -> bool:
     """Whether a forward-mode level is open: tangents may then ride on any
     operand, and the library's launches would drop them."""
-    return not torch.compiler.is_compiling() and torch.autograd.forward_ad._current_level >= 0
+    return forward_ad._current_level >= 0 and not torch.compiler.is_compiling()
 
 
 def differentiated(*tensors) -> bool:
@@ -273,10 +275,10 @@ def project_head(lin: nn.Module, x: torch.Tensor, kernel: bool) -> torch.Tensor:
 def plain_norm(norm: nn.Module) -> bool:
     """Whether calling this module is an RMSNorm of its weight and a given eps
     (None: PyTorch's own choice) and nothing else: no other class or forward, no hooks."""
-    hooks = nn.modules.module
-    return (type(norm) is RMSNorm and norm.eps is not None and norm.eps >= 0 and "forward" not in vars(norm)
-            and not (norm._forward_hooks or norm._forward_pre_hooks or hooks._global_forward_hooks
-                     or hooks._global_forward_pre_hooks))
+    own = norm.__dict__
+    return (type(norm) is RMSNorm and not own["_forward_hooks"] and not own["_forward_pre_hooks"]
+            and "forward" not in own and own.get("eps") is not None and own["eps"] >= 0
+            and not _module._global_forward_hooks and not _module._global_forward_pre_hooks)
 
 
 def add_norm(norm: nn.Module, x: torch.Tensor, d: torch.Tensor) -> tuple:
@@ -385,14 +387,15 @@ def prompt_attention(at, q, k, v, freqs, rope, k_cache_t, v_cache_t) -> torch.Te
             and not torch.compiler.is_compiling()
             and all(t.stride(1) == 1 and t.stride(0) % 8 == 0 and t.data_ptr() % 16 == 0
                     and t.dtype == k_cache_t.dtype for t in (q, k, v)))
-    norms = (at.q_norm, at.k_norm) if c.qk_norm else ()
-    if rows and all(plain_norm(n) and n.weight.dtype == q.dtype and n.weight.is_contiguous() and n.eps == norms[0].eps
-                    for n in norms):
+    qn, kn = (at.q_norm, at.k_norm) if c.qk_norm else (None, None)
+    if rows and (qn is None or (qn.weight.dtype == kn.weight.dtype == q.dtype and plain_norm(qn) and plain_norm(kn)
+                                and qn.eps == kn.eps and qn.weight.is_contiguous() and kn.weight.is_contiguous())):
         from ..hip_spmv import nmsparse_prefill_attention
 
-        weights = dict(zip(("q_norm", "k_norm"), (n.weight for n in norms)))
-        return nmsparse_prefill_attention(q, k, v, k_cache_t, v_cache_t, rope, hd,
-                                          norm_eps=norms[0].eps if norms else 0.0, **weights)
+        if qn is None:
+            return nmsparse_prefill_attention(q, k, v, k_cache_t, v_cache_t, rope, hd)
+        return nmsparse_prefill_attention(q, k, v, k_cache_t, v_cache_t, rope, hd, q_norm=qn.weight, k_norm=kn.weight,
+                                          norm_eps=qn.eps)
     q, k, v = q.reshape(P, c.n_heads, hd), k.reshape(P, c.n_kv_heads, hd), v.reshape(P, c.n_kv_heads, hd)
     if c.qk_norm:
         q, k = at.q_norm(q), at.k_norm(k)

@@ -270,36 +270,48 @@ def rows_route(rows: int, w: int, hs) -> bool:
     included, over 123 shapes and 160-2048 rows (us, nm_spmm_rows / library; a line's
     other side in brackets; bf16 as fp16):
 
-    * One product needs compressed columns to split: 5120 -> 2048 at 160 / 768 rows 25 /
-      28, 37 / 44, 8192 -> 4096 40 / 85, 83 / 90, 12800 -> 1280 34 / 51, 59 / 94 [2048 ->
-      1152 at 160 / 768 rows 18 / 15, 25 / 22; 3072 -> 2048 at 160 / 400 rows 22 / 21, 27 /
-      25; 4096 -> 1152 at 160 23 / 20].
-    * Several, of s outputs in all (1024-4096 compressed columns). Up to 256 rows: s =
+    * One product, up to 768 rows, needs compressed columns to split, fewer of them
+      the more rows and outputs there are: 12800 -> 1280 at 160 / 768 rows 34 / 51, 59 / 94,
+      8192 -> 4096 40 / 85, 83 / 90, 4096 -> 2048 at 160 / 256 / 768 24 / 24, 24 / 27, 33 / 38, 3840
+      -> 2048 at 300 26 / 28 [at 400-512 30 / 29], 3072 -> 2560 at 400 / 768 28 / 36, 31 / 35 [at
+      192 24 / 22], 4096 -> 1152 at 512 26 / 30 [at 160 23 / 20]; [2048 -> 1152 at 160 / 768 18 /
+      15, 25 / 22; 3072 -> 2048 at 160 / 400 22 / 21, 27 / 25].
+    * Several, of s outputs in all (512-4096 compressed columns). Up to 256 rows: s =
       32768 at 160 / 256 rows 46 / 58, 49 / 68; wider from 200 rows, s = 34816 at 208 / 256 74 /
       85, 81 / 87, s = 51200 at 200 / 224 97 / 109, 99 / 106 [34816 at 160 81 / 78].
-    * Up to 384 rows: s = 22528 at 257 / 384 rows 60 / 69, 71 / 78 [s = 28672 at 300 70 / 66;
-      34816 at 400 126 / 112].
+    * Up to 384 rows: s = 22528 at 257 / 384 rows 60 / 69, 71 / 78, 24576 at 257 / 352 64 / 69,
+      75 / 80 [s = 28672 at 300 70 / 66; 34816 at 400 126 / 112].
     * Up to 512 rows, three tiles of 128 giving way to two of 256: s = 15360 at 385 / 512
-      rows 27 / 38, 28 / 39; s = 20480 at 385 / 416 rows 43 / 54, 44 / 54 [at 480 76 / 66]; s =
-      28672 at 385 / 512 75 / 89, 82 / 93; s = 34816 at 500 / 512 134 / 147, 134 / 141 [at 480
-      132 / 119].
-    * More rows: s = 12288 at 513 / 768 rows 54 / 61, 78 / 83; s = 10240 at 1024
-      82 / 85 [s = 15360 at 640 65 / 54; s = 8192 at 1536 147 / 133]; with a narrow
-      product among them, which the library serves badly (q/k/v), s = 6144 at 2048 83 /
-      93, s = 10240 at 1200 137 / 196."""
+      rows 27 / 38, 28 / 39; s = 20480 at 385 / 448 43 / 54, 72 / 80 [at 480 76 / 66, where a tile of
+      the library fits]; s = 24576 at 448 64 / 67 [at 512 84 / 80]; s = 28672 at 385 / 512 75 /
+      89, 82 / 93; s = 34816 at 500 / 512 134 / 147, 134 / 141 [at 480 132 / 119].
+    * More rows: s = 12288 at 513 / 768 rows 54 / 61, 78 / 83; s = 10240 at 1024 82 / 85 [s =
+      8192 at 1536 147 / 133]; s = 15360 of 1024 columns at 600 46 / 54 [of 1536 at 640 65 /
+      54]; s = 17408 at 513 / 700 57 / 65, 65 / 74; s = 20480 at 600 78 / 92 [22528 at 560 94 /
+      89]; with a narrow product among them, which the library serves badly (q/k/v), s =
+      6144 at 2048 83 / 93, s = 10240 at 1200 137 / 196."""
     if rows < 160 or rows > _lib.NM_ROWS_MAX:
         return False
     if len(hs) == 1:
-        return rows <= 768 and w >= max(hs[0], 5120) and hs[0] > 1024 and w + hs[0] >= 6400
+        h = hs[0]
+        if rows > 768 or w < h or h <= 1024:
+            return False
+        if h < 2048:
+            return w >= 5120 and (w + h >= 6400 or rows >= 256) or w >= 4096 and rows >= 512
+        return (w >= 4096 or (w >= 3840 and rows <= 384)
+                or (w >= 3072 and rows > 384 and (rows > 512 or h >= 2560)))
     s = sum(hs)
     if rows <= 256:
         return s <= 32768 or (rows >= 200 and s <= 51200 and rows * s <= 3 << 22)
     if rows <= 384:
-        return s <= 22528
+        return s <= 24576
     if rows <= 512:
-        return (s <= 16384 or (s <= 25600 and rows <= 416) or 25600 < s <= 32768
-                or (32768 < s <= 36864 and rows >= 500))
-    return s <= 12288 and rows * s <= (3 << 22 if min(hs) <= 1024 else 5 << 21)
+        if s <= 22528:  # the library's tiles fit some row counts of some widths
+            return not (16384 < s < 18432 and 416 < rows < 465 or 18432 < s < 22528 and 464 < rows < 490)
+        return (s <= 25600 and rows <= 464) or 25600 < s <= 32768 or (32768 < s <= 36864 and rows >= 500)
+    if s <= 12288:
+        return rows * s <= (5 << 21 if 6144 < s < 9216 and min(hs) > 1024 else 3 << 22)
+    return s <= 20480 and rows * s <= 3 << 22 and (w <= 1024 or s > 16384)
 
 
 def nmsparse_spmm_forward_hip(x, mat_data, mat_index, w, h, BLOCK_WIDTH, VEC_WIDTH, *, out=None, config_id=-1,
